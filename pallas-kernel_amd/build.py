@@ -4,7 +4,7 @@
 
 Objects go to pallas-kernel_amd/_build/, the library to
 pallas-kernel_amd/tops/_lib/libtops_hip.so (both git-ignored).  --phase-clocks also builds
-tops/_lib/libtops_pipe_clocks.so: the pipelined sweep alone, compiled with
+tops/_lib/libtops_pipe_clocks.so: the strip sweep alone, compiled with
 TOPS_PHASE_CLOCKS (per-wave phase clocks, read by pallas-kernel_amd/phase_clocks.py).
 """
 from __future__ import annotations
@@ -69,11 +69,11 @@ CLOCKS_LIB = os.path.join(LIBDIR, "libtops_pipe_clocks.so")
 
 
 def build_phase_clocks(verbose: bool = True) -> str:
-    """The instrumented pipelined sweep (TOPS_PHASE_CLOCKS) as its own library."""
+    """The instrumented strip sweep (TOPS_PHASE_CLOCKS) as its own library."""
     os.makedirs(BUILD, exist_ok=True)
     os.makedirs(LIBDIR, exist_ok=True)
-    src = os.path.join(CSRC, "gla_sweep_pipe.hip")
-    obj = os.path.join(BUILD, "gla_sweep_pipe.clocks.o")
+    src = os.path.join(CSRC, "gla_strip.hip")
+    obj = os.path.join(BUILD, "gla_strip.clocks.o")
     r = subprocess.run([HIPCC] + COMMON + DEVICE + ["-DTOPS_PHASE_CLOCKS", "-c", src, "-o", obj],
                        capture_output=True, text=True)
     if r.returncode != 0:

@@ -54,14 +54,14 @@ struct SweepParams {
   // usual; 1 writes acc32 = result; 2 adds acc32 += result; 3 writes out = acc32 + result.
   float* acc32 = nullptr;
   int acc_mode = 0;
-  // fp16 checkpoints (the pipelined bf16 sweep only): ckpt then points at fp16
+  // fp16 checkpoints (bf16 inputs): ckpt then points at fp16
   // [total, H, K, V] holding the state divided by 2^e, one power of two per (chunk, head,
   // 64-column V tile) chosen from the tile's largest magnitude (at most 2^15 after scaling),
   // and ckpt_scale [total, H, NV] receives the factors 2^e.
   int ckpt16 = 0;
   float* ckpt_scale = nullptr;
-  // phase clocks of the pipelined sweep, [grid, 8 waves, 8] (read only by a library built
-  // with TOPS_PHASE_CLOCKS; see gla_sweep_pipe.hip)
+  // phase clocks of the strip sweep, [grid, 8 waves, 8] (read only by a library built with
+  // TOPS_PHASE_CLOCKS; see gla_strip.hip)
   unsigned long long* clocks = nullptr;
 };
 
@@ -70,12 +70,14 @@ struct SweepParams {
 template <typename TIn, bool REV, bool DELTA = false>
 hipError_t launch_gla_sweep(const SweepParams& p, hipStream_t s);
 
-// The software-pipelined sweep (gla_sweep_pipe.hip) for bf16 calls with per-channel gates:
-// same results as gla_sweep_kernel, the staging of chunk c + 1 overlapped with chunk c's
-// matrix products.  launch_gla_sweep routes eligible calls to it.
-bool gla_pipe_eligible(const SweepParams& p);
-template <bool REV>
-hipError_t launch_gla_pipe(const SweepParams& p, hipStream_t s);
+// The strip-specialised sweep (gla_strip.hip) for per-channel gates: launch_gla_sweep routes
+// eligible calls to it.
+bool gla_strip_eligible(const SweepParams& p);
+template <typename TIn, bool REV, bool DELTA>
+hipError_t launch_gla_strip(const SweepParams& p, hipStream_t s);
+// Its state-only pass: the end state s_fin and the decay sums dec_fin of every sequence.
+template <typename TIn, bool REV>
+hipError_t launch_gla_strip_state(const SweepParams& p, hipStream_t s);
 
 // Sweep with the gate on the value side (g = gv [B,T,H,V], bf16 inputs), forward or (REV)
 // the state-gradient recurrence: see gla_sweep.hip.

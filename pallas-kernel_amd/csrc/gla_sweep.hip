@@ -62,7 +62,7 @@ namespace tops {
 // GK: the per-channel gate mode only (kGateK, the GLA and KDA path), compiled on its own so
 // that the hot path carries no gate-mode branches; !GK serves the per-token and constant
 // gates (kGateS, kGateGamma, kGateGammaK) chosen at run time.
-// VAR selects the features an instance compiles (as in gla_sweep_pipe.hip): 1 = fp16
+// VAR selects the features an instance compiles (as in gla_strip.hip): 1 = fp16
 // checkpoints of every chunk, whole-width rows, no slices; 2 = no checkpoints and no slices;
 // 0 = the rest (fp32 or paired checkpoints, channel slices; no fp16 checkpoints).
 template <typename TIn, int KP, bool REV, bool DELTA, bool ST, bool GK, int YG = 0, int VAR = 0>
@@ -986,8 +986,8 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
 
 template <typename TIn, bool REV, bool DELTA>
 hipError_t launch_gla_sweep(const SweepParams& p, hipStream_t s) {
-  if constexpr (std::is_same<TIn, uint16_t>::value && !DELTA) {
-    if (gla_pipe_eligible(p)) return launch_gla_pipe<REV>(p, s);
+  if constexpr (!DELTA) {
+    if (gla_strip_eligible(p)) return launch_gla_strip<TIn, REV, false>(p, s);
   }
   // fp16 checkpoints: whole-width state rows with the plain layout (ckpt_par 0, no slices)
   const bool plain = !p.acc_mode && !p.ldk;
@@ -1007,7 +1007,7 @@ hipError_t launch_gla_sweep(const SweepParams& p, hipStream_t s) {
   } else if (var == 2) hipLaunchKernelGGL((gla_sweep_kernel<TIn, KPV, REV, DELTA, false, GKV, YGV, 2>), grid, dim3(512), 0, s, p); \
   else hipLaunchKernelGGL((gla_sweep_kernel<TIn, KPV, REV, DELTA, false, GKV, YGV, 0>), grid, dim3(512), 0, s, p)
   // fp16 checkpoints: the delta sweeps and the bf16 one-gate-per-token sweeps here, the
-  // per-channel-gate bf16 sweeps in the pipelined kernel (routed above)
+  // per-channel-gate bf16 sweeps in the strip kernel (routed above)
   const bool yg2 = std::is_same<TIn, uint16_t>::value && !DELTA && !gk && !p.gshift &&
                    (p.gate_mode == kGateS || p.gate_mode == kGateGamma);
   if (var == 1 && !DELTA && !yg2) return hipErrorInvalidValue;
@@ -1063,9 +1063,7 @@ hipError_t launch_gla_state_pass(const SweepParams& p, hipStream_t s) {
 #define TOPS_STATE(KPV, GKV) \
   hipLaunchKernelGGL((gla_sweep_kernel<TIn, KPV, REV, false, true, GKV>), grid, dim3(512), 0, s, p)
   if (p.gate_mode == kGateK) {
-    if (kp == 32) TOPS_STATE(32, true);
-    else if (kp == 64) TOPS_STATE(64, true);
-    else TOPS_STATE(128, true);
+    return launch_gla_strip_state<TIn, REV>(p, s);
   } else {
     if (kp == 32) TOPS_STATE(32, false);
     else if (kp == 64) TOPS_STATE(64, false);

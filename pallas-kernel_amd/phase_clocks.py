@@ -1,4 +1,4 @@
-"""Per-phase clock breakdown of the pipelined chunk sweep (gla_pipe_kernel) at a chunk_gla
+"""Per-phase clock breakdown of the strip chunk sweep (gla_strip_kernel) at a chunk_gla
 shape, from the instrumented library (built by ``python pallas-kernel_amd/build.py
 --phase-clocks``; the regular library compiles no clocks).
 
@@ -7,11 +7,10 @@ shape, from the instrumented library (built by ``python pallas-kernel_amd/build.
 Runs the forward training sweep (fp16 checkpoints), the reverse training sweep (dh, fp16
 checkpoints) and the inference forward (no checkpoints) on synthetic bf16 inputs (q, k, v /
 dO ~ N(0, 1), g = logsigmoid(N(0, 1)) / 16), and prints, per sweep, the shader-clock cycles
-per chunk that each wave spends in the six intervals of the chunk loop (mean over the waves
-of all workgroups; waves 0-1 also compute the two D tiles past the eighth), the clock rate
-seen by the waves (s_memtime over s_memrealtime) and the kernel's own time (HIP events).
-A wave's time between two barriers is its own work in that phase; its wait at the barrier
-is the rest of the slowest wave's work.
+per chunk that each wave spends in the intervals of the chunk loop (waves 0-3 consumers,
+4-7 producers; csrc/gla_strip.hip names the slots), the clock rate seen by the waves
+(s_memtime over s_memrealtime) and the kernel's own time (HIP events).  A wave's time between
+two barriers is its own work; its wait at the barrier is the rest of the slowest wave's work.
 """
 from __future__ import annotations
 
@@ -25,9 +24,10 @@ import torch.nn.functional as F
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB = os.path.join(HERE, "tops", "_lib", "libtops_pipe_clocks.so")
-PHASES = ["B1 wait", "plane writes + gate scan", "B2 wait",
-          "matrix phase (H^T, checkpoint, D tiles, state update, staging)", "B3 wait",
-          "output products"]
+PHASES = ["A: work (producers: after the D tiles)", "A: barrier wait",
+          "B: next T (consumers) / gate cumsum (producers)", "B: barrier wait",
+          "B: output block (consumers) / A: D tiles (producers)",
+          "B: state update (consumers) / X~ staging (producers)"]
 NW = 8
 
 
@@ -90,12 +90,12 @@ def run(B, T, H, K, V, reps=5, seed=0):
         per_chunk = acc[..., :6] / NT                       # [grid, wave, phase]
         mhz = float(acc[..., 6].sum() / acc[..., 7].sum()) * 100.0
         allw = per_chunk.mean(dim=(0, 1))
-        w01 = per_chunk[:, :2].mean(dim=(0, 1))
-        w27 = per_chunk[:, 2:].mean(dim=(0, 1))
+        wc = per_chunk[:, :4].mean(dim=(0, 1))
+        wp = per_chunk[:, 4:].mean(dim=(0, 1))
         loop_us = float(acc[..., 6].mean()) / mhz
         perw = per_chunk.mean(dim=0)                       # [wave, phase]
         res[name] = dict(
-            phases={p: dict(all=float(allw[i]), waves01=float(w01[i]), waves27=float(w27[i]),
+            phases={p: dict(all=float(allw[i]), consumers=float(wc[i]), producers=float(wp[i]),
                             per_wave=[round(float(perw[w, i])) for w in range(NW)])
                     for i, p in enumerate(PHASES)},
             cycles_per_chunk=float(allw.sum()), clock_mhz=mhz,
@@ -112,11 +112,11 @@ def markdown(res, shape):
                      f"kernel {r['kernel_ms']:.4f} ms (HIP events, median; min {r['kernel_ms_min']:.4f}); "
                      f"waves' clock {r['clock_mhz']:.0f} MHz; chunk loop {r['loop_us']:.1f} us per "
                      f"wave, {r['us_per_chunk']:.3f} us per chunk\n")
-        lines.append("| interval | cycles / chunk (all waves) | waves 0-1 | waves 2-7 | share |")
+        lines.append("| interval | cycles / chunk (all waves) | consumers | producers | share |")
         lines.append("|---|---|---|---|---|")
         tot = r["cycles_per_chunk"]
         for p, d in r["phases"].items():
-            lines.append(f"| {p} | {d['all']:.0f} | {d['waves01']:.0f} | {d['waves27']:.0f} | "
+            lines.append(f"| {p} | {d['all']:.0f} | {d['consumers']:.0f} | {d['producers']:.0f} | "
                          f"{100 * d['all'] / tot:.1f}% |")
         lines.append(f"| total | {tot:.0f} | | | |\n")
         lines.append("| interval | " + " | ".join(f"wave {w}" for w in range(NW)) + " |")
