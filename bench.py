@@ -41,10 +41,10 @@ _S = B * H * K * V * 4
 # set_checkpoint_layout("full32") the fp32-checkpoint ones: both are timed under one row.
 KERNELS = {
     # q, k, v, g read; o written; h0 read; ht written
-    "tops_gla_chunk_fwd": dict(kernel="gla_pipe_kernel<fwd>", entry="tops_gla_chunk_fwd_c16",
+    "tops_gla_chunk_fwd": dict(kernel="gla_strip_kernel<fwd>", entry="tops_gla_chunk_fwd_c16",
                                bytes=_TH * (2 * K + 2 * K + 2 * V + 4 * K + 2 * V) + 2 * _S),
     # q, k, g, dO read; dv written; dht read; dh0 written
-    "tops_gla_chunk_bwd_dh": dict(kernel="gla_pipe_kernel<rev>", entry="tops_gla_chunk_bwd_dh_c16",
+    "tops_gla_chunk_bwd_dh": dict(kernel="gla_strip_kernel<rev>", entry="tops_gla_chunk_bwd_dh_c16",
                                   bytes=_TH * (2 * K + 2 * K + 4 * K + 2 * V + 2 * V) + 2 * _S),
     # q, k, v, g, dO read; dq, dk, dg written
     "tops_gla_chunk_bwd_dqkg": dict(kernel="gla_dqkg_kernel", entry="tops_gla_chunk_bwd_dqkg_c16",

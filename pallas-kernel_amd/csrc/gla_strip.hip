@@ -25,6 +25,10 @@
 // X~, Y and D are single planes (written in the interval that does not read them), Z~ two.
 // Planes are row-major without padding, 16-byte pieces XOR-swizzled by row so that the row
 // reads, the transposed reads and the staging writes are free of bank conflicts.
+// Delta rule (KDA): forward, Y = v_new = u - w S comes from the state operand and the staged
+// planes of w 2^-Gm (against T = 2^Gm S), token-major, which is the operand layout of the
+// products that follow; reverse, the state update gains - w^T dv_new, and dv_new is stored
+// transposed per chunk for the WY backward.
 // The D tiles sit with the consumers, which have the X~ fragments in registers already: with
 // the producers they cost 80 KB more of LDS reads per chunk and made interval A
 // producer-bound (9,200 -> 8,900 cycles per training chunk, 8,000 -> 6,700 inference).  The
@@ -37,7 +41,11 @@
 // producer wave, ~400 per consumer wave and chunk) and LDS reads (~450 KB) next.  B8 T4096 H16
 // K=V=128 bf16, one workgroup per CU: training sweeps 362 / 356 -> 255 / 255 us forward /
 // reverse, inference forward 303 -> 224 us against a sweep whose eight waves each staged,
-// multiplied and passed the state through LDS.
+// multiplied and passed the state through LDS.  Delta rule, B4 T8192 H32 K=V=128 bf16:
+// forward with checkpoints 1187 -> 800 us, without 1047 -> 680, reverse 970 -> 710 (2.7 to
+// 3.5 GB per launch, 500-720 us at the copy rate); fp32, B1 T5000 H32 (64 workgroups, so
+// latency alone): 756 -> 370.  There producers keep the D tiles (the consumers carry w S) and
+// the default priority in interval A.
 #include <stdlib.h>
 
 #include <type_traits>
@@ -126,6 +134,9 @@ __global__ __launch_bounds__(512) void gla_strip_kernel(SweepParams p) {
   constexpr bool REV_DELTA = DELTA && REV;
   constexpr bool SY = SIN || FWD_DELTA;      // Y carries a lo half
   constexpr bool CONS_D = !FWD_DELTA;        // the consumers compute the D tiles
+  // reverse delta rule: Z~^T Y is taken in interval A, so Z~ and Y are single planes written
+  // in B with X~ (two Z~ planes, w and the checkpoint would not fit the 160 KB)
+  constexpr bool ZB = REV_DELTA;
   constexpr int KC = KP / 32;                // 32-channel blocks
   constexpr int NT = 2 * KC;                 // state tiles of a consumer
   constexpr int PL = C * KP;                 // elements of one plane
@@ -141,16 +152,18 @@ __global__ __launch_bounds__(512) void gla_strip_kernel(SweepParams p) {
   typedef Words<TIn> Wd;
 
   __shared__ __attribute__((aligned(16))) uint16_t sX[ST ? 8 : 2 * PL];
-  __shared__ __attribute__((aligned(16))) uint16_t sZ[4 * PL];
+  __shared__ __attribute__((aligned(16))) uint16_t sZ[(ZB ? 2 : 4) * PL];
   __shared__ __attribute__((aligned(16))) uint16_t sW[DELTA ? 2 * PL : 8];
   __shared__ __attribute__((aligned(16))) uint16_t sY[FWD_DELTA ? 8 : (SIN ? 2 : 1) * C * LY];
   __shared__ __attribute__((aligned(16))) uint4 sDt[ST ? 1 : 10 * 64];
   __shared__ __attribute__((aligned(16))) float sE[2 * KP];      // e of this and the next chunk
   __shared__ __attribute__((aligned(16))) float sTot[NRW * KP];  // gate totals per row wave
-  // fp16 checkpoints: the state entering the next chunk [K][BV] for the producers to store
-  constexpr int LS = BV + 4;
-  __shared__ __attribute__((aligned(16))) float sS[CK16 ? KP * LS : 4];
-  __shared__ uint32_t sMx[4];                // and each producer wave's largest |S|
+  // fp16 checkpoints: the state entering the chunk for the producers to store, fp32 [K][BV];
+  // the delta rule, short of LDS by its w planes, hands it over packed, fp16 [BV][K]
+  constexpr int LS = BV + 4, LC = KP + 8;
+  __shared__ __attribute__((aligned(16))) float sS[CK16 && !DELTA ? KP * LS : 4];
+  __shared__ __attribute__((aligned(16))) uint16_t sC[CK16 && DELTA ? BV * LC : 8];
+  __shared__ uint32_t sMx[4];                // largest |S| of each wave that takes the maxima
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -194,6 +207,7 @@ __global__ __launch_bounds__(512) void gla_strip_kernel(SweepParams p) {
   const int NTs = cdiv(L, C);
   const uint32_t rowK = (uint32_t)(H * LDK), rowV = (uint32_t)(H * V);
   auto cidx = [&](int it) { return REV ? NTs - 1 - it : it; };
+  auto zbuf = [&](int it) { return sZ + (ZB ? 0 : (it & 1) * (2 * PL)); };   // Z~ of a chunk
 
   // row reads of a swizzled plane: piece 4 kc + lg of row l16 (+ 16 rows per block)
   int xa[KC];
@@ -216,6 +230,14 @@ __global__ __launch_bounds__(512) void gla_strip_kernel(SweepParams p) {
     uint2 h, l;
     acc_to_bf16x4(a, h, l);
     sDt[(Rc * (Rc + 1) / 2 + Pc) * 64 + lane] = make_uint4(h.x, h.y, l.x, l.y);
+  };
+
+  // factor of a checkpoint tile from the wave maxima: 2^(14 - e), e the largest exponent
+  auto ckpt_scale = [&]() {
+    const uint32_t m = max(max(sMx[0], sMx[1]), max(sMx[2], sMx[3]));
+    int ex = (int)((m >> 23) & 0xffu) - 127;
+    ex = ex < -100 ? -100 : ex;
+    return __uint_as_float((uint32_t)(141 - ex) << 23);
   };
 
   if (wave >= 4) {
@@ -418,8 +440,9 @@ __global__ __launch_bounds__(512) void gla_strip_kernel(SweepParams p) {
     // checkpoint of the state entering the chunk: read in interval A (the wave maxima to sMx),
     // stored in B, 8 columns of a row per lane
     constexpr int CU = KP / 32;
-    f32x4 cs[CK16 ? 2 * CU : 1];
+    f32x4 cs[CK16 && !DELTA ? 2 * CU : 1];
     auto ckpt_read = [&]() {
+      if constexpr (DELTA) return;
 #pragma unroll
       for (int u = 0; u < CU; ++u) {
         const float* q = sS + ((ptid >> 3) + 32 * u) * LS + 8 * (ptid & 7);
@@ -429,12 +452,23 @@ __global__ __launch_bounds__(512) void gla_strip_kernel(SweepParams p) {
       state_absmax(cs, sMx, pw, lane);
     };
     auto ckpt_store = [&](int c) {
-      const uint32_t m = max(max(sMx[0], sMx[1]), max(sMx[2], sMx[3]));
-      int ex = (int)((m >> 23) & 0xffu) - 127;
-      ex = ex < -100 ? -100 : ex;
-      const float sinv = __uint_as_float((uint32_t)(141 - ex) << 23);
+      if constexpr (DELTA) {
+        // read transposed: lane holds columns 32 h + 8 lg + 0..7 of channel 16 cb + l16
+        const rsrc_t R = make_rsrc((uint16_t*)p.ckpt + ((size_t)(cbase + c) * H + hh) * LDK * V,
+                                   (long long)K * V * 2);
+#pragma unroll
+        for (int u = 0; u < CU; ++u) {
+          const int cb = (pw * CU + u) >> 1, h = (pw * CU + u) & 1;
+          const uint16_t* q = sC + (32 * h + 8 * lg + (l16 >> 2)) * LC + 16 * cb + 4 * (l16 & 3);
+          const int row = 16 * cb + l16, v = vt * BV + 32 * h + 8 * lg;
+          bst128(R, __builtin_bit_cast(uint4, tr2(q, q + 4 * LC)),
+                 (row < K && v < V) ? ((uint32_t)row * V + v) * 2u : kOOB, 0);
+        }
+        return;
+      }
+      const float sinv = ckpt_scale();
       const size_t slot = (size_t)(cbase + c) * H + hh;
-      if (ptid == 0) p.ckpt_scale[slot * p.NV + vt] = __uint_as_float((uint32_t)(113 + ex) << 23);
+      if (ptid == 0) p.ckpt_scale[slot * p.NV + vt] = 1.f / sinv;   // powers of two
       const rsrc_t R = make_rsrc((uint16_t*)p.ckpt + slot * LDK * V, (long long)K * V * 2);
       const int v = vt * BV + 8 * (ptid & 7);
 #pragma unroll
@@ -461,9 +495,11 @@ __global__ __launch_bounds__(512) void gla_strip_kernel(SweepParams p) {
     __syncthreads();
     sums(0);
     stage(rk, REV, true, sZ);
+    if constexpr (ZB) write_y();
     if constexpr (!ST) stage(rq, !REV, false, sX);
     if constexpr (FWD_DELTA) stage_w();
     load_g(1);
+    if constexpr (ZB) load_y(1);
     load_rows(pZ, 1, rk);
     if constexpr (!ST) load_rows(pX, 1, rq);
     if constexpr (FWD_DELTA) load_w(1);
@@ -475,8 +511,8 @@ __global__ __launch_bounds__(512) void gla_strip_kernel(SweepParams p) {
     clk.start();
     for (int it = 0; it < NTs; ++it) {
       // A: D and Y of this chunk, Z~ of the next
-      __builtin_amdgcn_s_setprio(2);
-      const uint16_t* z = sZ + (it & 1) * (2 * PL);
+      __builtin_amdgcn_s_setprio(DELTA ? 0 : 2);
+      const uint16_t* z = zbuf(it);
       if constexpr (CONS_D) {
       } else if (pw == 0) dtiles(std::integral_constant<int, 3>{}, 3, 0, z);
       else if (pw == 1) dtiles(std::integral_constant<int, 3>{}, 2, 0, z);
@@ -487,7 +523,7 @@ __global__ __launch_bounds__(512) void gla_strip_kernel(SweepParams p) {
       }
       clk.tick(4);
       if constexpr (CK16) ckpt_read();
-      if constexpr (!FWD_DELTA) {
+      if constexpr (!FWD_DELTA && !ZB) {
         write_y();
         load_y(it + 1);
       }
@@ -496,14 +532,22 @@ __global__ __launch_bounds__(512) void gla_strip_kernel(SweepParams p) {
         load_w(it + 1);
       }
       sums((it + 1) & 1);
-      stage(rk, REV, true, sZ + ((it + 1) & 1) * (2 * PL));
-      load_rows(pZ, it + 2, rk);
+      if constexpr (!ZB) {
+        stage(rk, REV, true, zbuf(it + 1));
+        load_rows(pZ, it + 2, rk);
+      }
       clk.tick(0);
       __syncthreads();
       clk.tick(1);
       // B: X~ (and w) of the next chunk, the cumsum of the one after
       __builtin_amdgcn_s_setprio(CK16 ? 2 : 0);
       if constexpr (CK16) ckpt_store(cidx(it));
+      if constexpr (ZB) {
+        stage(rk, REV, true, sZ);
+        load_rows(pZ, it + 2, rk);
+        write_y();
+        load_y(it + 2);
+      }
       if constexpr (!ST) {
         stage(rq, !REV, false, sX);
         clk.tick(5);
@@ -576,7 +620,17 @@ __global__ __launch_bounds__(512) void gla_strip_kernel(SweepParams p) {
     }
   };
   auto store_ckpt = [&](int c) {
-    if constexpr (VAR == 0) {
+    if constexpr (CK16 && DELTA) {
+      const float sinv = ckpt_scale();
+      if (tid == 0) p.ckpt_scale[((size_t)(cbase + c) * H + hh) * p.NV + vt] = 1.f / sinv;
+#pragma unroll
+      for (int kc = 0; kc < KC; ++kc) {
+        const f32x4 &a = S[2 * kc], &b = S[2 * kc + 1];
+        *(uint4*)(sC + (16 * j + l16) * LC + 32 * kc + 8 * lg) =
+            make_uint4(pack_f16x2(a[0] * sinv, a[1] * sinv), pack_f16x2(a[2] * sinv, a[3] * sinv),
+                       pack_f16x2(b[0] * sinv, b[1] * sinv), pack_f16x2(b[2] * sinv, b[3] * sinv));
+      }
+    } else if constexpr (VAR == 0) {
       if (!(p.ckpt && (p.ckpt_par == 0 || ((cbase + c) & 1) == p.ckpt_par - 1))) return;
       const rsrc_t R = make_rsrc(p.ckpt + ((size_t)(cbase + c) * H + hh) * LDK * V, (long long)K * V * 4);
 #pragma unroll
@@ -601,7 +655,9 @@ __global__ __launch_bounds__(512) void gla_strip_kernel(SweepParams p) {
   };
 
   auto publish_S = [&]() {                     // for the producers' checkpoint
-    if constexpr (CK16) {
+    if constexpr (CK16 && DELTA) {
+      state_absmax(S, sMx, wave, lane);
+    } else if constexpr (CK16) {
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -674,7 +730,7 @@ __global__ __launch_bounds__(512) void gla_strip_kernel(SweepParams p) {
     for (int Rb = 0; Rb < 4; ++Rb) o[Rb] = f32x4{0.f, 0.f, 0.f, 0.f};
     // and the wave's share of the D tiles, on the X~ fragments in registers: row block j of Z~
     // with up to three of its tiles; wave 3 also takes tile (R 3, P 0)
-    const uint16_t* zc = sZ + (it & 1) * (2 * PL);
+    const uint16_t* zc = zbuf(it);
     auto interval_a = [&](auto jc) {
       constexpr int J = decltype(jc)::value;   // Pc of the wave's row block (-1: no D tiles)
       constexpr int ND = J < 0 ? 0 : (J == 3 ? 2 : (J == 2 ? 2 : 3));
@@ -714,6 +770,31 @@ __global__ __launch_bounds__(512) void gla_strip_kernel(SweepParams p) {
 #pragma unroll
       for (int u = 0; u < ND; ++u) put_d(a[u], J == 3 ? 3 : J + u, J == 3 && u == 1 ? 0 : J);
     };
+    auto read_y = [&]() {
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const uint16_t* py = sY + ya + 32 * q * LY;
+        yh[q] = tr2(py, py + 16 * LY);
+        yl[q] = yh[q];
+        if constexpr (SY) yl[q] = tr2(py + C * LY, py + C * LY + 16 * LY);
+      }
+    };
+    // Z~^T Y of state tile t, added to a
+    auto zty = [&](int t, f32x4 a) {
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const uint16_t* pz = zc + za[t >> 1] + 4 * (t & 1) + 32 * q * KP;
+        const bf16x8 zh = tr2(pz, pz + 16 * KP), zl = tr2(pz + PL, pz + PL + 16 * KP);
+        a = mma<true, SY>(a, zh, zl, yh[q], yl[q]);
+      }
+      return a;
+    };
+    f32x4 dz[ZB ? NT : 1];
+    if constexpr (ZB) {
+      read_y();
+#pragma unroll
+      for (int t = 0; t < NT; ++t) dz[t] = zty(t, f32x4{0.f, 0.f, 0.f, 0.f});
+    }
     if constexpr (ST) {
     } else if constexpr (!CONS_D) interval_a(std::integral_constant<int, -1>{});
     else if (j == 0) interval_a(std::integral_constant<int, 0>{});
@@ -725,15 +806,7 @@ __global__ __launch_bounds__(512) void gla_strip_kernel(SweepParams p) {
     clk.tick(1);
 
     // ---------------- B: intra-chunk products, state update
-    if constexpr (!FWD_DELTA) {
-#pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const uint16_t* py = sY + ya + 32 * q * LY;
-        yh[q] = tr2(py, py + 16 * LY);
-        yl[q] = yh[q];
-        if constexpr (SY) yl[q] = tr2(py + C * LY, py + C * LY + 16 * LY);
-      }
-    }
+    if constexpr (!FWD_DELTA && !ZB) read_y();
     if constexpr (!ST) {
     uint4 d[10];
 #pragma unroll
@@ -792,20 +865,18 @@ __global__ __launch_bounds__(512) void gla_strip_kernel(SweepParams p) {
     }
     clk.tick(4);
     // state update: T += Z~^T Y (forward), S = e T
-    const uint16_t* z = sZ + (it & 1) * (2 * PL);
 #pragma unroll
     for (int kc = 0; kc < KC; ++kc) {
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
         const int t = 2 * kc + b;
-        f32x4 a = REV ? f32x4{0.f, 0.f, 0.f, 0.f} : T[t];
+        f32x4 a;
+        if constexpr (ZB) a = dz[t];
+        else a = zty(t, REV ? f32x4{0.f, 0.f, 0.f, 0.f} : T[t]);
         f32x4 w = {0.f, 0.f, 0.f, 0.f};
+        if constexpr (REV_DELTA) {
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          const uint16_t* pz = z + za[kc] + 4 * b + 32 * q * KP;
-          const bf16x8 zh = tr2(pz, pz + 16 * KP), zl = tr2(pz + PL, pz + PL + 16 * KP);
-          a = mma<true, SY>(a, zh, zl, yh[q], yl[q]);
-          if constexpr (REV_DELTA) {
+          for (int q = 0; q < 2; ++q) {
             const uint16_t* pww = sW + za[kc] + 4 * b + 32 * q * KP;
             const bf16x8 wh = tr2(pww, pww + 16 * KP), wl = tr2(pww + PL, pww + PL + 16 * KP);
             w = mma<true, true>(w, wh, wl, vh[q], vl[q]);
@@ -890,6 +961,10 @@ TOPS_STRIP_STATE(float)
 TOPS_STRIP_STATE(_Float16)
 #undef TOPS_STRIP_STATE
 
+template hipError_t launch_gla_strip<uint16_t, false, true>(const SweepParams&, hipStream_t);
+template hipError_t launch_gla_strip<float, false, true>(const SweepParams&, hipStream_t);
+template hipError_t launch_gla_strip<uint16_t, true, true>(const SweepParams&, hipStream_t);
+template hipError_t launch_gla_strip<float, true, true>(const SweepParams&, hipStream_t);
 template hipError_t launch_gla_strip<uint16_t, false, false>(const SweepParams&, hipStream_t);
 template hipError_t launch_gla_strip<uint16_t, true, false>(const SweepParams&, hipStream_t);
 template hipError_t launch_gla_strip<float, false, false>(const SweepParams&, hipStream_t);

@@ -65,13 +65,12 @@ struct SweepParams {
   unsigned long long* clocks = nullptr;
 };
 
-// TIn = uint16_t (bf16 bits) or float; REV = reverse (state-gradient) sweep;
-// DELTA = the KDA delta-rule sweep (v_new = u - w S replaces v).
-template <typename TIn, bool REV, bool DELTA = false>
+// TIn = uint16_t (bf16 bits), float or _Float16; REV = reverse (state-gradient) sweep.
+template <typename TIn, bool REV>
 hipError_t launch_gla_sweep(const SweepParams& p, hipStream_t s);
 
 // The strip-specialised sweep (gla_strip.hip) for per-channel gates: launch_gla_sweep routes
-// eligible calls to it.
+// eligible calls to it.  DELTA = the KDA delta-rule sweep (forward, v_new = u - w S replaces v).
 bool gla_strip_eligible(const SweepParams& p);
 template <typename TIn, bool REV, bool DELTA>
 hipError_t launch_gla_strip(const SweepParams& p, hipStream_t s);

@@ -8,6 +8,10 @@
 // (tops/ops/common/chunk_h.py:685-878) plus the dv part of K4 (chunk.py:1447-1509),
 // following the oracle tops/cpu/ops/gla/chunk.py:310-354, 387-427.
 //
+// Calls with per-channel gates, and KDA's delta rule, run on the strip-specialised sweep of
+// gla_strip.hip; this kernel keeps the other gate forms, the reverse-time recurrence and the
+// value-side gates.
+//
 // One workgroup (8 wave64, two per SIMD) owns one (sequence, head, 64-wide V tile) and
 // walks the sequence chunk by chunk (C = 64), forwards or backwards.  A K x 64 fp32 state S
 // lives in MFMA accumulators for the whole walk (4 tiles per wave at K = 128).  Per chunk,
@@ -28,11 +32,6 @@
 // column tiles 2 (w % 2), 2 (w % 2) + 1 (the two waves of a token block both compute its
 // intra-chunk D tiles: MFMA has the headroom, a split would cost a barrier).
 //
-// DELTA (the KDA delta rule): forward, Y = v_new = u - w S is computed per chunk before the
-// output and the state update (w 2^-Gm is read from HBM as the MFMA A operand against
-// H^T = 2^Gm S); reverse, the state update gains - w^T dv_new, and dv_new is written
-// transposed per chunk for the WY backward.
-//
 // YG (bf16): the gate is applied on the value side.  YG = 1 (forward): one log-gate per
 // (token, V column) (fused_recurrent_gla's gv), S[:, v] <- 2^gv S[:, v] + k v^T.  YG = 2
 // (forward and reverse): one log-gate per token (simple GLA's g [B,T,H], or g_gamma [H]),
@@ -50,7 +49,7 @@
 //
 // Pipelining: the raw q/k/g/Y of chunk c+1 are loaded into registers while chunk c is
 // computed; a full chunk takes a branch-free path (masked rows read out of range and are
-// zeroed by the buffer range check).  Two barriers per chunk (three or four with DELTA).
+// zeroed by the buffer range check).  Two barriers per chunk.
 #include <type_traits>
 
 #include "gla_sweep.h"
@@ -65,7 +64,7 @@ namespace tops {
 // VAR selects the features an instance compiles (as in gla_strip.hip): 1 = fp16
 // checkpoints of every chunk, whole-width rows, no slices; 2 = no checkpoints and no slices;
 // 0 = the rest (fp32 or paired checkpoints, channel slices; no fp16 checkpoints).
-template <typename TIn, int KP, bool REV, bool DELTA, bool ST, bool GK, int YG = 0, int VAR = 0>
+template <typename TIn, int KP, bool REV, bool ST, bool GK, int YG = 0, int VAR = 0>
 __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
   constexpr int NW = 8;                  // wave64s per workgroup
   constexpr int NTH = 64 * NW;
@@ -81,12 +80,10 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
   static_assert(NQ % CQL == 0, "KP must be a multiple of 32");
   static_assert(CQL == 8 && SGL == 4, "the segment scan takes 8 column quads x 4 segments");
   constexpr bool SIN = !In<TIn>::kExactBf16;
-  constexpr bool FWD_DELTA = DELTA && !REV;
-  constexpr bool REV_DELTA = DELTA && REV;
   constexpr bool GV = YG != 0;           // value-side gate (either form)
-  constexpr bool SY = SIN || FWD_DELTA || GV;  // the Y plane carries a lo half (fp32 Y, v_new, Y~)
+  constexpr bool SY = SIN || GV;         // the Y plane carries a lo half (fp32 Y, Y~)
   constexpr bool XL = !GV;               // the X / Z planes carry a lo half (gated q / k)
-  static_assert(!GV || (!DELTA && !ST && !GK && !SIN), "YG: the bf16 full sweeps only");
+  static_assert(!GV || (!ST && !GK && !SIN), "YG: the bf16 full sweeps only");
   constexpr int LQ = KP + 8, LT = C + 8, LH = KP + 8;
   constexpr int NHT = (KP / 16) * (BV / 16) / NW;  // state tiles per wave (4, 2, 1), one K block
   constexpr int ES = sizeof(TIn);
@@ -97,14 +94,8 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
 
   __shared__ __attribute__((aligned(16))) uint16_t sX[(XL ? 2 : 1) * C * LQ];
   __shared__ __attribute__((aligned(16))) uint16_t sZ[(XL ? 2 : 1) * C * LQ];
-  // the reverse delta rule's w^T plane [K][C]; the forward delta rule's causal D tiles
-  // (10 tiles x 64 lanes x 16 B, written after the output pass while the Z~ plane is still
-  // read by the state update).  The other sweeps read Z~ transposed out of its row-major
-  // plane and need neither.
-  __shared__ __attribute__((aligned(16))) uint16_t sZT[REV_DELTA ? 2 * KP * LT : (FWD_DELTA ? 10 * 64 * 8 : 1)];
   __shared__ __attribute__((aligned(16))) uint16_t sYT[(SY ? 2 : 1) * BV * LT];
-  // (the reverse delta rule reuses sHT for the [BV][LT] dv_new^T plane: size for both)
-  constexpr int NHTS = 2 * BV * (REV_DELTA && LT > LH ? LT : LH);
+  constexpr int NHTS = 2 * BV * LH;
   __shared__ __attribute__((aligned(16))) uint16_t sHT[NHTS];
   __shared__ __attribute__((aligned(16))) float sTot[NSGH * KP]; // gate totals per segment group
   // GV: the output factors 2^(G - Gm) [C][BV + 4] and the gate totals of the 16-row groups
@@ -113,27 +104,17 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
   __shared__ __attribute__((aligned(16))) float sGvTot[GV ? 4 * BV : 1];
   // Causal D tiles of the chunk shared through LDS (bf16 hi/lo per lane, 10 tiles x 1 KB):
   // each tile is computed once instead of once per column-tile wave, and the work is spread
-  // evenly over the waves.  Only where the 160 KB budget allows (not the delta sweeps).
+  // evenly over the waves.  Only where the 160 KB budget allows.
   constexpr int LDS_BASE = 2 * ((XL ? 2 : 1) * C * LQ) * 2 +
-                           (REV_DELTA ? 2 * KP * LT * 2 : (FWD_DELTA ? 10 * 64 * 16 : 0)) +
                            (SY ? 2 : 1) * BV * LT * 2 + NHTS * 2 + NSGH * KP * 4 +
                            (GV ? (C * LE + 4 * BV) * 4 : 0);
-  constexpr bool SHARED_D = !DELTA && !ST && LDS_BASE + 10 * 64 * 16 <= 160 * 1024;
+  constexpr bool SHARED_D = !ST && LDS_BASE + 10 * 64 * 16 <= 160 * 1024;
   __shared__ __attribute__((aligned(16))) uint4 sDt[SHARED_D ? 10 * 64 : 1];
   __shared__ uint32_t sMx[NW];   // fp16 checkpoints: each wave's largest |S| (fp32 bits)
-  // (forward delta rule) 2^-Gm of channel c, Gm = Gamma / 2, sits in the padding columns of the
-  // X hi plane (row c / 4, word c % 4): no MFMA fragment or staging write touches columns >= KP
-  auto egm_at = [&](int c4) { return (float*)(sX + (c4 >> 2) * LQ + KP); };
-
   const Plane PX{sX, XL ? sX + C * LQ : sX, LQ};
   const Plane PZ{sZ, XL ? sZ + C * LQ : sZ, LQ};
   const Plane PYt{sYT, SY ? sYT + BV * LT : sYT, LT};
   const Plane PHt{sHT, sHT + BV * LH, LH};
-  // reverse delta rule: once the output pass is done, w^T [K][C] goes to sZT and
-  // dv_new^T [BV][C] reuses sHT
-  const Plane PWt{sZT, sZT + KP * LT, LT};
-  const Plane PDt{sHT, sHT + BV * LT, LT};
-
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform
   const int l16 = lane & 15, lg = lane >> 4;
@@ -237,7 +218,7 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
   }
   // reverse-time recurrence (gshift): the state entering the last token is h0 decayed by
   // that token's gate
-  constexpr bool RSH = REV && !ST && !DELTA;
+  constexpr bool RSH = REV && !ST;
   const bool gsh = RSH && p.gshift;
   if (gsh && L > 0) {
     const size_t el = (size_t)(row0 + L - 1) * H + hh;
@@ -266,7 +247,7 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
   // loaded into the set just consumed.  One set is issued a whole chunk ahead (after B2),
   // which covers the load latency; the second set pays off only for the instances whose
   // output block keeps fewer registers live (bf16 without shared D tiles).
-  constexpr int PF = (DELTA || SIN || SHARED_D) ? 1 : 2;
+  constexpr int PF = (SIN || SHARED_D) ? 1 : 2;
   struct Raw {
     typename Wd::W4 rq[RPT], rk[RPT];
     uint4 rg[RPT];
@@ -308,23 +289,21 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
       else if (gk_mode) rs.rg[i] = bld128(Rg, go, gs);
       else rs.rg[i] = make_uint4(bld32(Rg, go, gs), 0u, 0u, 0u);
     }
-    if constexpr (!FWD_DELTA) {
-      const rsrc_t Ry = chunk_rsrc((const TIn*)p.y, e0, nval, (int)rowV, V);
+    const rsrc_t Ry = chunk_rsrc((const TIn*)p.y, e0, nval, (int)rowV, V);
 #pragma unroll
-      for (int i = 0; i < YR; ++i) rs.ry[i] = Wd::ld2(Ry, offY, i * rowV * ES);
-      if constexpr (YG == 1) {
-        const rsrc_t Rgv = chunk_rsrc(p.g, e0, nval, (int)rowV, V);
+    for (int i = 0; i < YR; ++i) rs.ry[i] = Wd::ld2(Ry, offY, i * rowV * ES);
+    if constexpr (YG == 1) {
+      const rsrc_t Rgv = chunk_rsrc(p.g, e0, nval, (int)rowV, V);
 #pragma unroll
-        for (int i = 0; i < YR; ++i) rs.rgv[i] = bld64(Rgv, offYg, i * rowV * 4);
-      } else if constexpr (YG == 2) {
-        // one word per row (the constant gate reads nothing: out of range)
-        const rsrc_t Rgs = chunk_rsrc(p.g, e0, nval, H, 1);
+      for (int i = 0; i < YR; ++i) rs.rgv[i] = bld64(Rgv, offYg, i * rowV * 4);
+    } else if constexpr (YG == 2) {
+      // one word per row (the constant gate reads nothing: out of range)
+      const rsrc_t Rgs = chunk_rsrc(p.g, e0, nval, H, 1);
 #pragma unroll
-        for (int i = 0; i < YR; ++i) {
-          const bool ok = yg_s;
-          const uint32_t w = bld32(Rgs, ok ? (uint32_t)(yseg * YR) * H * 4u : kOOB, i * H * 4);
-          rs.rgv[i] = make_uint2(w, w);
-        }
+      for (int i = 0; i < YR; ++i) {
+        const bool ok = yg_s;
+        const uint32_t w = bld32(Rgs, ok ? (uint32_t)(yseg * YR) * H * 4u : kOOB, i * H * 4);
+        rs.rgv[i] = make_uint2(w, w);
       }
     }
   };
@@ -341,49 +320,6 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
     const int c = cidx(it);
     const int t0 = c * C;
     const int nval = min(C, L - t0);
-
-    // ---------------- forward delta rule: w rows of this wave's token block (MFMA row layout)
-    // and u in the result layout, issued now so their latency overlaps the staging
-    // (bf16 only: the fp32 instantiation has no register room and loads them after B2)
-    constexpr bool HOIST = FWD_DELTA && !SIN;
-    uint4 wraw[KP / 32][2];
-    float ur[2][4];
-    auto load_wu = [&]() {
-      const size_t e0 = (size_t)(row0 + t0) * H + hh;
-      const rsrc_t Rw = chunk_rsrc(p.w, e0, nval, (int)rowK, LDK);
-      const rsrc_t Ru = chunk_rsrc(p.u, e0, nval, (int)rowV, V);
-      const int trow = 16 * R + l16;
-#pragma unroll
-      for (int kc = 0; kc < KP / 32; ++kc) {
-        const int k0 = 32 * kc + 8 * lg;
-        const uint32_t o = k0 < K ? ((uint32_t)trow * rowK + k0) * 4u : kOOB;
-        wraw[kc][0] = bld128(Rw, o, 0);
-        wraw[kc][1] = bld128(Rw, o == kOOB ? kOOB : o + 16u, 0);
-      }
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int vv = vt * BV + 16 * (2 * nh + j) + l16;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int tok = 16 * R + 4 * lg + r;
-          ur[j][r] = __uint_as_float(bld32(Ru, vv < V ? ((uint32_t)tok * rowV + vv) * 4u : kOOB, 0));
-        }
-      }
-    };
-    if constexpr (HOIST) load_wu();
-
-    // ---------------- reverse delta rule: w rows of this thread, consumed after barrier B3
-    float4 rw[RPT];
-    if constexpr (REV_DELTA) {
-      const size_t e0 = (size_t)(row0 + t0) * H + hh;
-      const rsrc_t Rw = chunk_rsrc(p.w, e0, nval, (int)rowK, LDK);
-#pragma unroll
-      for (int i = 0; i < RPT; ++i) {
-        const uint4 x = bld128(Rw, offG, i * rowK * 4);
-        rw[i] = make_float4(__uint_as_float(x.x), __uint_as_float(x.y), __uint_as_float(x.z),
-                            __uint_as_float(x.w));
-      }
-    }
 
     // ---------------- gate cumsum: thread rows, a DPP scan over the half-wave's row
     // segments, then segment-group totals through LDS
@@ -481,11 +417,6 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
     float gm[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) gm[j] = 0.5f * gam[j];
-    if constexpr (FWD_DELTA) {
-      if (seg == 0)
-        *(float4*)egm_at(c0) =
-            make_float4(fast_exp2(-gm[0]), fast_exp2(-gm[1]), fast_exp2(-gm[2]), fast_exp2(-gm[3]));
-    }
     // Gamma of this lane's state rows kr = 16 msb + 4 lg + r
     float sgam[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -498,7 +429,7 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
     for (int r = 0; r < 4; ++r) {
       const float g2 = 0.5f * sgam[r];
       sga[r] = fast_exp2(sgam[r]);
-      sal[r] = REV ? fast_exp2(sgam[r] - g2) : (DELTA ? 1.f : scale) * fast_exp2(g2);
+      sal[r] = REV ? fast_exp2(sgam[r] - g2) : scale * fast_exp2(g2);
       sbe[r] = REV ? scale * fast_exp2(g2) : fast_exp2(sgam[r] - g2);
     }
 
@@ -555,7 +486,7 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
             xk[j] = kv[j];
           } else {
             const float Gv = G[i][j] + pre[j];
-            xq[j] = (FWD_DELTA ? scale : 1.f) * qv[j] * fast_exp2(Gv - gm[j]);
+            xq[j] = qv[j] * fast_exp2(Gv - gm[j]);
             xk[j] = kv[j] * fast_exp2(gm[j] - Gv);
           }
         }
@@ -567,24 +498,22 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
         *(uint2*)(PZ.hi + (r0 + i) * PZ.ld + c0) = make_uint2(zh[i][0], zh[i][1]);
         if constexpr (XL) *(uint2*)(PZ.lo + (r0 + i) * PZ.ld + c0) = make_uint2(zl[i][0], zl[i][1]);
       }
-      if constexpr (!FWD_DELTA) {
-        float ya[YR], yb[YR];
+      float ya[YR], yb[YR];
 #pragma unroll
-        for (int i = 0; i < YR; ++i) unpack2(rs.ry[i], ya[i], yb[i]);
-        if constexpr (GV) {
-          // Y~ = Y 2^(s(Gm - G)) into the Y plane; the output factor 2^(s(G - Gm)) into sE
+      for (int i = 0; i < YR; ++i) unpack2(rs.ry[i], ya[i], yb[i]);
+      if constexpr (GV) {
+        // Y~ = Y 2^(s(Gm - G)) into the Y plane; the output factor 2^(s(G - Gm)) into sE
 #pragma unroll
-          for (int i = 0; i < YR; ++i) {
-            float ga = gvc[i][0] + prev[0] - gmv[0], gb = gvc[i][1] + prev[1] - gmv[1];
-            if constexpr (REV) { ga = -ga; gb = -gb; }
-            ya[i] *= fast_exp2(-ga);
-            yb[i] *= fast_exp2(-gb);
-            *(float2*)(sE + (yseg * YR + i) * LE + 2 * yc) = make_float2(fast_exp2(ga), fast_exp2(gb));
-          }
+        for (int i = 0; i < YR; ++i) {
+          float ga = gvc[i][0] + prev[0] - gmv[0], gb = gvc[i][1] + prev[1] - gmv[1];
+          if constexpr (REV) { ga = -ga; gb = -gb; }
+          ya[i] *= fast_exp2(-ga);
+          yb[i] *= fast_exp2(-gb);
+          *(float2*)(sE + (yseg * YR + i) * LE + 2 * yc) = make_float2(fast_exp2(ga), fast_exp2(gb));
         }
-        put_n<SY, YR>(PYt, 2 * yc, yseg * YR, ya);
-        put_n<SY, YR>(PYt, 2 * yc + 1, yseg * YR, yb);
       }
+      put_n<SY, YR>(PYt, 2 * yc, yseg * YR, ya);
+      put_n<SY, YR>(PYt, 2 * yc + 1, yseg * YR, yb);
     }
     __syncthreads();  // B2: all planes visible
 
@@ -598,25 +527,7 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
     // ---------------- prefetch the chunk PF steps ahead while this one is computed
     if (it + PF < NTs) load_chunk(cidx(it + PF), rs);
 
-    // ---------------- reverse delta rule: first half of the state update (Z~^T Y)
-    f32x4 d1[NHT];
-    if constexpr (REV_DELTA) {
-#pragma unroll
-      for (int i = 0; i < NHT; ++i) {
-        const int nn = (wave * NHT + i) % (BV / 16);
-        d1[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kc = 0; kc < C / 32; ++kc) {
-          const bf16x8 bh = PYt.hi8(16 * nn + l16, 32 * kc + 8 * lg);
-          bf16x8 bl = bh;
-          if constexpr (SY) bl = PYt.lo8(16 * nn + l16, 32 * kc + 8 * lg);
-          d1[i] = mma<true, SY>(d1[i], tr_read8(PZ.hi, PZ.ld, 32 * kc, 16 * msb, lane),
-                                tr_read8(PZ.lo, PZ.ld, 32 * kc, 16 * msb, lane), bh, bl);
-        }
-      }
-    }
-
-    // ---------------- state update: S = 2^Gamma S + beta (Z~^T Y) [- w^T dv_new]
+    // ---------------- state update: S = 2^Gamma S + beta (Z~^T Y)
     auto state_update = [&]() {
       // (shared-D build) every fragment first, then the NHT independent accumulation chains
       // interleaved term by term, so neither LDS latency nor MFMA dependencies serialise
@@ -654,12 +565,7 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
       for (int i = 0; i < NHT; ++i) {
         const int nn = (wave * NHT + i) % (BV / 16);
         f32x4 d = {0.f, 0.f, 0.f, 0.f};
-        if constexpr (REV_DELTA) {
-#pragma unroll
-          for (int kc = 0; kc < C / 32; ++kc)
-            d = mma<true, true>(d, PWt.hi8(16 * msb + l16, 32 * kc + 8 * lg), PWt.lo8(16 * msb + l16, 32 * kc + 8 * lg),
-                                PDt.hi8(16 * nn + l16, 32 * kc + 8 * lg), PDt.lo8(16 * nn + l16, 32 * kc + 8 * lg));
-        } else if constexpr (!SHARED_D) {
+        if constexpr (!SHARED_D) {
 #pragma unroll
           for (int kc = 0; kc < C / 32; ++kc) {
             const bf16x8 bh = PYt.hi8(16 * nn + l16, 32 * kc + 8 * lg);
@@ -675,8 +581,7 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          if constexpr (REV_DELTA) S[i][r] = sga[r] * S[i][r] + sbe[r] * d1[i][r] - d[r];
-          else if constexpr (GV) S[i][r] = cga[i] * S[i][r] + cbe[i] * d[r];
+          if constexpr (GV) S[i][r] = cga[i] * S[i][r] + cbe[i] * d[r];
           else S[i][r] = sga[r] * S[i][r] + sbe[r] * d[r];
         }
       }
@@ -697,7 +602,6 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
     };
     if constexpr (!SHARED_D) load_x();
     // D tiles (P, R) on the causal side: lane holds D[16P+4lg+r][16R+l16]
-    const float dsc = FWD_DELTA ? 1.f : scale;   // the delta forward folds scale into X
     uint2 dh[4], dl[4];
     // causal D tile t = Rc (Rc + 1) / 2 + Pc, Pc <= Rc (Rc = R, Pc = P forward; 3 - R, 3 - P
     // reverse), packed bf16 hi / lo per lane; three independent MFMA chains (lo.hi, hi.lo,
@@ -735,7 +639,7 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
       for (int r = 0; r < 4; ++r) {
         const int pp = 16 * Pt + 4 * lg + r;
         const bool keep = REV ? (pp >= rr) : (pp <= rr);
-        acc[r] = keep ? acc[r] * dsc : 0.f;
+        acc[r] = keep ? acc[r] * scale : 0.f;
       }
       uint2 th, tl;
       acc_to_bf16x4(acc, th, tl);
@@ -755,10 +659,6 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
         }
       }
     };
-    // forward delta rule (no LDS left for the shared tiles): the D tiles are computed now, in
-    // the same even split (wave w: tiles w, w + 8), and handed over through the Z plane once
-    // the v_new phase below has passed B3 (Z is not read after the D tiles)
-    uint4 dz[2];
     if constexpr (SHARED_D) {
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
@@ -770,12 +670,6 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
       __syncthreads();  // B3: D tiles visible
       load_x();
       read_d(sDt);
-    } else if constexpr (FWD_DELTA) {
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int t = wave + 8 * u;
-        if (t < 10) dz[u] = dtile(t);
-      }
     } else {
 #pragma unroll
     for (int P = 0; P < 4; ++P) {
@@ -793,159 +687,54 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
         for (int r = 0; r < 4; ++r) {
           const int pp = 16 * P + 4 * lg + r;
           const bool keep = REV ? (pp >= rr) : (pp <= rr);
-          t[r] = keep ? t[r] * dsc : 0.f;
+          t[r] = keep ? t[r] * scale : 0.f;
         }
         acc_to_bf16x4(t, dh[P], dl[P]);
       }
     }
     }  // SHARED_D
 
-    if constexpr (FWD_DELTA) {
-      // v_new = u - w S for (token block R, column tiles 2nh, 2nh+1).  The A operand
-      // w 2^-Gm is read straight from HBM in the MFMA row layout (against H^T = 2^Gm S).
-      const size_t e0 = (size_t)(row0 + t0) * H + hh;
-      const rsrc_t Rvn = chunk_rsrc(p.y32, e0, nval, (int)rowV, V);
-      const rsrc_t Rw = chunk_rsrc(p.w, e0, nval, (int)rowK, LDK);
-      const rsrc_t Ru = chunk_rsrc(p.u, e0, nval, (int)rowV, V);
-      bf16x8 wh[KP / 32], wl[KP / 32];
+    // out^T tiles (nn, R); lane writes out[token 16R + l16][v = 16 nn + 4 lg + 0..3]
+    const int tok = 16 * R + l16;
+    const size_t eo = (size_t)(row0 + t0) * H + hh;
+    const rsrc_t Ro = chunk_rsrc((const TIn*)p.out, eo, nval, (int)rowV, V);
+    const uint32_t oo = ((uint32_t)tok * rowV + vt * BV + 4 * lg) * ES;
 #pragma unroll
-      for (int kc = 0; kc < KP / 32; ++kc) {
-        const int k0 = 32 * kc + 8 * lg;
-        float a[8];
-        if constexpr (HOIST) {
-          unpack4(wraw[kc][0], a);
-          unpack4(wraw[kc][1], a + 4);
-        } else {
-          const int trow = 16 * R + l16;
-          const uint32_t o = k0 < K ? ((uint32_t)trow * rowK + k0) * 4u : kOOB;
-          unpack4(bld128(Rw, o, 0), a);
-          unpack4(bld128(Rw, o == kOOB ? kOOB : o + 16u, 0), a + 4);
+    for (int j = 0; j < 2; ++j) {
+      const int nn = 2 * nh + j;
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kc = 0; kc < KP / 32; ++kc)
+        acc = mma<true, XL>(acc, PHt.hi8(16 * nn + l16, 32 * kc + 8 * lg),
+                            PHt.lo8(16 * nn + l16, 32 * kc + 8 * lg), xh[kc], xl[kc]);
+      // out^T += Y^T D  (contraction over p, two 16-blocks per MFMA)
+#pragma unroll
+      for (int Pp = 0; Pp < 2; ++Pp) {
+        const int P0 = 2 * Pp, P1 = 2 * Pp + 1;
+        const bool live = REV ? (P1 >= R) : (P0 <= R);
+        if (live) {
+          const bf16x8 ah = PYt.hi44(16 * nn + l16, 16 * P0 + 4 * lg, 16 * P1 + 4 * lg);
+          bf16x8 al = ah;
+          if constexpr (SY) al = PYt.lo44(16 * nn + l16, 16 * P0 + 4 * lg, 16 * P1 + 4 * lg);
+          acc = mma<SY, true>(acc, ah, al, cat44(dh[P0], dh[P1]), cat44(dl[P0], dl[P1]));
         }
-        const float4 g0 = *(const float4*)egm_at(k0), g1 = *(const float4*)egm_at(k0 + 4);
-        const float eg[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
-        uint32_t h4[4], l4[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) split_bf16x2(a[2 * e] * eg[2 * e], a[2 * e + 1] * eg[2 * e + 1], h4[e], l4[e]);
-        wh[kc] = __builtin_bit_cast(bf16x8, make_uint4(h4[0], h4[1], h4[2], h4[3]));
-        wl[kc] = __builtin_bit_cast(bf16x8, make_uint4(l4[0], l4[1], l4[2], l4[3]));
       }
+      if constexpr (RSH) {
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int nn = 2 * nh + j;
-        const int vv = vt * BV + 16 * nn + l16;
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kc = 0; kc < KP / 32; ++kc)
-          acc = mma<true, true>(acc, wh[kc], wl[kc], PHt.hi8(16 * nn + l16, 32 * kc + 8 * lg),
-                                PHt.lo8(16 * nn + l16, 32 * kc + 8 * lg));
-        // lane holds (token 16R + 4lg + r, column 16nn + l16)
-        float vn[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int tok = 16 * R + 4 * lg + r;
-          const uint32_t o = vv < V ? ((uint32_t)tok * rowV + vv) * 4u : kOOB;
-          vn[r] = (HOIST ? ur[j][r] : __uint_as_float(bld32(Ru, o, 0))) - acc[r];
-          bst32(Rvn, __float_as_uint(vn[r]), o, 0);
-        }
-        put_n<true, 4>(PYt, 16 * nn + l16, 16 * R + 4 * lg, vn);
+        for (int r = 0; r < 4; ++r) acc[r] *= p.oscale;
       }
-      __syncthreads();  // B3: v_new^T plane complete
-      uint4* zD = (uint4*)sZT;
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int t = wave + 8 * u;
-        if (t < 10) zD[t * 64 + lane] = dz[u];
+      if constexpr (GV) {
+        const float4 e4 = *(const float4*)(sE + tok * LE + 16 * nn + 4 * lg);
+        acc[0] *= e4.x; acc[1] *= e4.y; acc[2] *= e4.z; acc[3] *= e4.w;
       }
-      __syncthreads();  // B3b: D tiles visible
-      read_d(zD);
-    }
-
-    if constexpr (REV_DELTA) {
-      // dv_new = k~ (alpha dS) + D^T dO, token-major: lane holds (token 16R + 4lg + r,
-      // column 16nn + l16); stored transposed per chunk ([V][C]) and kept for the update
-      f32x4 dvn[2];
-      const rsrc_t Rd = make_rsrc(p.y32 + ((size_t)(cbase + c) * H + hh) * V * C, (long long)V * C * 4);
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int nn = 2 * nh + j;
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kc = 0; kc < KP / 32; ++kc)
-          acc = mma<true, true>(acc, xh[kc], xl[kc], PHt.hi8(16 * nn + l16, 32 * kc + 8 * lg),
-                                PHt.lo8(16 * nn + l16, 32 * kc + 8 * lg));
-#pragma unroll
-        for (int Pp = 0; Pp < 2; ++Pp) {
-          const int P0 = 2 * Pp, P1 = 2 * Pp + 1;
-          if (P1 >= R) {
-            const bf16x8 bh = PYt.hi44(16 * nn + l16, 16 * P0 + 4 * lg, 16 * P1 + 4 * lg);
-            bf16x8 bl = bh;
-            if constexpr (SY) bl = PYt.lo44(16 * nn + l16, 16 * P0 + 4 * lg, 16 * P1 + 4 * lg);
-            acc = mma<true, SY>(acc, cat44(dh[P0], dh[P1]), cat44(dl[P0], dl[P1]), bh, bl);
-          }
-        }
-        dvn[j] = acc;
-        const int vv = vt * BV + 16 * nn + l16;
-        bst128(Rd, make_uint4(__float_as_uint(acc[0]), __float_as_uint(acc[1]), __float_as_uint(acc[2]),
-                              __float_as_uint(acc[3])),
-               vv < V ? ((uint32_t)vv * C + 16 * R + 4 * lg) * 4u : kOOB, 0);
-      }
-      __syncthreads();  // B3: every wave is done with X, Z, Z^T, Y^T and H^T
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const float x[4] = {dvn[j][0], dvn[j][1], dvn[j][2], dvn[j][3]};
-        put_n<true, 4>(PDt, 16 * (2 * nh + j) + l16, 16 * R + 4 * lg, x);
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        float x[RPT];
-#pragma unroll
-        for (int i = 0; i < RPT; ++i) x[i] = j == 0 ? rw[i].x : (j == 1 ? rw[i].y : (j == 2 ? rw[i].z : rw[i].w));
-        put_n<true, RPT>(PWt, c0 + j, r0, x);
-      }
-      __syncthreads();  // B4: w^T and dv_new^T planes visible
-    } else {
-      // out^T tiles (nn, R); lane writes out[token 16R + l16][v = 16 nn + 4 lg + 0..3]
-      const int tok = 16 * R + l16;
-      const size_t eo = (size_t)(row0 + t0) * H + hh;
-      const rsrc_t Ro = chunk_rsrc((const TIn*)p.out, eo, nval, (int)rowV, V);
-      const uint32_t oo = ((uint32_t)tok * rowV + vt * BV + 4 * lg) * ES;
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int nn = 2 * nh + j;
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kc = 0; kc < KP / 32; ++kc)
-          acc = mma<true, XL>(acc, PHt.hi8(16 * nn + l16, 32 * kc + 8 * lg),
-                              PHt.lo8(16 * nn + l16, 32 * kc + 8 * lg), xh[kc], xl[kc]);
-        // out^T += Y^T D  (contraction over p, two 16-blocks per MFMA)
-#pragma unroll
-        for (int Pp = 0; Pp < 2; ++Pp) {
-          const int P0 = 2 * Pp, P1 = 2 * Pp + 1;
-          const bool live = REV ? (P1 >= R) : (P0 <= R);
-          if (live) {
-            const bf16x8 ah = PYt.hi44(16 * nn + l16, 16 * P0 + 4 * lg, 16 * P1 + 4 * lg);
-            bf16x8 al = ah;
-            if constexpr (SY) al = PYt.lo44(16 * nn + l16, 16 * P0 + 4 * lg, 16 * P1 + 4 * lg);
-            acc = mma<SY, true>(acc, ah, al, cat44(dh[P0], dh[P1]), cat44(dl[P0], dl[P1]));
-          }
-        }
-        if constexpr (RSH) {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) acc[r] *= p.oscale;
-        }
-        if constexpr (GV) {
-          const float4 e4 = *(const float4*)(sE + tok * LE + 16 * nn + 4 * lg);
-          acc[0] *= e4.x; acc[1] *= e4.y; acc[2] *= e4.z; acc[3] *= e4.w;
-        }
-        const int v0 = vt * BV + 16 * nn + 4 * lg;
-        if (VAR != 0 || p.acc_mode == 0) {
-          Wd::st4(Ro, acc, v0 < V ? oo : kOOB, (uint32_t)(16 * nn * ES));
-        } else {
-          // channel slices: the fp32 sum of the slices' outputs (element offset as oo's)
-          const rsrc_t Ra = chunk_rsrc(p.acc32, eo, nval, (int)rowV, V);
-          const uint32_t fo = (v0 < V) ? ((uint32_t)tok * rowV + v0) * 4u : kOOB;
-          acc_slice_t<TIn>(Ro, Ra, acc, fo, v0 < V ? oo : kOOB, (uint32_t)(16 * nn * ES), p.acc_mode);
-        }
+      const int v0 = vt * BV + 16 * nn + 4 * lg;
+      if (VAR != 0 || p.acc_mode == 0) {
+        Wd::st4(Ro, acc, v0 < V ? oo : kOOB, (uint32_t)(16 * nn * ES));
+      } else {
+        // channel slices: the fp32 sum of the slices' outputs (element offset as oo's)
+        const rsrc_t Ra = chunk_rsrc(p.acc32, eo, nval, (int)rowV, V);
+        const uint32_t fo = (v0 < V) ? ((uint32_t)tok * rowV + v0) * 4u : kOOB;
+        acc_slice_t<TIn>(Ro, Ra, acc, fo, v0 < V ? oo : kOOB, (uint32_t)(16 * nn * ES), p.acc_mode);
       }
     }
 
@@ -984,11 +773,9 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
   }
 }
 
-template <typename TIn, bool REV, bool DELTA>
+template <typename TIn, bool REV>
 hipError_t launch_gla_sweep(const SweepParams& p, hipStream_t s) {
-  if constexpr (!DELTA) {
-    if (gla_strip_eligible(p)) return launch_gla_strip<TIn, REV, false>(p, s);
-  }
+  if (gla_strip_eligible(p)) return launch_gla_strip<TIn, REV, false>(p, s);
   // fp16 checkpoints: whole-width state rows with the plain layout (ckpt_par 0, no slices)
   const bool plain = !p.acc_mode && !p.ldk;
   if (p.ckpt16 && (!p.ckpt || !p.ckpt_scale || p.ckpt_par || !plain)) return hipErrorInvalidValue;
@@ -996,26 +783,15 @@ hipError_t launch_gla_sweep(const SweepParams& p, hipStream_t s) {
   if (var == 1 && !std::is_same<TIn, uint16_t>::value) return hipErrorInvalidValue;
   const int kp = p.K <= 32 ? 32 : (p.K <= 64 ? 64 : 128);
   dim3 grid(p.NV * p.H * p.N);
-  const bool gk = DELTA || p.gate_mode == kGateK;
+  const bool gk = p.gate_mode == kGateK;
 #define TOPS_SWEEP(KPV, GKV) \
-  hipLaunchKernelGGL((gla_sweep_kernel<TIn, KPV, REV, DELTA, false, GKV>), grid, dim3(512), 0, s, p)
-  // the delta sweeps (KDA) and the bf16 value-side-gate sweeps are compiled per feature set
-#define TOPS_SWEEP_V(KPV, GKV, YGV) \
-  if (var == 1) { \
-    if constexpr (std::is_same<TIn, uint16_t>::value) \
-      hipLaunchKernelGGL((gla_sweep_kernel<TIn, KPV, REV, DELTA, false, GKV, YGV, 1>), grid, dim3(512), 0, s, p); \
-  } else if (var == 2) hipLaunchKernelGGL((gla_sweep_kernel<TIn, KPV, REV, DELTA, false, GKV, YGV, 2>), grid, dim3(512), 0, s, p); \
-  else hipLaunchKernelGGL((gla_sweep_kernel<TIn, KPV, REV, DELTA, false, GKV, YGV, 0>), grid, dim3(512), 0, s, p)
-  // fp16 checkpoints: the delta sweeps and the bf16 one-gate-per-token sweeps here, the
-  // per-channel-gate bf16 sweeps in the strip kernel (routed above)
-  const bool yg2 = std::is_same<TIn, uint16_t>::value && !DELTA && !gk && !p.gshift &&
+  hipLaunchKernelGGL((gla_sweep_kernel<TIn, KPV, REV, false, GKV>), grid, dim3(512), 0, s, p)
+  // fp16 checkpoints: the bf16 one-gate-per-token sweeps here, the per-channel-gate bf16
+  // sweeps in the strip kernel (routed above)
+  const bool yg2 = std::is_same<TIn, uint16_t>::value && !gk && !p.gshift &&
                    (p.gate_mode == kGateS || p.gate_mode == kGateGamma);
-  if (var == 1 && !DELTA && !yg2) return hipErrorInvalidValue;
-  if constexpr (DELTA) {
-    if (kp == 32) { TOPS_SWEEP_V(32, true, 0); }
-    else if (kp == 64) { TOPS_SWEEP_V(64, true, 0); }
-    else { TOPS_SWEEP_V(128, true, 0); }
-  } else if (gk) {
+  if (var == 1 && !yg2) return hipErrorInvalidValue;
+  if (gk) {
     if (kp == 32) TOPS_SWEEP(32, true);
     else if (kp == 64) TOPS_SWEEP(64, true);
     else TOPS_SWEEP(128, true);
@@ -1023,8 +799,8 @@ hipError_t launch_gla_sweep(const SweepParams& p, hipStream_t s) {
              (p.gate_mode == kGateS || p.gate_mode == kGateGamma)) {
     // one gate per token (bf16): on the value side, q and k stay exact
 #define TOPS_SWEEP_YG(KPV, VARV) \
-  hipLaunchKernelGGL((gla_sweep_kernel<uint16_t, KPV, REV, false, false, false, 2, VARV>), grid, dim3(512), 0, s, p)
-    if constexpr (std::is_same<TIn, uint16_t>::value && !DELTA) {
+  hipLaunchKernelGGL((gla_sweep_kernel<uint16_t, KPV, REV, false, false, 2, VARV>), grid, dim3(512), 0, s, p)
+    if constexpr (std::is_same<TIn, uint16_t>::value) {
 #define TOPS_SWEEP_YGV(KPV) \
   if (var == 1) TOPS_SWEEP_YG(KPV, 1); else if (var == 2) TOPS_SWEEP_YG(KPV, 2); else TOPS_SWEEP_YG(KPV, 0)
       if (kp == 32) { TOPS_SWEEP_YGV(32); }
@@ -1038,7 +814,6 @@ hipError_t launch_gla_sweep(const SweepParams& p, hipStream_t s) {
     else if (kp == 64) TOPS_SWEEP(64, false);
     else TOPS_SWEEP(128, false);
   }
-#undef TOPS_SWEEP_V
 #undef TOPS_SWEEP
   return hipGetLastError();
 }
@@ -1048,7 +823,7 @@ hipError_t launch_gla_sweep_gv(const SweepParams& p, hipStream_t s) {
   const int kp = p.K <= 32 ? 32 : (p.K <= 64 ? 64 : 128);
   dim3 grid(p.NV * p.H * p.N);
 #define TOPS_SWEEP_GV(KPV) \
-  hipLaunchKernelGGL((gla_sweep_kernel<uint16_t, KPV, REV, false, false, false, 1>), grid, dim3(512), 0, s, p)
+  hipLaunchKernelGGL((gla_sweep_kernel<uint16_t, KPV, REV, false, false, 1>), grid, dim3(512), 0, s, p)
   if (kp == 32) TOPS_SWEEP_GV(32);
   else if (kp == 64) TOPS_SWEEP_GV(64);
   else TOPS_SWEEP_GV(128);
@@ -1061,7 +836,7 @@ hipError_t launch_gla_state_pass(const SweepParams& p, hipStream_t s) {
   const int kp = p.K <= 32 ? 32 : (p.K <= 64 ? 64 : 128);
   dim3 grid(p.NV * p.H * p.N);
 #define TOPS_STATE(KPV, GKV) \
-  hipLaunchKernelGGL((gla_sweep_kernel<TIn, KPV, REV, false, true, GKV>), grid, dim3(512), 0, s, p)
+  hipLaunchKernelGGL((gla_sweep_kernel<TIn, KPV, REV, true, GKV>), grid, dim3(512), 0, s, p)
   if (p.gate_mode == kGateK) {
     return launch_gla_strip_state<TIn, REV>(p, s);
   } else {
@@ -1080,16 +855,12 @@ template hipError_t launch_gla_state_pass<float, true>(const SweepParams&, hipSt
 template hipError_t launch_gla_state_pass<_Float16, false>(const SweepParams&, hipStream_t);
 template hipError_t launch_gla_state_pass<_Float16, true>(const SweepParams&, hipStream_t);
 
-template hipError_t launch_gla_sweep<uint16_t, false, false>(const SweepParams&, hipStream_t);
-template hipError_t launch_gla_sweep<uint16_t, true, false>(const SweepParams&, hipStream_t);
-template hipError_t launch_gla_sweep<float, false, false>(const SweepParams&, hipStream_t);
-template hipError_t launch_gla_sweep<float, true, false>(const SweepParams&, hipStream_t);
-template hipError_t launch_gla_sweep<_Float16, false, false>(const SweepParams&, hipStream_t);
-template hipError_t launch_gla_sweep<_Float16, true, false>(const SweepParams&, hipStream_t);
-template hipError_t launch_gla_sweep<uint16_t, false, true>(const SweepParams&, hipStream_t);
-template hipError_t launch_gla_sweep<uint16_t, true, true>(const SweepParams&, hipStream_t);
-template hipError_t launch_gla_sweep<float, false, true>(const SweepParams&, hipStream_t);
-template hipError_t launch_gla_sweep<float, true, true>(const SweepParams&, hipStream_t);
+template hipError_t launch_gla_sweep<uint16_t, false>(const SweepParams&, hipStream_t);
+template hipError_t launch_gla_sweep<uint16_t, true>(const SweepParams&, hipStream_t);
+template hipError_t launch_gla_sweep<float, false>(const SweepParams&, hipStream_t);
+template hipError_t launch_gla_sweep<float, true>(const SweepParams&, hipStream_t);
+template hipError_t launch_gla_sweep<_Float16, false>(const SweepParams&, hipStream_t);
+template hipError_t launch_gla_sweep<_Float16, true>(const SweepParams&, hipStream_t);
 
 }  // namespace tops
 

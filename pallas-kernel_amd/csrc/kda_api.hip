@@ -84,8 +84,8 @@ static int kda_fwd_impl(const void* q, const void* k, const void* v, const float
     sp.ckpt16 = 1;
     sp.ckpt_scale = h_scale;
   }
-  e = dtype == TOPS_BF16 ? launch_gla_sweep<uint16_t, false, true>(sp, s)
-                         : launch_gla_sweep<float, false, true>(sp, s);
+  e = dtype == TOPS_BF16 ? launch_gla_strip<uint16_t, false, true>(sp, s)
+                         : launch_gla_strip<float, false, true>(sp, s);
   if (e != hipSuccess) return tops_set_error(TOPS_ERR_LAUNCH, hipGetErrorString(e));
   return TOPS_OK;
 }
@@ -143,7 +143,7 @@ static int kda_bwd_impl(const void* q, const void* k, const void* v, const float
     sp.ckpt16 = 1;
     sp.ckpt_scale = dh_scale;
   }
-  hipError_t e = bf ? launch_gla_sweep<uint16_t, true, true>(sp, s) : launch_gla_sweep<float, true, true>(sp, s);
+  hipError_t e = bf ? launch_gla_strip<uint16_t, true, true>(sp, s) : launch_gla_strip<float, true, true>(sp, s);
   if (e != hipSuccess) return tops_set_error(TOPS_ERR_LAUNCH, hipGetErrorString(e));
   if (bf) {
     // 2+3. the WY backward and dq, dk, dg in one kernel (the WY parts through LDS)

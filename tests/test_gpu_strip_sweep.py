@@ -44,3 +44,46 @@ def test_strip_sweep_tile_edges(T, K, V, dt, cuda_device):
     for n, a, r in [(n, got[n], ref[n]) for n in ref] + [("o inf", oi, ref["o"]), ("ht inf", hi, ref["ht"])]:
         e, lim = rel(host(a), r), out_bound(r, dtype, a.dtype)
         assert e < lim, f"{n}: rel-err {e:.3e} vs oracle (bound {lim:.2e})"
+
+
+KDA_CASES = [(T, K, V, dt) for dt in ("bf16", "f32")
+             for T, K, V in ((1, 8, 8), (63, 40, 56), (65, 64, 72), (128, 72, 128),
+                             (129, 128, 120), (200, 128, 64))]
+
+
+@pytest.mark.parametrize("T,K,V,dt", KDA_CASES, ids=lambda x: str(x))
+def test_strip_sweep_delta_rule_tile_edges(T, K, V, dt, cuda_device):
+    """The delta-rule instances, forward (with checkpoints and without) and reverse, against
+    the oracle (tops/cpu/ops/kda/naive.py:121-313, chunk_bwd.py:525-668); gate gradients
+    against the scale of the k * dk terms they are differences of."""
+    import numpy as np
+    from oracle import kda as OK
+    from _inputs import kda_inputs
+    from tops.ops.kda import chunk_kda
+    dtype = {"bf16": torch.bfloat16, "f32": torch.float32}[dt]
+    B, H = 2, 2
+    d = kda_inputs(B, T, H, K, V, 700 + T, gate_div=4.0, h0=True, grads=True)
+    x = {n: to_dev(d[n], dtype, cuda_device).requires_grad_() for n in "qkv"}
+    x |= {n: to_dev(d[n], torch.float32, cuda_device).requires_grad_() for n in ("g", "beta", "h0")}
+    print(f"delta-rule strip sweep T={T} K={K} V={V} {dt}", flush=True)
+    sc = K ** -0.5
+    o, ht = chunk_kda(*(x[n] for n in ("q", "k", "v", "g", "beta")), scale=sc,
+                      initial_state=x["h0"], output_final_state=True)
+    torch.autograd.backward((o, ht), (to_dev(d["do"], dtype, cuda_device),
+                                      to_dev(d["dht"], torch.float32, cuda_device)))
+    with torch.no_grad():
+        oi, hi = chunk_kda(*(x[n] for n in ("q", "k", "v", "g", "beta")), scale=sc,
+                           initial_state=x["h0"], output_final_state=True)
+    s = {n: seen(d[n], dtype) for n in ("q", "k", "v", "do")}
+    a = (s["q"], s["k"], s["v"], np.float64(d["g"]), np.float64(d["beta"]))
+    ro, rht = OK.chunk_kda(*a, sc, np.float64(d["h0"]), True)
+    rq, rk, rv, rb, rg, rh0 = OK.chunk_kda_bwd(*a, sc, np.float64(d["h0"]), s["do"], np.float64(d["dht"]))
+    pairs = [("o", o, ro), ("ht", ht, rht), ("o inf", oi, ro), ("ht inf", hi, rht),
+             ("dq", x["q"].grad, rq), ("dk", x["k"].grad, rk), ("dv", x["v"].grad, rv),
+             ("dbeta", x["beta"].grad, rb), ("dg", x["g"].grad, rg), ("dh0", x["h0"].grad, rh0)]
+    for n, got, ref in pairs:
+        ref = np.asarray(ref)
+        err = np.linalg.norm(host(got) - ref)
+        base = np.linalg.norm(s["k"] * rk) if n == "dg" else np.linalg.norm(ref)
+        lim = out_bound(ref, dtype, torch.bfloat16 if n == "dg" and dt == "bf16" else got.dtype)
+        assert err <= lim * max(base, np.linalg.norm(ref)), f"{n}: rel-err {err / base:.3e} (bound {lim:.2e})"
