@@ -51,34 +51,11 @@
 #include <type_traits>
 
 #include "gla_sweep.h"
+#include "strip.h"
 #include "tops_common.h"
 #include "tops_hip.h"
 
 namespace tops {
-
-namespace {
-
-// piece swizzle of plane row r (see above); KP channels per row, 16-byte pieces
-template <int KP>
-__device__ __forceinline__ constexpr int swz(int r) {
-  const int b0 = r & 1, b1 = (r >> 1) & 1, b2 = (r >> 2) & 1, b3 = (r >> 3) & 1;
-  return KP == 128 ? (((b1 ^ b3) << 3) | (b0 << 2) | (b3 << 1) | b2)
-                   : (KP == 64 ? ((b1 << 2) | (b3 << 1) | b2) : ((b3 << 1) | b2));
-}
-
-__device__ __forceinline__ bf16x8 lds8(const uint16_t* p) {
-  return __builtin_bit_cast(bf16x8, *(const uint4*)p);
-}
-// transposed read: this lane's address of a 4-row block (tr_read8's lane layout), two blocks
-__device__ __forceinline__ bf16x8 tr2(const uint16_t* pa, const uint16_t* pb) {
-  typedef __attribute__((address_space(3))) v4i16 lds_v4;
-  const v4i16 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4*)pa);
-  const v4i16 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4*)pb);
-  const uint2 ua = __builtin_bit_cast(uint2, a), ub = __builtin_bit_cast(uint2, b);
-  return __builtin_bit_cast(bf16x8, make_uint4(ua.x, ua.y, ub.x, ub.y));
-}
-
-}  // namespace
 
 // Phase clocks (a library built with -DTOPS_PHASE_CLOCKS only; the regular build compiles
 // none of this): per wave, the shader clock (s_memtime) summed over the chunks, slots 0 work
@@ -230,14 +207,6 @@ __global__ __launch_bounds__(512) void gla_strip_kernel(SweepParams p) {
     uint2 h, l;
     acc_to_bf16x4(a, h, l);
     sDt[(Rc * (Rc + 1) / 2 + Pc) * 64 + lane] = make_uint4(h.x, h.y, l.x, l.y);
-  };
-
-  // factor of a checkpoint tile from the wave maxima: 2^(14 - e), e the largest exponent
-  auto ckpt_scale = [&]() {
-    const uint32_t m = max(max(sMx[0], sMx[1]), max(sMx[2], sMx[3]));
-    int ex = (int)((m >> 23) & 0xffu) - 127;
-    ex = ex < -100 ? -100 : ex;
-    return __uint_as_float((uint32_t)(141 - ex) << 23);
   };
 
   if (wave >= 4) {
@@ -466,7 +435,7 @@ __global__ __launch_bounds__(512) void gla_strip_kernel(SweepParams p) {
         }
         return;
       }
-      const float sinv = ckpt_scale();
+      const float sinv = ckpt_tile_scale(sMx);
       const size_t slot = (size_t)(cbase + c) * H + hh;
       if (ptid == 0) p.ckpt_scale[slot * p.NV + vt] = 1.f / sinv;   // powers of two
       const rsrc_t R = make_rsrc((uint16_t*)p.ckpt + slot * LDK * V, (long long)K * V * 2);
@@ -621,7 +590,7 @@ __global__ __launch_bounds__(512) void gla_strip_kernel(SweepParams p) {
   };
   auto store_ckpt = [&](int c) {
     if constexpr (CK16 && DELTA) {
-      const float sinv = ckpt_scale();
+      const float sinv = ckpt_tile_scale(sMx);
       if (tid == 0) p.ckpt_scale[((size_t)(cbase + c) * H + hh) * p.NV + vt] = 1.f / sinv;
 #pragma unroll
       for (int kc = 0; kc < KC; ++kc) {

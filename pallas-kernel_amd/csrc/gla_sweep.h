@@ -78,6 +78,12 @@ hipError_t launch_gla_strip(const SweepParams& p, hipStream_t s);
 template <typename TIn, bool REV>
 hipError_t launch_gla_strip_state(const SweepParams& p, hipStream_t s);
 
+// The strip-specialised sweep for one gate per token (gla_strip_s.hip; bf16): full or, with
+// state_only, the state pass.
+bool gla_strip_s_eligible(const SweepParams& p);
+template <bool REV>
+hipError_t launch_gla_strip_s(const SweepParams& p, bool state_only, hipStream_t s);
+
 // Sweep with the gate on the value side (g = gv [B,T,H,V], bf16 inputs), forward or (REV)
 // the state-gradient recurrence: see gla_sweep.hip.
 template <bool REV>

@@ -32,13 +32,12 @@
 // column tiles 2 (w % 2), 2 (w % 2) + 1 (the two waves of a token block both compute its
 // intra-chunk D tiles: MFMA has the headroom, a split would cost a barrier).
 //
-// YG (bf16): the gate is applied on the value side.  YG = 1 (forward): one log-gate per
-// (token, V column) (fused_recurrent_gla's gv), S[:, v] <- 2^gv S[:, v] + k v^T.  YG = 2
-// (forward and reverse): one log-gate per token (simple GLA's g [B,T,H], or g_gamma [H]),
-// which factors out of every q.k product: D[i][j] = 2^(G_i - G_j) (q_i.k_j).  Either way q and
-// k enter ungated (exact bf16: the X / Z planes carry no lo half), Y~ = Y 2^(s(Gm - G)) is
-// split into hi / lo (s = 1 forward, -1 reverse), every output element is multiplied by
-// 2^(s(G - Gm)) of its (token, column) from an fp32 LDS plane, and S decays per column:
+// GV (bf16): the gate is applied on the value side, one log-gate per (token, V column)
+// (fused_recurrent_gla's gv), S[:, v] <- 2^gv S[:, v] + k v^T, and its state-gradient
+// recurrence.  q and k enter ungated (exact bf16: the X / Z planes carry no lo half),
+// Y~ = Y 2^(s(Gm - G)) is split into hi / lo (s = 1 forward, -1 reverse), every output element
+// is multiplied by 2^(s(G - Gm)) of its (token, column) from an fp32 LDS plane, and S decays
+// per column:
 //   forward:  o^T = (scale 2^Gm S)^T q^T + v~^T M,  S = 2^Gamma S + 2^(Gamma-Gm) (k^T v~)
 //   reverse:  dv^T = (2^(Gamma-Gm) S)^T k^T + dO~^T M,  S = 2^Gamma S + scale 2^Gm (q^T dO~)
 // with M[i][j] = scale q_i.k_j on the causal side.
@@ -61,10 +60,7 @@ namespace tops {
 // GK: the per-channel gate mode only (kGateK, the GLA and KDA path), compiled on its own so
 // that the hot path carries no gate-mode branches; !GK serves the per-token and constant
 // gates (kGateS, kGateGamma, kGateGammaK) chosen at run time.
-// VAR selects the features an instance compiles (as in gla_strip.hip): 1 = fp16
-// checkpoints of every chunk, whole-width rows, no slices; 2 = no checkpoints and no slices;
-// 0 = the rest (fp32 or paired checkpoints, channel slices; no fp16 checkpoints).
-template <typename TIn, int KP, bool REV, bool ST, bool GK, int YG = 0, int VAR = 0>
+template <typename TIn, int KP, bool REV, bool ST, bool GK, bool GV = false>
 __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
   constexpr int NW = 8;                  // wave64s per workgroup
   constexpr int NTH = 64 * NW;
@@ -80,10 +76,9 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
   static_assert(NQ % CQL == 0, "KP must be a multiple of 32");
   static_assert(CQL == 8 && SGL == 4, "the segment scan takes 8 column quads x 4 segments");
   constexpr bool SIN = !In<TIn>::kExactBf16;
-  constexpr bool GV = YG != 0;           // value-side gate (either form)
   constexpr bool SY = SIN || GV;         // the Y plane carries a lo half (fp32 Y, Y~)
   constexpr bool XL = !GV;               // the X / Z planes carry a lo half (gated q / k)
-  static_assert(!GV || (!ST && !GK && !SIN), "YG: the bf16 full sweeps only");
+  static_assert(!GV || (!ST && !GK && !SIN), "GV: the bf16 full sweeps only");
   constexpr int LQ = KP + 8, LT = C + 8, LH = KP + 8;
   constexpr int NHT = (KP / 16) * (BV / 16) / NW;  // state tiles per wave (4, 2, 1), one K block
   constexpr int ES = sizeof(TIn);
@@ -110,7 +105,7 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
                            (GV ? (C * LE + 4 * BV) * 4 : 0);
   constexpr bool SHARED_D = !ST && LDS_BASE + 10 * 64 * 16 <= 160 * 1024;
   __shared__ __attribute__((aligned(16))) uint4 sDt[SHARED_D ? 10 * 64 : 1];
-  __shared__ uint32_t sMx[NW];   // fp16 checkpoints: each wave's largest |S| (fp32 bits)
+
   const Plane PX{sX, XL ? sX + C * LQ : sX, LQ};
   const Plane PZ{sZ, XL ? sZ + C * LQ : sZ, LQ};
   const Plane PYt{sYT, SY ? sYT + BV * LT : sYT, LT};
@@ -148,7 +143,7 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
   n = __builtin_amdgcn_readfirstlane(n);
   const int H = p.H, K = p.K, V = p.V;
   // row length of q / k / g and of the state rows
-  const int LDK = (VAR == 0 && p.ldk > 0) ? p.ldk : K;
+  const int LDK = p.ldk > 0 ? p.ldk : K;
   const float scale = p.scale;
 
   int L, row0, cbase;
@@ -181,10 +176,7 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
   const uint32_t offYg = ycolok ? ((uint32_t)(yseg * YR) * rowV + yv) * 4u : kOOB;   // GV gates
   // gate load: per-channel [.., K] float4, or the per-(token, head) scalar read as the first
   // word of a 16-byte load; the gamma mode loads nothing (out of range -> 0)
-  const int gmode = GK ? kGateK : (GV ? kGateGamma : p.gate_mode);   // YG: no K-side gate
-  // YG = 2: the value-side gate is per token, g [B,T,H] (kGateS) or the constant g_gamma [H]
-  const bool yg_s = YG == 2 && p.gate_mode == kGateS;
-  const float yg_gam = (YG == 2 && p.gate_mode == kGateGamma) ? p.g[hh] : 0.f;
+  const int gmode = GK ? kGateK : (GV ? kGateGamma : p.gate_mode);   // GV: no K-side gate
   const bool gk_mode = GK || gmode == kGateK;
   const uint32_t offGm = gk_mode ? offG : (gmode == kGateS ? (uint32_t)r0 * H * 4u : kOOB);
   const uint32_t gstride = gk_mode ? rowK * 4 : (uint32_t)H * 4;
@@ -252,7 +244,7 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
     typename Wd::W4 rq[RPT], rk[RPT];
     uint4 rg[RPT];
     typename Wd::W2 ry[YR];
-    uint2 rgv[GV ? YR : 1];              // YG: the gates of the two Y columns
+    uint2 rgv[GV ? YR : 1];              // GV: the gates of the two Y columns
   };
   Raw rsA, rsB;
   auto load_chunk = [&](int c, Raw& rs) {
@@ -292,19 +284,10 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
     const rsrc_t Ry = chunk_rsrc((const TIn*)p.y, e0, nval, (int)rowV, V);
 #pragma unroll
     for (int i = 0; i < YR; ++i) rs.ry[i] = Wd::ld2(Ry, offY, i * rowV * ES);
-    if constexpr (YG == 1) {
+    if constexpr (GV) {
       const rsrc_t Rgv = chunk_rsrc(p.g, e0, nval, (int)rowV, V);
 #pragma unroll
       for (int i = 0; i < YR; ++i) rs.rgv[i] = bld64(Rgv, offYg, i * rowV * 4);
-    } else if constexpr (YG == 2) {
-      // one word per row (the constant gate reads nothing: out of range)
-      const rsrc_t Rgs = chunk_rsrc(p.g, e0, nval, H, 1);
-#pragma unroll
-      for (int i = 0; i < YR; ++i) {
-        const bool ok = yg_s;
-        const uint32_t w = bld32(Rgs, ok ? (uint32_t)(yseg * YR) * H * 4u : kOOB, i * H * 4);
-        rs.rgv[i] = make_uint2(w, w);
-      }
     }
   };
 
@@ -338,7 +321,7 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
 #pragma unroll
       for (int i = 0; i < YR; ++i) {
         float a = __uint_as_float(rs.rgv[i].x), b = __uint_as_float(rs.rgv[i].y);
-        if (YG == 2 && !yg_s) a = b = yseg * YR + i < nval ? yg_gam : 0.f;
+
         gvc[i][0] = a * kLog2e + (i > 0 ? gvc[i - 1][0] : 0.f);
         gvc[i][1] = b * kLog2e + (i > 0 ? gvc[i - 1][1] : 0.f);
       }
@@ -387,7 +370,7 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
       gam[0] += t.x; gam[1] += t.y; gam[2] += t.z; gam[3] += t.w;
     }
     }
-    // YG: Gm of the thread's Y columns (and the prefix of its rows), and per state tile the
+    // GV: Gm of the thread's Y columns (and the prefix of its rows), and per state tile the
     // factors of the lane's column 16 nn + l16: 2^Gamma (decay), the update scaling and alpha
     // (forward 2^(Gamma - Gm) and scale 2^Gm, reverse scale 2^Gm and 2^(Gamma - Gm))
     float gmv[2] = {0.f, 0.f};
@@ -452,9 +435,7 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
     // staging: stored after the next chunk's prefetch instead, the checkpoints measured
     // slower (the memory counter retires in issue order, so the waits for the prefetched
     // loads at the top of the next chunk then also cover the stores).
-    if constexpr (!ST && VAR == 1) {
-      state_absmax<NHT>(S, sMx, wave, lane);   // the tile maximum is read after B2
-    } else if constexpr (!ST && VAR == 0) {
+    if constexpr (!ST) {
       if (p.ckpt && (p.ckpt_par == 0 || ((cbase + c) & 1) == p.ckpt_par - 1)) {
         const rsrc_t Rck = make_rsrc(p.ckpt + ((size_t)(cbase + c) * H + hh) * LDK * V,
                                      (long long)K * V * 4);
@@ -516,13 +497,6 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
       put_n<SY, YR>(PYt, 2 * yc + 1, yseg * YR, yb);
     }
     __syncthreads();  // B2: all planes visible
-
-    // fp16 checkpoint of S, from the wave maxima taken before B2 (stored ahead of the
-    // prefetch below: the memory counter retires in issue order)
-    if constexpr (!ST && VAR == 1)
-      store_state16<NHT, NW>(S, sMx, (uint16_t*)p.ckpt + ((size_t)(cbase + c) * H + hh) * LDK * V,
-                             p.ckpt_scale + ((size_t)(cbase + c) * H + hh) * p.NV + vt, K, V,
-                             vt, wave, msb, lane, tid);
 
     // ---------------- prefetch the chunk PF steps ahead while this one is computed
     if (it + PF < NTs) load_chunk(cidx(it + PF), rs);
@@ -728,7 +702,7 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
         acc[0] *= e4.x; acc[1] *= e4.y; acc[2] *= e4.z; acc[3] *= e4.w;
       }
       const int v0 = vt * BV + 16 * nn + 4 * lg;
-      if (VAR != 0 || p.acc_mode == 0) {
+      if (p.acc_mode == 0) {
         Wd::st4(Ro, acc, v0 < V ? oo : kOOB, (uint32_t)(16 * nn * ES));
       } else {
         // channel slices: the fp32 sum of the slices' outputs (element offset as oo's)
@@ -776,39 +750,18 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
 template <typename TIn, bool REV>
 hipError_t launch_gla_sweep(const SweepParams& p, hipStream_t s) {
   if (gla_strip_eligible(p)) return launch_gla_strip<TIn, REV, false>(p, s);
-  // fp16 checkpoints: whole-width state rows with the plain layout (ckpt_par 0, no slices)
-  const bool plain = !p.acc_mode && !p.ldk;
-  if (p.ckpt16 && (!p.ckpt || !p.ckpt_scale || p.ckpt_par || !plain)) return hipErrorInvalidValue;
-  const int var = p.ckpt16 ? 1 : ((plain && !p.ckpt) ? 2 : 0);
-  if (var == 1 && !std::is_same<TIn, uint16_t>::value) return hipErrorInvalidValue;
+  if constexpr (std::is_same<TIn, uint16_t>::value) {
+    if (gla_strip_s_eligible(p)) return launch_gla_strip_s<REV>(p, false, s);
+  }
+  if (p.ckpt16) return hipErrorInvalidValue;   // the strip kernels write fp16 checkpoints
   const int kp = p.K <= 32 ? 32 : (p.K <= 64 ? 64 : 128);
   dim3 grid(p.NV * p.H * p.N);
-  const bool gk = p.gate_mode == kGateK;
 #define TOPS_SWEEP(KPV, GKV) \
   hipLaunchKernelGGL((gla_sweep_kernel<TIn, KPV, REV, false, GKV>), grid, dim3(512), 0, s, p)
-  // fp16 checkpoints: the bf16 one-gate-per-token sweeps here, the per-channel-gate bf16
-  // sweeps in the strip kernel (routed above)
-  const bool yg2 = std::is_same<TIn, uint16_t>::value && !gk && !p.gshift &&
-                   (p.gate_mode == kGateS || p.gate_mode == kGateGamma);
-  if (var == 1 && !yg2) return hipErrorInvalidValue;
-  if (gk) {
+  if (p.gate_mode == kGateK) {
     if (kp == 32) TOPS_SWEEP(32, true);
     else if (kp == 64) TOPS_SWEEP(64, true);
     else TOPS_SWEEP(128, true);
-  } else if (std::is_same<TIn, uint16_t>::value && !p.gshift &&
-             (p.gate_mode == kGateS || p.gate_mode == kGateGamma)) {
-    // one gate per token (bf16): on the value side, q and k stay exact
-#define TOPS_SWEEP_YG(KPV, VARV) \
-  hipLaunchKernelGGL((gla_sweep_kernel<uint16_t, KPV, REV, false, false, 2, VARV>), grid, dim3(512), 0, s, p)
-    if constexpr (std::is_same<TIn, uint16_t>::value) {
-#define TOPS_SWEEP_YGV(KPV) \
-  if (var == 1) TOPS_SWEEP_YG(KPV, 1); else if (var == 2) TOPS_SWEEP_YG(KPV, 2); else TOPS_SWEEP_YG(KPV, 0)
-      if (kp == 32) { TOPS_SWEEP_YGV(32); }
-      else if (kp == 64) { TOPS_SWEEP_YGV(64); }
-      else { TOPS_SWEEP_YGV(128); }
-#undef TOPS_SWEEP_YGV
-    }
-#undef TOPS_SWEEP_YG
   } else {
     if (kp == 32) TOPS_SWEEP(32, false);
     else if (kp == 64) TOPS_SWEEP(64, false);
@@ -823,7 +776,7 @@ hipError_t launch_gla_sweep_gv(const SweepParams& p, hipStream_t s) {
   const int kp = p.K <= 32 ? 32 : (p.K <= 64 ? 64 : 128);
   dim3 grid(p.NV * p.H * p.N);
 #define TOPS_SWEEP_GV(KPV) \
-  hipLaunchKernelGGL((gla_sweep_kernel<uint16_t, KPV, REV, false, false, 1>), grid, dim3(512), 0, s, p)
+  hipLaunchKernelGGL((gla_sweep_kernel<uint16_t, KPV, REV, false, false, true>), grid, dim3(512), 0, s, p)
   if (kp == 32) TOPS_SWEEP_GV(32);
   else if (kp == 64) TOPS_SWEEP_GV(64);
   else TOPS_SWEEP_GV(128);
@@ -833,17 +786,15 @@ hipError_t launch_gla_sweep_gv(const SweepParams& p, hipStream_t s) {
 
 template <typename TIn, bool REV>
 hipError_t launch_gla_state_pass(const SweepParams& p, hipStream_t s) {
+  if (p.gate_mode == kGateK) return launch_gla_strip_state<TIn, REV>(p, s);
+  if (std::is_same<TIn, uint16_t>::value && gla_strip_s_eligible(p)) return launch_gla_strip_s<REV>(p, true, s);
   const int kp = p.K <= 32 ? 32 : (p.K <= 64 ? 64 : 128);
   dim3 grid(p.NV * p.H * p.N);
-#define TOPS_STATE(KPV, GKV) \
-  hipLaunchKernelGGL((gla_sweep_kernel<TIn, KPV, REV, true, GKV>), grid, dim3(512), 0, s, p)
-  if (p.gate_mode == kGateK) {
-    return launch_gla_strip_state<TIn, REV>(p, s);
-  } else {
-    if (kp == 32) TOPS_STATE(32, false);
-    else if (kp == 64) TOPS_STATE(64, false);
-    else TOPS_STATE(128, false);
-  }
+#define TOPS_STATE(KPV) \
+  hipLaunchKernelGGL((gla_sweep_kernel<TIn, KPV, REV, true, false>), grid, dim3(512), 0, s, p)
+  if (kp == 32) TOPS_STATE(32);
+  else if (kp == 64) TOPS_STATE(64);
+  else TOPS_STATE(128);
 #undef TOPS_STATE
   return hipGetLastError();
 }

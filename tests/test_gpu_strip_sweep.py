@@ -87,3 +87,54 @@ def test_strip_sweep_delta_rule_tile_edges(T, K, V, dt, cuda_device):
         base = np.linalg.norm(s["k"] * rk) if n == "dg" else np.linalg.norm(ref)
         lim = out_bound(ref, dtype, torch.bfloat16 if n == "dg" and dt == "bf16" else got.dtype)
         assert err <= lim * max(base, np.linalg.norm(ref)), f"{n}: rel-err {err / base:.3e} (bound {lim:.2e})"
+
+
+SIMPLE_CASES = [(T, K, V, gate) for gate in ("token", "head")
+                for T, K, V in ((1, 8, 8), (63, 40, 56), (64, 32, 64), (65, 64, 72),
+                                (127, 72, 128), (129, 104, 8), (200, 128, 128))]
+
+
+@pytest.mark.parametrize("T,K,V,gate", SIMPLE_CASES, ids=lambda x: str(x))
+def test_strip_sweep_token_gate_tile_edges(T, K, V, gate, cuda_device):
+    """One gate per token, or a constant per head (bf16), against the oracle
+    (tops/cpu/ops/simple_gla/chunk.py:53-129, 668-788), with checkpoints and without."""
+    import numpy as np
+    from _inputs import simple_gla_inputs
+    from tops.ops.simple_gla import chunk_simple_gla
+    bf, f32 = torch.bfloat16, torch.float32
+    B, H = 2, 3
+    d = simple_gla_inputs(B, T, H, K, V, 500 + T, h0=True, grads=True)
+    x = {n: to_dev(d[n], bf, cuda_device).requires_grad_() for n in "qkv"}
+    x["h0"] = to_dev(d["h0"], f32, cuda_device).requires_grad_()
+    g = to_dev(d["g"], f32, cuda_device).requires_grad_()
+    gam = to_dev(d["g_gamma"], f32, cuda_device)
+    kw = dict(g=g) if gate == "token" else dict(g_gamma=gam)
+    print(f"token-gate strip sweep T={T} K={K} V={V} {gate}", flush=True)
+
+    def call():
+        return chunk_simple_gla(x["q"], x["k"], x["v"], initial_state=x["h0"],
+                                output_final_state=True, **kw)
+    o, ht = call()
+    torch.autograd.backward((o, ht), (to_dev(d["do"], bf, cuda_device),
+                                      to_dev(d["dht"], f32, cuda_device)))
+    with torch.no_grad():
+        oi, hi = call()
+    # the oracle of per-channel gates on the broadcast gate
+    gfull = d["g"] if gate == "token" else np.broadcast_to(d["g_gamma"], d["g"].shape)
+    gk = np.ascontiguousarray(np.broadcast_to(gfull[..., None], gfull.shape + (K,)))
+    s = {n: seen(d[n], bf) for n in ("q", "k", "v", "do")}
+    ro, rht = O.chunk_gla(s["q"], s["k"], s["v"], gk, initial_state=d["h0"],
+                          output_final_state=True, chunk_size=64)
+    rq, rk, rv, rg, rh0 = O.chunk_gla_bwd(s["q"], s["k"], s["v"], gk, K ** -0.5, d["h0"], s["do"],
+                                          d["dht"], chunk_size=64)
+    pairs = [("o", o, ro), ("ht", ht, rht), ("o inf", oi, ro), ("ht inf", hi, rht),
+             ("dq", x["q"].grad, rq), ("dk", x["k"].grad, rk), ("dv", x["v"].grad, rv),
+             ("dh0", x["h0"].grad, rh0)]
+    for n, got, ref in pairs:
+        e, lim = rel(host(got), ref), out_bound(ref, bf, got.dtype)
+        assert e < lim, f"{n}: rel-err {e:.3e} vs oracle (bound {lim:.2e})"
+    if gate == "token":
+        # the sum of K per-channel gradients, each a difference of q dq and k dk terms
+        err = np.linalg.norm(host(g.grad) - rg.sum(-1))
+        scale = np.linalg.norm((np.abs(s["q"] * rq) + np.abs(s["k"] * rk)).sum(-1))
+        assert err <= 1e-3 * scale, f"dg: {err / scale:.3e} of its terms"
