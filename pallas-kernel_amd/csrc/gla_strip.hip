@@ -2,7 +2,8 @@
 // KDA delta rule): the same recurrences as gla_sweep_kernel (gla_sweep.hip), which cites the
 // reference functions they replace.
 //
-// One workgroup of 8 wave64 owns one (sequence, head, 64-wide V tile).  Waves 0-3 (one per
+// One workgroup of 8 wave64 owns one (sequence, head, 64-wide V tile; the delta rule also
+// takes 16- and 32-wide tiles, one or two consumers).  Waves 0-3 (one per
 // SIMD) are consumers: wave j holds the fp32 state of 16 V columns, all K rows, in MFMA
 // accumulators for the whole walk, and runs every product that touches it.  Waves 4-7 are
 // producers: they load the raw q / k / g / Y rows, do the gate cumsum, the exponentials and
@@ -44,7 +45,7 @@
 // multiplied and passed the state through LDS.  Delta rule, B4 T8192 H32 K=V=128 bf16:
 // forward with checkpoints 1187 -> 800 us, without 1047 -> 680, reverse 970 -> 710 (2.7 to
 // 3.5 GB per launch, 500-720 us at the copy rate); fp32, B1 T5000 H32 (64 workgroups, so
-// latency alone): 756 -> 370.  There producers keep the D tiles (the consumers carry w S) and
+// latency alone): 756 -> 370, 289 on 16-column tiles.  There producers keep the D tiles (the consumers carry w S) and
 // the default priority in interval A.
 #include <stdlib.h>
 
@@ -102,15 +103,17 @@ struct PhaseClock<true> {
 // VAR: 1 = fp16 checkpoints of every chunk (training), 2 = no checkpoints (inference), 3 = the
 // end state and the decay sums only (the state pass of sequence-parallel segments: Z~ and Y,
 // no X~, no output), 0 = the rest (fp32 or paired checkpoints, channel slices).
-template <typename TIn, int KP, bool REV, bool DELTA, int VAR>
-__global__ __launch_bounds__(512) void gla_strip_kernel(SweepParams p) {
-  constexpr int C = kChunk, BV = 64;
+template <typename TIn, int KP, bool REV, bool DELTA, int VAR, int BV = 64>
+__global__ __launch_bounds__(64 * (BV / 16 + 4)) void gla_strip_kernel(SweepParams p) {
+  constexpr int C = kChunk;
+  constexpr int NC = BV / 16, NPW = 4;       // consumer waves, then producer waves
+  static_assert(BV == 64 || VAR == 2, "narrow tiles: no checkpoints (their factors cover 64 columns)");
   constexpr int ES = sizeof(TIn);
   constexpr bool SIN = !In<TIn>::kExactBf16;
   constexpr bool FWD_DELTA = DELTA && !REV;
   constexpr bool REV_DELTA = DELTA && REV;
   constexpr bool SY = SIN || FWD_DELTA;      // Y carries a lo half
-  constexpr bool CONS_D = !FWD_DELTA;        // the consumers compute the D tiles
+  constexpr bool CONS_D = !FWD_DELTA && NC == 4;        // the consumers compute the D tiles
   // reverse delta rule: Z~^T Y is taken in interval A, so Z~ and Y are single planes written
   // in B with X~ (two Z~ planes, w and the checkpoint would not fit the 160 KB)
   constexpr bool ZB = REV_DELTA;
@@ -124,7 +127,7 @@ __global__ __launch_bounds__(512) void gla_strip_kernel(SweepParams p) {
   constexpr int NQ = KP / 4;
   constexpr int QW = NQ < 16 ? NQ : 16, SW = 64 / QW;
   constexpr int NCW = NQ / QW;               // waves across the columns
-  constexpr int NRW = 4 / NCW;               // waves down the rows
+  constexpr int NRW = NPW / NCW;               // waves down the rows
   constexpr int RPT = C / (NRW * SW);        // rows per thread (8, 4, 2)
   typedef Words<TIn> Wd;
 
@@ -209,10 +212,10 @@ __global__ __launch_bounds__(512) void gla_strip_kernel(SweepParams p) {
     sDt[(Rc * (Rc + 1) / 2 + Pc) * 64 + lane] = make_uint4(h.x, h.y, l.x, l.y);
   };
 
-  if (wave >= 4) {
+  if (wave >= NC) {
     // ------------------------------------------------------------------ producers
-    const int pw = wave - 4;
-    const int ptid = tid - 256;
+    const int pw = wave - NC;
+    const int ptid = tid - 64 * NC;
     const int cq = (lane % QW) + QW * (pw % NCW);
     const int rw = pw / NCW;
     const int sl = lane / QW;                 // row segment within the wave
@@ -224,7 +227,8 @@ __global__ __launch_bounds__(512) void gla_strip_kernel(SweepParams p) {
 #pragma unroll
     for (int i = 0; i < RPT; ++i)
       wa[i] = (r0 + i) * KP + (((cq >> 1) ^ swz<KP>((r0 + i) & 15)) << 3) + 4 * (cq & 1);
-    const int yr = ptid >> 2, ycol = 16 * (ptid & 3);
+    const int yr = ptid / NC, ycol = 16 * (ptid % NC);
+    const bool yok = yr < C;                  // (more producer threads than pieces)
     const int yv = vt * BV + ycol;
     constexpr int YP = 16 / (16 / ES);        // 16-byte pieces of a thread's 16 columns
 
@@ -265,7 +269,7 @@ __global__ __launch_bounds__(512) void gla_strip_kernel(SweepParams p) {
 #pragma unroll
       for (int i = 0; i < YP; ++i) {
         const int v = yv + i * (16 / ES);      // (V % 8 == 0: a piece is inside or outside)
-        ry[i] = bld128(R, v < V ? ((uint32_t)yr * rowV + v) * ES : kOOB, 0);
+        ry[i] = bld128(R, yok && v < V ? ((uint32_t)yr * rowV + v) * ES : kOOB, 0);
       }
     };
 
@@ -360,6 +364,7 @@ __global__ __launch_bounds__(512) void gla_strip_kernel(SweepParams p) {
       }
     };
     auto write_y = [&]() {
+      if (!yok) return;
       uint16_t* dst = sY + yr * LY + ycol;
       if constexpr (!SIN) {
 #pragma unroll
@@ -480,7 +485,7 @@ __global__ __launch_bounds__(512) void gla_strip_kernel(SweepParams p) {
     clk.start();
     for (int it = 0; it < NTs; ++it) {
       // A: D and Y of this chunk, Z~ of the next
-      __builtin_amdgcn_s_setprio(DELTA ? 0 : 2);
+      __builtin_amdgcn_s_setprio(DELTA && NC == 4 ? 0 : 2);
       const uint16_t* z = zbuf(it);
       if constexpr (CONS_D) {
       } else if (pw == 0) dtiles(std::integral_constant<int, 3>{}, 3, 0, z);
@@ -532,7 +537,7 @@ __global__ __launch_bounds__(512) void gla_strip_kernel(SweepParams p) {
       __syncthreads();
       clk.tick(3);
     }
-    clk.finish(p.clocks, blockIdx.x * 8 + wave);
+    clk.finish(p.clocks, blockIdx.x * (NC + NPW) + wave);
     if constexpr (ST) {
       if (p.dec_fin && vt == 0 && rw == 0 && sl == 0 && colok)
         *(float4*)(p.dec_fin + (size_t)(n * H + hh) * LDK + c0) =
@@ -868,7 +873,7 @@ __global__ __launch_bounds__(512) void gla_strip_kernel(SweepParams p) {
     __syncthreads();
     clk.tick(3);
   }
-  clk.finish(p.clocks, blockIdx.x * 8 + wave);
+  clk.finish(p.clocks, blockIdx.x * (NC + NPW) + wave);
 
   if (p.s_fin) {
     const rsrc_t Rsf = make_rsrc(p.s_fin + s_base, (long long)LDK * V * 4);
@@ -897,6 +902,29 @@ hipError_t launch_gla_strip(const SweepParams& p, hipStream_t s) {
   if (p.ckpt16 && (!plain || p.ckpt_par || !p.ckpt || !p.ckpt_scale)) return hipErrorInvalidValue;
   const int var = p.ckpt16 ? 1 : ((plain && !p.ckpt) ? 2 : 0);
   dim3 grid(p.NV * p.H * p.N);
+  if constexpr (DELTA && !REV) {
+    // Few heads and sequences leave CUs idle and the sweep is one long chain: the narrowest
+    // value tile whose workgroups are still one round on the chip's 256 CUs (B1 T5000 H32
+    // K=V=128 fp32: 64 columns 367 us, 32 columns 302, 16 columns 289, the staging repeated
+    // but each consumer alone with its LDS reads; the per-channel-gate sweeps, whose
+    // consumers share the D tiles, gain nothing: 27 us at B1 T512 H4 against 30)
+    constexpr long long kCus = 256;
+    const long long wgs = (long long)p.H * p.N;
+    const int bv = (var != 2 || wgs * p.NV > kCus / 2) ? 64 : (wgs * ((p.V + 15) / 16) <= kCus ? 16 : 32);
+    if (bv < 64 && wgs * ((p.V + bv - 1) / bv) <= kCus) {
+      SweepParams q = p;
+      q.NV = (p.V + bv - 1) / bv;
+      const dim3 gn((unsigned)(q.NV * wgs)), bn(64 * (bv / 16 + 4));
+#define TOPS_NARROW(KPV) \
+  if (bv == 16) hipLaunchKernelGGL((gla_strip_kernel<TIn, KPV, REV, DELTA, 2, 16>), gn, bn, 0, s, q); \
+  else hipLaunchKernelGGL((gla_strip_kernel<TIn, KPV, REV, DELTA, 2, 32>), gn, bn, 0, s, q)
+      if (kp == 32) { TOPS_NARROW(32); }
+      else if (kp == 64) { TOPS_NARROW(64); }
+      else { TOPS_NARROW(128); }
+#undef TOPS_NARROW
+      return hipGetLastError();
+    }
+  }
 #define TOPS_STRIP(KPV, VARV) \
   hipLaunchKernelGGL((gla_strip_kernel<TIn, KPV, REV, DELTA, VARV>), grid, dim3(512), 0, s, p)
 #define TOPS_STRIP_K(KPV) \

@@ -138,3 +138,34 @@ def test_strip_sweep_token_gate_tile_edges(T, K, V, gate, cuda_device):
         err = np.linalg.norm(host(g.grad) - rg.sum(-1))
         scale = np.linalg.norm((np.abs(s["q"] * rq) + np.abs(s["k"] * rk)).sum(-1))
         assert err <= 1e-3 * scale, f"dg: {err / scale:.3e} of its terms"
+
+
+@pytest.mark.parametrize("B,H,V,dt", [(1, 2, 128, "bf16"), (1, 2, 8, "f32"), (1, 20, 128, "bf16"),
+                                      (1, 40, 72, "f32"), (2, 33, 128, "bf16")],
+                         ids=lambda x: str(x))
+def test_strip_sweep_delta_rule_narrow_tiles(B, H, V, dt, cuda_device):
+    """The forward delta rule without checkpoints takes 16- or 32-column tiles while their
+    workgroups are one round on the chip.  Both sides of the rule's lines (20 heads of 128
+    columns: 160 workgroups of 16 columns; 40 of 72: 200; 66 heads: 64-column tiles) within
+    the bounds of the oracle, and the same up to fp32 rounding as those heads in a call of four
+    times as many, which takes wider tiles."""
+    import numpy as np
+    from oracle import kda as OK
+    from _inputs import kda_inputs
+    from tops.ops.kda import chunk_kda
+    dtype = {"bf16": torch.bfloat16, "f32": torch.float32}[dt]
+    T, K = 130, 64
+    d = kda_inputs(B, T, H, K, V, 40 + H, gate_div=4.0, h0=True)
+    x = [to_dev(d[n], dtype, cuda_device) for n in "qkv"] + \
+        [to_dev(d[n], torch.float32, cuda_device) for n in ("g", "beta")]
+    h0 = to_dev(d["h0"], torch.float32, cuda_device)
+    print(f"narrow tiles B={B} H={H} V={V} {dt}", flush=True)
+    o, ht = chunk_kda(*x, initial_state=h0, output_final_state=True)
+    ro, rht = OK.chunk_kda(*(seen(d[n], dtype) for n in "qkv"), np.float64(d["g"]),
+                           np.float64(d["beta"]), K ** -0.5, np.float64(d["h0"]), True)
+    for n, got, ref in (("o", o, ro), ("ht", ht, rht)):
+        e, lim = rel(host(got), ref), out_bound(ref, dtype, got.dtype)
+        assert e < lim, f"{n}: rel-err {e:.3e} vs oracle (bound {lim:.2e})"
+    rep = [torch.cat([t] * 4, 2).contiguous() for t in x]      # four times the heads: wider tiles
+    o4, ht4 = chunk_kda(*rep, initial_state=torch.cat([h0] * 4, 1), output_final_state=True)
+    assert rel(host(o4[:, :, :H]), host(o)) <= 1e-3 and rel(host(ht4[:, :H]), host(ht)) <= 1e-5
