@@ -166,15 +166,20 @@ def timing_events() -> dict:
 
 
 def call(name: str, *args) -> None:
+    """Call an entry point.  A tensor argument passes its device address; `args` holds the
+    tensors until the launch is queued, so a temporary made in the argument list stays
+    allocated that long (freeing it afterwards is stream-ordered behind the launch)."""
+    fn = _bound.get(name) or _fn(name)
+    a = [x.data_ptr() if isinstance(x, torch.Tensor) else x for x in args]
     if _timing is not None:
         ev0 = torch.cuda.Event(enable_timing=True)
         ev1 = torch.cuda.Event(enable_timing=True)
         ev0.record()
-        rc = _fn(name)(*args)
+        rc = fn(*a)
         ev1.record()
         _timing.setdefault(name, []).append((ev0, ev1))
     else:
-        rc = _fn(name)(*args)
+        rc = fn(*a)
     if rc != 0:
         msg = lib().tops_last_error().decode()
         if rc == -2:
@@ -188,7 +193,8 @@ class _Ptr(int):
     the tensor go back to the caching allocator at once, and a later argument's own
     allocation (a copy, an upload) could then take that block and write it before the kernel
     that reads it is queued.  Holding the tensor until `call` returns closes that window;
-    freeing it afterwards is stream-ordered behind the launch."""
+    freeing it afterwards is stream-ordered behind the launch.  (The hot paths hand their
+    tensors to `call` itself, which holds them the same way without an object per argument.)"""
 
     def __new__(cls, t):
         p = super().__new__(cls, t.data_ptr())
@@ -200,7 +206,13 @@ def ptr(t) -> int | None:
     return None if t is None else _Ptr(t)
 
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream() -> int:
+    """The current stream of the current device (its raw handle, without a Stream object)."""
+    if _raw_stream is not None and torch.cuda.is_initialized():
+        return _raw_stream(torch.cuda.current_device())
     return torch.cuda.current_stream().cuda_stream
 
 

@@ -65,8 +65,8 @@ class _ShortConv(torch.autograd.Function):
         ydt = _out_dtype(x, weight)
         y = torch.empty(B, T, D, device=x.device, dtype=ydt)
         fs = torch.empty(n, D, W, device=x.device, dtype=xk.dtype) if want_state else None
-        N.call("tops_short_conv_fwd", N.ptr(xk), N.dtype_code(xk.dtype), N.ptr(w32), N.ptr(b32),
-               N.ptr(y), N.dtype_code(ydt), N.ptr(fs), N.ptr(cu), B, T, D, W, n, act, N.stream())
+        N.call("tops_short_conv_fwd", xk, N.dtype_code(xk.dtype), w32, b32,
+               y, N.dtype_code(ydt), fs, cu, B, T, D, W, n, act, N.stream())
         ctx.save_for_backward(xk, w32, b32, cu)
         ctx.meta = (act, n, x.dtype, weight.dtype, None if bias is None else bias.dtype,
                     tuple(weight.shape))
@@ -87,9 +87,9 @@ class _ShortConv(torch.autograd.Function):
         db = None if b32 is None else torch.empty(D, device=xk.device, dtype=torch.float32)
         n_ws = int(N.lib().tops_short_conv_bwd_workspace(B, T, D, W))
         ws = torch.empty(max(n_ws, 1), device=xk.device, dtype=torch.float32)
-        N.call("tops_short_conv_bwd", N.ptr(xk), N.dtype_code(xk.dtype), N.ptr(w32), N.ptr(b32),
-               N.ptr(dy), N.dtype_code(dy.dtype), N.ptr(dx), N.ptr(dw), N.ptr(db), N.ptr(ws),
-               n_ws, N.ptr(cu), B, T, D, W, n, act, N.stream())
+        N.call("tops_short_conv_bwd", xk, N.dtype_code(xk.dtype), w32, b32,
+               dy, N.dtype_code(dy.dtype), dx, dw, db, ws,
+               n_ws, cu, B, T, D, W, n, act, N.stream())
         return (dx.to(x_dt), dw.reshape(w_shape).to(w_dt),
                 None if db is None else db.to(b_dt), None, None, None, None)
 
@@ -136,8 +136,8 @@ def short_conv_step(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | 
     b32 = None if bias is None else bias.to(torch.float32).contiguous()
     ydt = _out_dtype(x, weight)
     y = torch.empty(n, D, device=x.device, dtype=ydt)
-    N.call("tops_short_conv_step", N.ptr(xs), N.dtype_code(xs.dtype), N.ptr(cin), N.ptr(cout),
-           N.ptr(w32), N.ptr(b32), N.ptr(y), N.dtype_code(ydt), n, D, W, _act(activation),
+    N.call("tops_short_conv_step", xs, N.dtype_code(xs.dtype), cin, cout,
+           w32, b32, y, N.dtype_code(ydt), n, D, W, _act(activation),
            N.stream())
     return y.reshape(x.shape), None if cout is None else cout.to(cache.dtype)
 

@@ -34,8 +34,8 @@ class _RMSNormGated(torch.autograd.Function):
         w32 = None if weight is None else weight.detach().to(torch.float32).contiguous()
         rows = x.numel() // D if D else 0
         y = torch.empty_like(xk)
-        N.call("tops_rmsnorm_gated_fwd", N.ptr(xk), N.dtype_code(xk.dtype), N.ptr(gk),
-               0 if gk is None else N.dtype_code(gk.dtype), N.ptr(w32), N.ptr(y), rows, D,
+        N.call("tops_rmsnorm_gated_fwd", xk, N.dtype_code(xk.dtype), gk,
+               0 if gk is None else N.dtype_code(gk.dtype), w32, y, rows, D,
                float(eps), N.stream())
         ctx.save_for_backward(xk, gk, w32)
         ctx.eps = float(eps)
@@ -57,9 +57,9 @@ class _RMSNormGated(torch.autograd.Function):
             dw = torch.empty(D, device=xk.device, dtype=torch.float32)
             n_ws = int(N.lib().tops_rmsnorm_gated_bwd_workspace(rows, D))
             ws = torch.empty(max(n_ws, 1), device=xk.device, dtype=torch.float32)
-        N.call("tops_rmsnorm_gated_bwd", N.ptr(xk), N.dtype_code(xk.dtype), N.ptr(gk),
-               0 if gk is None else N.dtype_code(gk.dtype), N.ptr(w32), N.ptr(dy), N.ptr(dx),
-               N.ptr(dg), N.ptr(dw), N.ptr(ws), n_ws, rows, D, ctx.eps, N.stream())
+        N.call("tops_rmsnorm_gated_bwd", xk, N.dtype_code(xk.dtype), gk,
+               0 if gk is None else N.dtype_code(gk.dtype), w32, dy, dx,
+               dg, dw, ws, n_ws, rows, D, ctx.eps, N.stream())
         x_dt, g_dt, w_dt = ctx.dtypes
         return (dx.to(x_dt), None if dg is None else dg.to(g_dt),
                 None if dw is None else dw.to(w_dt), None)

@@ -52,7 +52,7 @@ _GATE_CODE = {GATE_K: 0, GATE_S: 1, GATE_GAMMA: 2, GATE_GAMMA_K: 3}
 def _gate_ptrs(gate):
     """(g, g_gamma) pointer pair of the simple-GLA entry points."""
     mode, gt = gate
-    return (N.ptr(gt) if mode == GATE_S else None, N.ptr(gt) if mode == GATE_GAMMA else None)
+    return (gt if mode == GATE_S else None, gt if mode == GATE_GAMMA else None)
 
 
 def _segment_states(z, y, gate, s_in, scale, sp, reverse: bool):
@@ -67,12 +67,12 @@ def _segment_states(z, y, gate, s_in, scale, sp, reverse: bool):
     if pc.n:
         s_loc = torch.empty(pc.n, H, K, V, device=dev, dtype=torch.float32)
         dec = torch.empty(pc.n, H, K, device=dev, dtype=torch.float32)
-        N.call("tops_chunk_state_pass", N.ptr(z), N.ptr(y), N.ptr(gt), _GATE_CODE[mode],
-               N.ptr(s_loc), N.ptr(dec), N.ptr(pc.start_dev), N.ptr(pc.end_dev), B * T, H, K, V,
+        N.call("tops_chunk_state_pass", z, y, gt, _GATE_CODE[mode],
+               s_loc, dec, pc.start_dev, pc.end_dev, B * T, H, K, V,
                pc.n, N.chunk_dtype_code(z.dtype), float(scale), int(reverse), N.stream())
     init = torch.empty(sp.Nv, H, K, V, device=dev, dtype=torch.float32)
-    N.call("tops_chunk_state_combine", N.ptr(s_loc), N.ptr(dec), N.ptr(s_in), N.ptr(init),
-           N.ptr(sp.seg_first_dev), N.ptr(pc.first_dev), N.ptr(pc.dst_dev),
+    N.call("tops_chunk_state_combine", s_loc, dec, s_in, init,
+           sp.seg_first_dev, pc.first_dev, pc.dst_dev,
            len(sp.seg_first) - 1, H, K, V, int(reverse), N.stream())
     return init
 
@@ -121,7 +121,7 @@ def states_fp32(hs):
 
 
 def _sptr(hs):
-    return N.ptr(hs.h if isinstance(hs, States16) else hs)
+    return hs.h if isinstance(hs, States16) else hs
 
 
 def pack_states(hs):
@@ -158,23 +158,23 @@ def _fwd_tile(q, k, v, gate, h0, scale, output_final_state, plan: ChunkPlan, kee
         fin = torch.empty(sp.Nv, H, K, V, device=q.device, dtype=torch.float32) \
             if output_final_state else None
         cu, offs, Bx, Tx, Nx = sp.cu_dev, sp.offsets_dev, 1, B * T, sp.Nv
-    tail = (N.ptr(s0), N.ptr(o), N.ptr(fin), _sptr(hs), N.ptr(cu), N.ptr(offs),
+    tail = (s0, o, fin, _sptr(hs), cu, offs,
             Bx, Tx, H, K, V, Nx, N.chunk_dtype_code(q.dtype), float(scale), N.stream())
     if c16 and mode == GATE_K:
-        N.call("tops_gla_chunk_fwd_c16", N.ptr(q), N.ptr(k), N.ptr(v), N.ptr(gt), N.ptr(s0),
-               N.ptr(o), N.ptr(fin), N.ptr(hs.h), N.ptr(hs.scale), *tail[4:])
+        N.call("tops_gla_chunk_fwd_c16", q, k, v, gt, s0,
+               o, fin, hs.h, hs.scale, *tail[4:])
     elif c16:
-        N.call("tops_simple_gla_chunk_fwd_c16", N.ptr(q), N.ptr(k), N.ptr(v), *_gate_ptrs(gate),
-               N.ptr(s0), N.ptr(o), N.ptr(fin), N.ptr(hs.h), N.ptr(hs.scale), *tail[4:])
+        N.call("tops_simple_gla_chunk_fwd_c16", q, k, v, *_gate_ptrs(gate),
+               s0, o, fin, hs.h, hs.scale, *tail[4:])
     elif keep_states == PAIRED:
-        N.call("tops_chunk_fwd_paired", N.ptr(q), N.ptr(k), N.ptr(v), N.ptr(gt),
+        N.call("tops_chunk_fwd_paired", q, k, v, gt,
                _GATE_CODE[mode], *tail)
     elif mode == GATE_K:
-        N.call("tops_gla_chunk_fwd", N.ptr(q), N.ptr(k), N.ptr(v), N.ptr(gt), *tail)
+        N.call("tops_gla_chunk_fwd", q, k, v, gt, *tail)
     elif mode == GATE_GAMMA_K:
-        N.call("tops_gla_chunk_fwd_gamma", N.ptr(q), N.ptr(k), N.ptr(v), N.ptr(gt), *tail)
+        N.call("tops_gla_chunk_fwd_gamma", q, k, v, gt, *tail)
     else:
-        N.call("tops_simple_gla_chunk_fwd", N.ptr(q), N.ptr(k), N.ptr(v), *_gate_ptrs(gate),
+        N.call("tops_simple_gla_chunk_fwd", q, k, v, *_gate_ptrs(gate),
                *tail)
     ht = fin
     if sp is not None and fin is not None:
@@ -215,39 +215,39 @@ def _bwd_tile(q, k, v, gate, do, dht, hs, scale, plan: ChunkPlan, want_dh0: bool
         fin = torch.empty(sp.Nv, H, K, V, device=q.device, dtype=torch.float32) \
             if want_dh0 else None
         cu, offs, Bx, Tx, Nx = sp.cu_dev, sp.offsets_dev, 1, B * T, sp.Nv
-    dh_args = (N.ptr(do), N.ptr(s0), _sptr(dh_work), N.ptr(dv), N.ptr(fin), N.ptr(cu), N.ptr(offs),
+    dh_args = (do, s0, _sptr(dh_work), dv, fin, cu, offs,
                Bx, Tx, H, K, V, Nx, dt, float(scale), st)
-    dqkg_tail = (N.ptr(do), _sptr(hs), _sptr(dh_work), N.ptr(dq), N.ptr(dk), N.ptr(dg),
-                 N.ptr(plan.cu_dev), N.ptr(plan.offsets_dev), N.ptr(plan.chunk_map_dev),
+    dqkg_tail = (do, _sptr(hs), _sptr(dh_work), dq, dk, dg,
+                 plan.cu_dev, plan.offsets_dev, plan.chunk_map_dev,
                  plan.total, B, T, H, K, V, plan.N, dt, float(scale), st)
     if c16 and mode == GATE_K:
-        N.call("tops_gla_chunk_bwd_dh_c16", N.ptr(q), N.ptr(k), N.ptr(gt), N.ptr(do), N.ptr(s0),
-               N.ptr(dh_work.h), N.ptr(dh_work.scale), *dh_args[3:])
-        N.call("tops_gla_chunk_bwd_dqkg_c16", N.ptr(q), N.ptr(k), N.ptr(v), N.ptr(gt), N.ptr(do),
-               N.ptr(hs.h), N.ptr(hs.scale), N.ptr(dh_work.h), N.ptr(dh_work.scale),
+        N.call("tops_gla_chunk_bwd_dh_c16", q, k, gt, do, s0,
+               dh_work.h, dh_work.scale, *dh_args[3:])
+        N.call("tops_gla_chunk_bwd_dqkg_c16", q, k, v, gt, do,
+               hs.h, hs.scale, dh_work.h, dh_work.scale,
                *dqkg_tail[3:])
     elif c16:
-        N.call("tops_simple_gla_chunk_bwd_dh_c16", N.ptr(q), N.ptr(k), *_gate_ptrs(gate),
-               N.ptr(do), N.ptr(s0), N.ptr(dh_work.h), N.ptr(dh_work.scale), *dh_args[3:])
-        N.call("tops_simple_gla_chunk_bwd_dqkg_c16", N.ptr(q), N.ptr(k), N.ptr(v),
-               *_gate_ptrs(gate), N.ptr(do), N.ptr(hs.h), N.ptr(hs.scale), N.ptr(dh_work.h),
-               N.ptr(dh_work.scale), *dqkg_tail[3:])
+        N.call("tops_simple_gla_chunk_bwd_dh_c16", q, k, *_gate_ptrs(gate),
+               do, s0, dh_work.h, dh_work.scale, *dh_args[3:])
+        N.call("tops_simple_gla_chunk_bwd_dqkg_c16", q, k, v,
+               *_gate_ptrs(gate), do, hs.h, hs.scale, dh_work.h,
+               dh_work.scale, *dqkg_tail[3:])
     elif paired:
         code = _GATE_CODE[mode]
-        N.call("tops_chunk_bwd_dh_paired", N.ptr(q), N.ptr(k), N.ptr(gt), code, *dh_args)
-        N.call("tops_chunk_bwd_dqkg_paired", N.ptr(q), N.ptr(k), N.ptr(v), N.ptr(gt), code,
-               N.ptr(do), N.ptr(h0), N.ptr(dht), N.ptr(hs), N.ptr(dq), N.ptr(dk), N.ptr(dg),
+        N.call("tops_chunk_bwd_dh_paired", q, k, gt, code, *dh_args)
+        N.call("tops_chunk_bwd_dqkg_paired", q, k, v, gt, code,
+               do, h0, dht, hs, dq, dk, dg,
                *dqkg_tail[6:])
     elif mode == GATE_K:
-        N.call("tops_gla_chunk_bwd_dh", N.ptr(q), N.ptr(k), N.ptr(gt), *dh_args)
-        N.call("tops_gla_chunk_bwd_dqkg", N.ptr(q), N.ptr(k), N.ptr(v), N.ptr(gt), *dqkg_tail)
+        N.call("tops_gla_chunk_bwd_dh", q, k, gt, *dh_args)
+        N.call("tops_gla_chunk_bwd_dqkg", q, k, v, gt, *dqkg_tail)
     elif mode == GATE_GAMMA_K:
-        N.call("tops_gla_chunk_bwd_dh_gamma", N.ptr(q), N.ptr(k), N.ptr(gt), *dh_args)
-        N.call("tops_gla_chunk_bwd_dqkg_gamma", N.ptr(q), N.ptr(k), N.ptr(v), N.ptr(gt),
+        N.call("tops_gla_chunk_bwd_dh_gamma", q, k, gt, *dh_args)
+        N.call("tops_gla_chunk_bwd_dqkg_gamma", q, k, v, gt,
                *dqkg_tail)
     else:
-        N.call("tops_simple_gla_chunk_bwd_dh", N.ptr(q), N.ptr(k), *_gate_ptrs(gate), *dh_args)
-        N.call("tops_simple_gla_chunk_bwd_dqkg", N.ptr(q), N.ptr(k), N.ptr(v), *_gate_ptrs(gate),
+        N.call("tops_simple_gla_chunk_bwd_dh", q, k, *_gate_ptrs(gate), *dh_args)
+        N.call("tops_simple_gla_chunk_bwd_dqkg", q, k, v, *_gate_ptrs(gate),
                *dqkg_tail)
     dh0 = fin
     if sp is not None and fin is not None:
@@ -303,11 +303,11 @@ def _fwd_sliced(q, k, v, gate, h0, scale, output_final_state, plan: ChunkPlan, k
     for a in range(nk):
         k0 = a * Kp
         acc = _acc(a, nk)
-        N.call("tops_chunk_fwd_slice", N.ptr(q[..., k0:k0 + Kp]), N.ptr(k[..., k0:k0 + Kp]),
-               N.ptr(v), N.ptr(_k_gate(gate, k0, Kp)), code, N.ptr(_kv_view(h0, k0, Kp)),
-               N.ptr(o) if acc in (0, 3) else None, N.ptr(o_sum), acc,
-               N.ptr(_kv_view(ht, k0, Kp)), N.ptr(_kv_view(hs, k0, Kp)), N.ptr(plan.cu_dev),
-               N.ptr(plan.offsets_dev), B, T, H, Kp, V, plan.N, K, dt, float(scale), st)
+        N.call("tops_chunk_fwd_slice", q[..., k0:k0 + Kp], k[..., k0:k0 + Kp],
+               v, _k_gate(gate, k0, Kp), code, _kv_view(h0, k0, Kp),
+               o if acc in (0, 3) else None, o_sum, acc,
+               _kv_view(ht, k0, Kp), _kv_view(hs, k0, Kp), plan.cu_dev,
+               plan.offsets_dev, B, T, H, Kp, V, plan.N, K, dt, float(scale), st)
     return o, ht, hs
 
 
@@ -332,14 +332,14 @@ def _bwd_sliced(q, k, v, gate, do, dht, hs, scale, plan: ChunkPlan, want_dh0: bo
     dq_sum = torch.empty(B, T, H, K, device=dev, dtype=f32) if nv > 1 else None
     dk_sum = torch.empty_like(dq_sum) if nv > 1 else None
     code, dt, st = _GATE_CODE[mode], N.chunk_dtype_code(q.dtype), N.stream()
-    cu, offs = N.ptr(plan.cu_dev), N.ptr(plan.offsets_dev)
+    cu, offs = plan.cu_dev, plan.offsets_dev
     for a in range(nk):
         k0 = a * Kp
         acc = _acc(a, nk)
-        N.call("tops_chunk_bwd_dh_slice", N.ptr(q[..., k0:k0 + Kp]), N.ptr(k[..., k0:k0 + Kp]),
-               N.ptr(_k_gate(gate, k0, Kp)), code, N.ptr(do), N.ptr(_kv_view(dht, k0, Kp)),
-               N.ptr(_kv_view(dh_work, k0, Kp)), N.ptr(dv) if acc in (0, 3) else None,
-               N.ptr(dv_sum), acc, N.ptr(_kv_view(dh0, k0, Kp)), cu, offs, B, T, H, Kp, V,
+        N.call("tops_chunk_bwd_dh_slice", q[..., k0:k0 + Kp], k[..., k0:k0 + Kp],
+               _k_gate(gate, k0, Kp), code, do, _kv_view(dht, k0, Kp),
+               _kv_view(dh_work, k0, Kp), dv if acc in (0, 3) else None,
+               dv_sum, acc, _kv_view(dh0, k0, Kp), cu, offs, B, T, H, Kp, V,
                plan.N, K, dt, float(scale), st)
     first = True
     for a in range(nk):
@@ -350,15 +350,15 @@ def _bwd_sliced(q, k, v, gate, do, dht, hs, scale, plan: ChunkPlan, want_dh0: bo
             acc = _acc(b, nv)
             dga = None if dg is None else (dg[..., ks] if k_dg else dg)
             dg_accum = int(b > 0) if k_dg else int(not first)
-            N.call("tops_chunk_bwd_dqkg_slice", N.ptr(q[..., ks]), N.ptr(k[..., ks]),
-                   N.ptr(v[..., v0:v0 + Vp]), N.ptr(_k_gate(gate, k0, Kp)), code,
-                   N.ptr(do[..., v0:v0 + Vp]), N.ptr(_kv_view(hs, k0, Kp, v0, Vp)),
-                   N.ptr(_kv_view(dh_work, k0, Kp, v0, Vp)),
-                   N.ptr(dq[..., ks]) if acc in (0, 3) else None,
-                   N.ptr(dk[..., ks]) if acc in (0, 3) else None, N.ptr(dga),
-                   N.ptr(None if dq_sum is None else dq_sum[..., ks]),
-                   N.ptr(None if dk_sum is None else dk_sum[..., ks]), acc, dg_accum, cu, offs,
-                   N.ptr(plan.chunk_map_dev), plan.total, B, T, H, Kp, Vp, plan.N, K, V, dt,
+            N.call("tops_chunk_bwd_dqkg_slice", q[..., ks], k[..., ks],
+                   v[..., v0:v0 + Vp], _k_gate(gate, k0, Kp), code,
+                   do[..., v0:v0 + Vp], _kv_view(hs, k0, Kp, v0, Vp),
+                   _kv_view(dh_work, k0, Kp, v0, Vp),
+                   dq[..., ks] if acc in (0, 3) else None,
+                   dk[..., ks] if acc in (0, 3) else None, dga,
+                   None if dq_sum is None else dq_sum[..., ks],
+                   None if dk_sum is None else dk_sum[..., ks], acc, dg_accum, cu, offs,
+                   plan.chunk_map_dev, plan.total, B, T, H, Kp, Vp, plan.N, K, V, dt,
                    float(scale), st)
             first = False
     return dq, dk, dv, dg, dh0

@@ -22,7 +22,7 @@ from __future__ import annotations
 
 import torch
 
-from ...utils import ChunkPlan, cdiv, inference_inputs, to_device
+from ...utils import ChunkPlan, cdiv, f32, inference_inputs, to_device
 from .._chunk_core import (GATE_K, GATE_GAMMA, GATE_GAMMA_K, PAIRED, check_qkv, paired_states,
                            pack_states, states_fp32, unpack_states, chunk_fwd as _core_fwd,
                            chunk_bwd as _core_bwd)
@@ -54,8 +54,8 @@ class _ChunkGLA(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, gt, h0, mode, scale, output_final_state, cu_seqlens):
         q, k, v = (x.contiguous() for x in (q, k, v))
-        g32 = gt.detach().contiguous().to(torch.float32)
-        h032 = None if h0 is None else h0.contiguous().to(torch.float32)
+        g32 = f32(gt.detach())
+        h032 = f32(h0)
         plan = ChunkPlan.get(q.shape[0], q.shape[1], cu_seqlens, q.device)
         train = any(ctx.needs_input_grad[:5])
         o, ht, hs = _core_fwd(q, k, v, (mode, g32), h032, scale, output_final_state, plan,
@@ -73,7 +73,7 @@ class _ChunkGLA(torch.autograd.Function):
         q, k, v, g32, hs, hsc, h032 = ctx.saved_tensors
         hs = unpack_states(hs, hsc)
         do = do.contiguous().to(q.dtype)
-        dht = None if dht is None else dht.contiguous().to(torch.float32)
+        dht = f32(dht)
         want_dh0 = ctx.h0_info is not None
         want_dg = bool(ctx.needs_input_grad[3])
         dq, dk, dv, dg, dh0 = _core_bwd(q, k, v, (ctx.mode, g32), do, dht, hs, ctx.scale,
@@ -203,8 +203,8 @@ def chunk_gla_fwd(q, k, v, g, g_gamma, g_cumsum, scale, initial_state, output_fi
         mode, gt = _gate(q, g, g_gamma)
     plan = ChunkPlan.get(B, T, cu_seqlens, q.device)
     q, k, v = (x.contiguous() for x in (q, k, v))
-    g32 = gt.detach().contiguous().to(torch.float32)
-    h0 = None if initial_state is None else initial_state.contiguous().to(torch.float32)
+    g32 = f32(gt.detach())
+    h0 = f32(initial_state)
     o, ht, hs = _core_fwd(q, k, v, (mode, g32), h0, scale, output_final_state, plan,
                           keep_states=C == 64)
     qp, kp = pad.pad(q), pad.pad(k)
@@ -244,15 +244,15 @@ def chunk_gla_bwd(q, k, v, g, g_gamma, g_cumsum, scale, initial_state, h, A, do,
     mode, gt = _gate(q, g, g_gamma)
     plan = ChunkPlan.get(B, T, cu_seqlens, q.device)
     q, k, v = (x.contiguous() for x in (q, k, v))
-    g32 = gt.detach().contiguous().to(torch.float32)
-    h0 = None if initial_state is None else initial_state.contiguous().to(torch.float32)
+    g32 = f32(gt.detach())
+    h0 = f32(initial_state)
     if h is None or int(chunk_size) != 64:
         _, _, hs = _core_fwd(q, k, v, (mode, g32), h0, scale, False, plan, keep_states=True)
     else:
         hs = h.reshape(plan.total, H, K, V).contiguous().to(torch.float32)
     want_dh0 = initial_state is not None or dht is not None
     dq, dk, dv, dg, dh0 = _core_bwd(q, k, v, (mode, g32), do.contiguous().to(q.dtype),
-                                    None if dht is None else dht.contiguous().to(torch.float32),
+                                    f32(dht),
                                     hs, scale, plan, want_dh0, True)
     if g is None and g_gamma is not None:
         gg = torch.as_tensor(g_gamma)

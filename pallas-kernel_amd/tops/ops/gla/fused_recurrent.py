@@ -31,7 +31,7 @@ import numpy as np
 import torch
 
 from ... import _native as N
-from ...utils import ChunkPlan, inference_inputs, to_device
+from ...utils import ChunkPlan, f32 as _f32, inference_inputs, to_device
 
 
 def _cu_dev(cu_seqlens, device):
@@ -91,18 +91,14 @@ def _sliced(q, k, v, gk, gv, scale, initial_state, output_final_state, reverse, 
     return o.to(q.dtype), ht
 
 
-def _f32(x):
-    return None if x is None else x.contiguous().to(torch.float32)
-
-
 def _fwd(q, k, v, gk32, gv32, h032, scale, output_final_state, reverse, cu, n, want_o32):
     B, T, H, K = q.shape
     V = v.shape[-1]
     o = torch.empty_like(v)
     o32 = torch.empty(B, T, H, V, device=q.device, dtype=torch.float32) if want_o32 else None
     ht = torch.empty(n, H, K, V, device=q.device, dtype=torch.float32) if output_final_state else None
-    N.call("tops_gla_fused_recurrent_fwd", N.ptr(q), N.ptr(k), N.ptr(v), N.ptr(gk32), N.ptr(gv32),
-           N.ptr(h032), N.ptr(o), N.ptr(o32), N.ptr(ht), N.ptr(cu), B, T, H, K, V, n,
+    N.call("tops_gla_fused_recurrent_fwd", q, k, v, gk32, gv32,
+           h032, o, o32, ht, cu, B, T, H, K, V, n,
            N.dtype_code(q.dtype), float(scale), int(bool(reverse)), N.stream())
     return o, o32, ht
 
@@ -117,9 +113,9 @@ def _bwd(q, k, v, gk32, gv32, o32, do, dht32, h032, scale, reverse, cu, n):
     ws_bytes = N.lib().tops_gla_fused_recurrent_bwd_workspace(B, T, H, K, V, n,
                                                               int(gv32 is not None))
     ws = torch.empty((ws_bytes + 3) // 4, device=q.device, dtype=torch.float32)
-    N.call("tops_gla_fused_recurrent_bwd", N.ptr(q), N.ptr(k), N.ptr(v), N.ptr(gk32), N.ptr(gv32),
-           N.ptr(o32), N.ptr(do), N.ptr(dht32), N.ptr(h032), N.ptr(dq), N.ptr(dk), N.ptr(dv),
-           N.ptr(dgk), N.ptr(dgv), N.ptr(dh0), N.ptr(ws), N.ptr(cu), B, T, H, K, V, n,
+    N.call("tops_gla_fused_recurrent_bwd", q, k, v, gk32, gv32,
+           o32, do, dht32, h032, dq, dk, dv,
+           dgk, dgv, dh0, ws, cu, B, T, H, K, V, n,
            N.dtype_code(q.dtype), float(scale), int(bool(reverse)), N.stream())
     return dq, dk, dv, dgk, dgv, dh0
 
@@ -195,8 +191,8 @@ def reverse_chunk_native(q, k, v, mode, g, initial_state, scale, output_final_st
     o = torch.empty_like(v)
     ht = torch.empty(plan.N, H, K, V, device=q.device, dtype=torch.float32) \
         if output_final_state else None
-    N.call("tops_chunk_reverse_fwd", N.ptr(q), N.ptr(k), N.ptr(v), N.ptr(gt), _REV_GATE_CODE[mode],
-           N.ptr(_f32(initial_state)), N.ptr(o), N.ptr(ht), N.ptr(plan.cu_dev), B, T, H, K, V,
+    N.call("tops_chunk_reverse_fwd", q, k, v, gt, _REV_GATE_CODE[mode],
+           _f32(initial_state), o, ht, plan.cu_dev, B, T, H, K, V,
            plan.N, N.dtype_code(q.dtype), float(scale), N.stream())
     return o, ht
 
@@ -220,8 +216,8 @@ def gv_chunk_native(q, k, v, gv, initial_state, scale, output_final_state, cu_se
     o = torch.empty_like(v)
     ht = torch.empty(plan.N, H, K, V, device=q.device, dtype=torch.float32) \
         if output_final_state else None
-    N.call("tops_gla_chunk_fwd_gv", N.ptr(q), N.ptr(k), N.ptr(v), N.ptr(_f32(gv)),
-           N.ptr(_f32(initial_state)), N.ptr(o), N.ptr(ht), N.ptr(plan.cu_dev), B, T, H, K, V,
+    N.call("tops_gla_chunk_fwd_gv", q, k, v, _f32(gv),
+           _f32(initial_state), o, ht, plan.cu_dev, B, T, H, K, V,
            plan.N, N.dtype_code(q.dtype), float(scale), N.stream())
     return o, ht
 
@@ -264,8 +260,8 @@ class _GvChunk(torch.autograd.Function):
         o32 = torch.empty(B, T, H, V, device=q.device, dtype=torch.float32)
         o = torch.empty(B, T, H, V, device=q.device, dtype=q.dtype)
         ht = torch.empty(plan.N, H, K, V, device=q.device, dtype=torch.float32)
-        N.call("tops_gla_chunk_fwd_gv32", N.ptr(q), N.ptr(k), N.ptr(v), N.ptr(gv32), N.ptr(h032),
-               N.ptr(o32), N.ptr(o), N.ptr(ht), N.ptr(plan.cu_dev), B, T, H, K, V, plan.N,
+        N.call("tops_gla_chunk_fwd_gv32", q, k, v, gv32, h032,
+               o32, o, ht, plan.cu_dev, B, T, H, K, V, plan.N,
                N.dtype_code(q.dtype), float(scale), N.stream())
         ctx.save_for_backward(q, k, v, gv32, h032, o32, ht)
         ctx.scale, ctx.cu = scale, cu_seqlens
@@ -295,22 +291,22 @@ class _GvChunk(torch.autograd.Function):
         # dk: the key-gated state-gradient sweep on the transposed state gradient (its dv)
         dk = torch.empty_like(q)
         dht_t = None if dht32 is None else dht32.transpose(-1, -2).contiguous()   # [N, H, V, K]
-        N.call("tops_gla_chunk_rev_dv", N.ptr(do), N.ptr(v), N.ptr(gv), N.ptr(q), N.ptr(dht_t),
-               N.ptr(dk), None, N.ptr(plan.cu_dev), B, T, H, V, K, plan.N,
+        N.call("tops_gla_chunk_rev_dv", do, v, gv, q, dht_t,
+               dk, None, plan.cu_dev, B, T, H, V, K, plan.N,
                N.dtype_code(q.dtype), float(scale), N.stream())
         # dv (fp32) and dh0: the value-gated state-gradient sweep
         dv32 = torch.empty(B, T, H, V, device=dev, dtype=torch.float32)
         dh0 = None if h0 is None else torch.empty_like(h0)
-        N.call("tops_gla_chunk_bwd_dv_gv32", N.ptr(q), N.ptr(k), N.ptr(do), N.ptr(gv), N.ptr(dht32),
-               N.ptr(dv32), N.ptr(dh0), N.ptr(plan.cu_dev), B, T, H, K, V, plan.N,
+        N.call("tops_gla_chunk_bwd_dv_gv32", q, k, do, gv, dht32,
+               dv32, dh0, plan.cu_dev, B, T, H, K, V, plan.N,
                N.dtype_code(q.dtype), float(scale), N.stream())
         # dgv: suffix sums of o dO - v dv, plus the final state's term (tops_gv_gate_grad)
         c = None if dht32 is None else (dht32 * ht).sum(-2).contiguous()      # [N, H, V]
         # and the bf16 dv, rounded from dv32 on the same walk
         dgv = torch.empty(B, T, H, V, device=dev, dtype=torch.float32)
         dv = torch.empty(B, T, H, V, device=dev, dtype=v.dtype)
-        N.call("tops_gv_gate_grad", N.ptr(o32), N.ptr(do), N.ptr(v), N.ptr(dv32), N.ptr(c),
-               N.ptr(dgv), N.ptr(dv), N.ptr(plan.cu_dev), B, T, H, V, plan.N,
+        N.call("tops_gv_gate_grad", o32, do, v, dv32, c,
+               dgv, dv, plan.cu_dev, B, T, H, V, plan.N,
                N.dtype_code(q.dtype), N.stream())
         gdt, hdt = ctx.dtypes
         return (dq, dk, dv, dgv.to(gdt), None if dh0 is None else dh0.to(hdt),
@@ -361,9 +357,9 @@ def decode_native(q, k, v, gk, gv, initial_state, scale, output_final_state, rev
     q, k, v = (x.contiguous() for x in (q, k, v))
     o = torch.empty_like(v)
     ht = torch.empty(n, H, K, V, device=q.device, dtype=torch.float32) if output_final_state else None
-    N.call("tops_gla_fused_recurrent_fwd_decode", N.ptr(q), N.ptr(k), N.ptr(v), N.ptr(_f32(gk)),
-           N.ptr(_f32(gv)), N.ptr(_f32(initial_state)), N.ptr(o), None, N.ptr(ht),
-           N.ptr(_cu_dev(cu_seqlens, q.device)), B, T, H, K, V, n, N.dtype_code(q.dtype),
+    N.call("tops_gla_fused_recurrent_fwd_decode", q, k, v, _f32(gk),
+           _f32(gv), _f32(initial_state), o, None, ht,
+           _cu_dev(cu_seqlens, q.device), B, T, H, K, V, n, N.dtype_code(q.dtype),
            float(scale), int(bool(reverse)), N.stream())
     return o, ht
 
@@ -457,10 +453,10 @@ def fused_recurrent_gla_norm_gate(q, k, v, gk=None, gv=None, g=None, weight=None
     q, k, v = (x.contiguous() for x in (q, k, v))
     y = torch.empty_like(v)
     ht = torch.empty(n, H, K, V, device=q.device, dtype=torch.float32) if output_final_state else None
-    N.call("tops_gla_fused_recurrent_fwd_decode_norm_gate", N.ptr(q), N.ptr(k), N.ptr(v),
-           N.ptr(_f32(gk)), N.ptr(_f32(gv)), N.ptr(_f32(initial_state)),
-           N.ptr(None if g is None else g.contiguous()), N.ptr(_f32(weight)), float(eps),
-           N.ptr(y), N.ptr(ht), N.ptr(_cu_dev(cu_seqlens, q.device)), B, T, H, K, V, n,
+    N.call("tops_gla_fused_recurrent_fwd_decode_norm_gate", q, k, v,
+           _f32(gk), _f32(gv), _f32(initial_state),
+           None if g is None else g.contiguous(), _f32(weight), float(eps),
+           y, ht, _cu_dev(cu_seqlens, q.device), B, T, H, K, V, n,
            N.dtype_code(q.dtype), float(scale), int(bool(reverse)), N.stream())
     return y, ht
 
@@ -535,20 +531,19 @@ def fused_recurrent_gla_conv_norm_gate(x_q, x_k, x_v, conv_weights, conv_biases=
         return y, ht, (tuple(new) if any(c is not None for c in new) else None)
     xs = [x.contiguous() for x in (x_q, x_k, x_v)]
     dev = x_q.device
-    w32 = [w.to(torch.float32).contiguous() for w in ws]
-    b32 = [None if b is None else b.to(torch.float32).contiguous() for b in bs]
+    w32 = [_f32(w) for w in ws]
+    b32 = [_f32(b) for b in bs]
     # a decode step reads and rolls the caches; a prefill reads none and keeps the last W inputs
     keep = output_final_state or (step and cs[0] is not None)
-    cin = [None if (c is None or not step) else c.to(torch.float32).contiguous() for c in cs]
+    cin = [None if not step else _f32(c) for c in cs]
     cout = [torch.empty(n, D, W, device=dev, dtype=torch.float32) if keep else None for D in dims]
     y = torch.empty(B, T, H, V, device=dev, dtype=ydt)
     ht = torch.empty(n, H, K, V, device=dev, dtype=torch.float32) if output_final_state else None
-    N.call("tops_gla_decode_conv_norm_gate", *(N.ptr(x) for x in xs), *(N.ptr(w) for w in w32),
-           *(N.ptr(b) for b in b32), *(N.ptr(c) for c in cin), *(N.ptr(c) for c in cout), W,
-           _act(conv_activation), N.ptr(_f32(gk)), N.ptr(_f32(initial_state)),
-           N.ptr(None if g is None else g.contiguous()), N.ptr(_f32(weight)), float(eps), N.ptr(y),
-           int(ydt == torch.float32 and x_q.dtype != torch.float32), N.ptr(ht),
-           N.ptr(_cu_dev(cu_seqlens, dev)), B, T, H, K, V, n, N.dtype_code(x_q.dtype),
+    N.call("tops_gla_decode_conv_norm_gate", *xs, *w32, *b32, *cin, *cout, W,
+           _act(conv_activation), _f32(gk), _f32(initial_state),
+           None if g is None else g.contiguous(), _f32(weight), float(eps), y,
+           int(ydt == torch.float32 and x_q.dtype != torch.float32), ht,
+           _cu_dev(cu_seqlens, dev), B, T, H, K, V, n, N.dtype_code(x_q.dtype),
            float(scale), N.stream())
     new = None
     if keep:

@@ -25,7 +25,8 @@ import numpy as np
 import torch
 
 from ... import _native as N
-from ...utils import CHUNK, ChunkPlan, cdiv, checkpoint_layout, inference_inputs
+from ...utils import (CHUNK, ChunkPlan, cdiv, checkpoint_layout, f32 as to_f32,
+                      inference_inputs)
 from .._chunk_core import States16, check_qkv, pack_states, unpack_states
 
 
@@ -58,17 +59,17 @@ def _fwd(q, k, v, g32, b32, h0, scale, output_final_state, plan: ChunkPlan, keep
     w = torch.empty(B, T, H, K, device=dev, dtype=f32)
     tt = torch.empty(plan.total, H, CHUNK, CHUNK, device=dev, dtype=f32) if keep else None
     vn = torch.empty(B, T, H, V, device=dev, dtype=f32) if keep else None
-    tail = (N.ptr(plan.cu_dev), N.ptr(plan.offsets_dev), N.ptr(plan.chunk_map_dev), plan.total,
+    tail = (plan.cu_dev, plan.offsets_dev, plan.chunk_map_dev, plan.total,
             B, T, H, K, V, plan.N, N.dtype_code(q.dtype), float(scale), N.stream())
-    head = (N.ptr(q), N.ptr(k), N.ptr(v), N.ptr(g32), N.ptr(b32), N.ptr(h0), N.ptr(o), N.ptr(ht),
-            N.ptr(u), N.ptr(w), N.ptr(tt), N.ptr(vn))
+    head = (q, k, v, g32, b32, h0, o, ht,
+            u, w, tt, vn)
     if keep and _c16(q):
         hs = States16(torch.empty(plan.total, H, K, V, device=dev, dtype=torch.float16),
                       torch.empty(plan.total, H, cdiv(V, 64), device=dev, dtype=f32))
-        N.call("tops_kda_chunk_fwd_c16", *head, N.ptr(hs.h), N.ptr(hs.scale), *tail)
+        N.call("tops_kda_chunk_fwd_c16", *head, hs.h, hs.scale, *tail)
     else:
         hs = torch.empty(plan.total, H, K, V, device=dev, dtype=f32) if keep else None
-        N.call("tops_kda_chunk_fwd", *head, N.ptr(hs), *tail)
+        N.call("tops_kda_chunk_fwd", *head, hs, *tail)
     return o, ht, (w, tt, vn, hs)
 
 
@@ -83,23 +84,23 @@ def _bwd(q, k, v, g32, b32, do, dht, saved, scale, plan: ChunkPlan, want_dh0: bo
     dg = torch.empty(B, T, H, K, device=dev, dtype=f32)
     dh0 = torch.empty(plan.N, H, K, V, device=dev, dtype=f32) if want_dh0 else None
     dvn_work = torch.empty(plan.total, H, V, CHUNK, device=dev, dtype=f32)
-    tail = (N.ptr(dh0), N.ptr(plan.cu_dev), N.ptr(plan.offsets_dev), N.ptr(plan.chunk_map_dev),
+    tail = (dh0, plan.cu_dev, plan.offsets_dev, plan.chunk_map_dev,
             plan.total, B, T, H, K, V, plan.N, N.dtype_code(q.dtype), float(scale), N.stream())
     if isinstance(hs, States16):
         dh_work = States16(torch.empty_like(hs.h), torch.empty_like(hs.scale))
-        N.call("tops_kda_chunk_bwd_c16", N.ptr(q), N.ptr(k), N.ptr(v), N.ptr(g32), N.ptr(b32),
-               N.ptr(w), N.ptr(tt), N.ptr(vn), N.ptr(hs.h), N.ptr(hs.scale), N.ptr(do), N.ptr(dht),
-               N.ptr(dh_work.h), N.ptr(dh_work.scale), N.ptr(dvn_work), N.ptr(dq), N.ptr(dk),
-               N.ptr(dv), N.ptr(dbeta), N.ptr(dg), *tail)
+        N.call("tops_kda_chunk_bwd_c16", q, k, v, g32, b32,
+               w, tt, vn, hs.h, hs.scale, do, dht,
+               dh_work.h, dh_work.scale, dvn_work, dq, dk,
+               dv, dbeta, dg, *tail)
         return dq, dk, dv, dbeta, dg, dh0
     dh_work = torch.empty_like(hs)
     # bf16 keeps the WY parts of dk / dg on chip (one kernel); fp32 passes them through HBM
     split = q.dtype == torch.float32
     dk_work = torch.empty(B, T, H, K, device=dev, dtype=f32) if split else None
     dg_work = torch.empty(B, T, H, K, device=dev, dtype=f32) if split else None
-    N.call("tops_kda_chunk_bwd", N.ptr(q), N.ptr(k), N.ptr(v), N.ptr(g32), N.ptr(b32), N.ptr(w),
-           N.ptr(tt), N.ptr(vn), N.ptr(hs), N.ptr(do), N.ptr(dht), N.ptr(dh_work), N.ptr(dvn_work),
-           N.ptr(dk_work), N.ptr(dg_work), N.ptr(dq), N.ptr(dk), N.ptr(dv), N.ptr(dbeta), N.ptr(dg),
+    N.call("tops_kda_chunk_bwd", q, k, v, g32, b32, w,
+           tt, vn, hs, do, dht, dh_work, dvn_work,
+           dk_work, dg_work, dq, dk, dv, dbeta, dg,
            *tail)
     return dq, dk, dv, dbeta, dg, dh0
 
@@ -108,9 +109,9 @@ class _ChunkKDA(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, g, beta, scale, h0, output_final_state, cu_seqlens):
         q, k, v = (x.contiguous() for x in (q, k, v))
-        g32 = g.contiguous().to(torch.float32)
-        b32 = beta.contiguous().to(torch.float32)
-        h032 = None if h0 is None else h0.contiguous().to(torch.float32)
+        g32 = to_f32(g)
+        b32 = to_f32(beta)
+        h032 = to_f32(h0)
         plan = ChunkPlan.get(q.shape[0], q.shape[1], cu_seqlens, q.device)
         train = any(ctx.needs_input_grad[:5]) or (h0 is not None and ctx.needs_input_grad[6])
         o, ht, saved = _fwd(q, k, v, g32, b32, h032, scale, output_final_state, plan, keep=train)
@@ -125,7 +126,7 @@ class _ChunkKDA(torch.autograd.Function):
         q, k, v, g32, b32, w, tt, vn, hs, hsc = ctx.saved_tensors
         hs = unpack_states(hs, hsc)
         do = do.contiguous().to(q.dtype)
-        dht = None if dht is None else dht.contiguous().to(torch.float32)
+        dht = to_f32(dht)
         g_dt, b_dt, h0_dt = ctx.dtypes
         dq, dk, dv, dbeta, dg, dh0 = _bwd(q, k, v, g32, b32, do, dht, (w, tt, vn, hs), ctx.scale,
                                           ctx.plan, want_dh0=h0_dt is not None)
@@ -248,9 +249,9 @@ def chunk_kda_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Te
     if scale is None:
         scale = q.shape[-1] ** -0.5
     q, k, v = (x.contiguous() for x in (q, k, v))
-    g32 = g.contiguous().to(torch.float32)
-    b32 = beta.contiguous().to(torch.float32)
-    h0 = None if initial_state is None else initial_state.contiguous().to(torch.float32)
+    g32 = to_f32(g)
+    b32 = to_f32(beta)
+    h0 = to_f32(initial_state)
     plan = ChunkPlan.get(q.shape[0], q.shape[1], cu_seqlens, q.device)
     from .gate import kda_gate_chunk_cumsum
     with torch.no_grad():

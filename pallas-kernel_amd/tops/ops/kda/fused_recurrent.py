@@ -27,7 +27,7 @@ from __future__ import annotations
 import torch
 
 from ... import _native as N
-from ...utils import to_device
+from ...utils import f32, to_device
 from ..gla.fused_recurrent import decode_sized
 from .chunk import _prologue, chunk_kda
 from .l2norm import l2norm
@@ -47,12 +47,11 @@ def _decode(q, k, v, g, beta, scale, h0, output_final_state, cu_seqlens, n):
     if not decode_sized(T, cu_seqlens):
         return None
     q, k, v = (x.contiguous() for x in (q, k, v))
-    f32 = lambda x: None if x is None else x.contiguous().to(torch.float32)  # noqa: E731
     o = torch.empty_like(v)
     ht = torch.empty(n, H, K, V, device=q.device, dtype=torch.float32) if output_final_state else None
     cu = None if cu_seqlens is None else to_device(cu_seqlens, q.device, torch.int32)
-    N.call("tops_kda_fused_recurrent_fwd_decode", N.ptr(q), N.ptr(k), N.ptr(v), N.ptr(f32(g)),
-           N.ptr(f32(beta)), N.ptr(f32(h0)), N.ptr(o), N.ptr(ht), N.ptr(cu), B, T, H, K, V, n,
+    N.call("tops_kda_fused_recurrent_fwd_decode", q, k, v, f32(g),
+           f32(beta), f32(h0), o, ht, cu, B, T, H, K, V, n,
            N.dtype_code(q.dtype), float(K ** -0.5 if scale is None else scale), N.stream())
     return o, ht
 

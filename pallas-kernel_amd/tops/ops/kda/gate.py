@@ -79,8 +79,8 @@ def _gate_fwd(g: torch.Tensor, A_log, dt_bias, lower_bound) -> torch.Tensor:
     y = torch.empty(g.shape, device=g.device, dtype=torch.float32)
     mode, lb = _mode(lower_bound)
     rows = g.numel() // (H * K) if H * K else 0
-    N.call("tops_kda_gate_fwd", N.ptr(gk), N.dtype_code(gk.dtype), N.ptr(a32), N.ptr(b32),
-           N.ptr(y), rows, H, K, ha, hb, mode, lb, N.stream())
+    N.call("tops_kda_gate_fwd", gk, N.dtype_code(gk.dtype), a32, b32,
+           y, rows, H, K, ha, hb, mode, lb, N.stream())
     return y
 
 
@@ -102,8 +102,8 @@ def _gate_bwd(g: torch.Tensor, A_log, dt_bias, dyg: torch.Tensor, lower_bound):
         raise ValueError(f"tops_kda_gate_bwd_workspace({rows}, {H}, {K}) failed")
     ws = torch.empty(max(n_ws, 1), device=g.device, dtype=torch.float32)
     mode, lb = _mode(lower_bound)
-    N.call("tops_kda_gate_bwd", N.ptr(gk), N.dtype_code(gk.dtype), N.ptr(a32), N.ptr(b32),
-           N.ptr(dy), N.ptr(dg), N.ptr(dA), N.ptr(db), N.ptr(ws), n_ws, rows, H, K, ha, hb,
+    N.call("tops_kda_gate_bwd", gk, N.dtype_code(gk.dtype), a32, b32,
+           dy, dg, dA, db, ws, n_ws, rows, H, K, ha, hb,
            mode, lb, N.stream())
     return (dg.to(g.dtype), dA.to(A_log.dtype),
             None if db is None else db.to(dt_bias.dtype))
@@ -182,9 +182,9 @@ def _cumsum(g, A_log, dt_bias, lower_bound, mode, scale, chunk_size: int, cu_seq
         return out
     plan = ChunkPlan.get(B, T, cu_seqlens, g.device, int(chunk_size))
     with torch.no_grad():
-        N.call("tops_kda_gate_chunk_cumsum", N.ptr(gk), N.dtype_code(gk.dtype), N.ptr(a32),
-               N.ptr(b32), N.ptr(out), N.ptr(plan.cu_dev), N.ptr(plan.offsets_dev),
-               N.ptr(plan.chunk_map_dev), plan.total, B, T, H, K, ha, hb, int(chunk_size),
+        N.call("tops_kda_gate_chunk_cumsum", gk, N.dtype_code(gk.dtype), a32,
+               b32, out, plan.cu_dev, plan.offsets_dev,
+               plan.chunk_map_dev, plan.total, B, T, H, K, ha, hb, int(chunk_size),
                mode, lb, float(scale), N.stream())
     return out
 

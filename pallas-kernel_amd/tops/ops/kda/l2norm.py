@@ -27,7 +27,7 @@ class _L2Norm(torch.autograd.Function):
         D = x.shape[-1]
         rows = x.numel() // D if D else 0
         y = torch.empty(x.shape, device=x.device, dtype=torch.float32)
-        N.call("tops_l2norm_fwd", N.ptr(xk), N.dtype_code(xk.dtype), N.ptr(y), rows, D,
+        N.call("tops_l2norm_fwd", xk, N.dtype_code(xk.dtype), y, rows, D,
                N.stream())
         ctx.save_for_backward(xk)
         ctx.in_dtype = x.dtype
@@ -40,7 +40,7 @@ class _L2Norm(torch.autograd.Function):
         rows = xk.numel() // D if D else 0
         dy = dy.contiguous().to(torch.float32)
         dx = torch.empty_like(xk)
-        N.call("tops_l2norm_bwd", N.ptr(xk), N.dtype_code(xk.dtype), N.ptr(dy), N.ptr(dx),
+        N.call("tops_l2norm_bwd", xk, N.dtype_code(xk.dtype), dy, dx,
                rows, D, N.stream())
         return dx.to(ctx.in_dtype)
 

@@ -20,7 +20,7 @@ from __future__ import annotations
 
 import torch
 
-from ...utils import ChunkPlan, inference_inputs
+from ...utils import ChunkPlan, f32, inference_inputs
 from .._chunk_core import (GATE_S, GATE_GAMMA, PAIRED, check_qkv, chunk_fwd as _core_fwd,
                            chunk_bwd as _core_bwd, pack_states, paired_states,
                            unpack_states)
@@ -45,8 +45,8 @@ class _ChunkSimpleGLA(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, gt, h0, mode, scale, output_final_state, cu_seqlens):
         q, k, v = (x.contiguous() for x in (q, k, v))
-        g32 = gt.detach().contiguous().to(torch.float32)
-        h032 = None if h0 is None else h0.contiguous().to(torch.float32)
+        g32 = f32(gt.detach())
+        h032 = f32(h0)
         plan = ChunkPlan.get(q.shape[0], q.shape[1], cu_seqlens, q.device)
         train = any(ctx.needs_input_grad[:5])
         o, ht, hs = _core_fwd(q, k, v, (mode, g32), h032, scale, output_final_state, plan,
@@ -64,7 +64,7 @@ class _ChunkSimpleGLA(torch.autograd.Function):
         q, k, v, g32, hs, hsc, h032 = ctx.saved_tensors
         hs = unpack_states(hs, hsc)
         do = do.contiguous().to(q.dtype)
-        dht = None if dht is None else dht.contiguous().to(torch.float32)
+        dht = f32(dht)
         dq, dk, dv, dg, dh0 = _core_bwd(q, k, v, (ctx.mode, g32), do, dht, hs, ctx.scale,
                                         ctx.plan, ctx.h0_info is not None, h0=h032,
                                         paired=ctx.paired)
@@ -135,9 +135,9 @@ def chunk_simple_gla_fwd(q, k, v, g=None, g_gamma=None, scale=None, initial_stat
     if scale is None:
         scale = q.shape[-1] ** -0.5
     plan = ChunkPlan.get(q.shape[0], q.shape[1], cu_seqlens, q.device)
-    h0 = None if initial_state is None else initial_state.contiguous().to(torch.float32)
+    h0 = f32(initial_state)
     o, ht, _ = _core_fwd(q.contiguous(), k.contiguous(), v.contiguous(),
-                         (mode, gt.contiguous().to(torch.float32)), h0, scale,
+                         (mode, f32(gt)), h0, scale,
                          output_final_state, plan, keep_states=False)
     return o, ht
 
@@ -183,9 +183,9 @@ def _bwd_all(q, k, v, do, g, g_gamma, scale, h0, dht, cu_seqlens):
         scale = q.shape[-1] ** -0.5
     plan = ChunkPlan.get(q.shape[0], q.shape[1], cu_seqlens, q.device)
     q, k, v = (x.contiguous() for x in (q, k, v))
-    g32 = gt.contiguous().to(torch.float32)
-    h032 = None if h0 is None else h0.contiguous().to(torch.float32)
+    g32 = f32(gt)
+    h032 = f32(h0)
     _, _, hs = _core_fwd(q, k, v, (mode, g32), h032, scale, False, plan, keep_states=True)
     return _core_bwd(q, k, v, (mode, g32), do.contiguous().to(q.dtype),
-                     None if dht is None else dht.contiguous().to(torch.float32), hs, scale, plan,
+                     f32(dht), hs, scale, plan,
                      h0 is not None)

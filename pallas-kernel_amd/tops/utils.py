@@ -26,6 +26,13 @@ def inference_inputs(*ts):
     return tuple(t.detach() if isinstance(t, torch.Tensor) else t for t in ts)
 
 
+def f32(x):
+    """x (or None) as contiguous float32, itself where it is that already."""
+    if x is None or (x.dtype == torch.float32 and x.is_contiguous()):
+        return x
+    return x.contiguous().to(torch.float32)
+
+
 def _host_cu(cu_seqlens) -> np.ndarray:
     if isinstance(cu_seqlens, torch.Tensor):
         cu_seqlens = cu_seqlens.detach().cpu().numpy()
@@ -100,7 +107,7 @@ class ChunkPlan:
         """The plan for these sizes / sequence boundaries, reused across calls (the maps
         depend only on the boundaries)."""
         cu = None if cu_seqlens is None else _host_cu(cu_seqlens)
-        key = (B, T, C, str(torch.device(device)), None if cu is None else cu.tobytes())
+        key = (B, T, C, torch.device(device), None if cu is None else cu.tobytes())
         plan = _PLANS.get(key)
         if plan is None:
             plan = cls(B, T, cu, device, C)
