@@ -176,6 +176,12 @@ __global__ __launch_bounds__(512, 1) void kda_bwd_fused_kernel(KdaBwdParams p) {
   // B: dAkk tiles (registers, all passes).  dar[a][J] (J <= t): lane holds
   // dAkk[16t + l16][16J + 4lg + r];  dac[a][J] (J >= t): beta_i dAkk[16J + 4lg + r][16t + l16]
   constexpr int NVW = (NVB + 3) / 4;     // V blocks per B wave
+  // Group B requests the state rows of a pass a pass ahead, where the previous ones have been
+  // split (past the last pass the descriptor's bound returns zeros): at the head of the pass
+  // their latency stood before its first product, since one workgroup per CU has no other
+  // waves to hide it.  Backward entry 2960 -> 2745 us at B4 T8192 H32 K=V=128.  Only fp16 rows,
+  // half the registers of fp32 ones, and only group B: group A has none left (spills, 3130 us)
+  constexpr bool AHEAD = C16;
   // ================================================================ channel passes
   const rsrc_t Rdh = C16 ? make_rsrc((const uint16_t*)p.dhs + so, KVB) : make_rsrc(p.dhs + so, KVB);
   const rsrc_t Rdq = make_rsrc_rows((uint16_t*)p.dq, e0, nrows, K);
@@ -483,6 +489,7 @@ __global__ __launch_bounds__(512, 1) void kda_bwd_fused_kernel(KdaBwdParams p) {
   auto runB = [&](auto RHc) {
   constexpr int rh = decltype(RHc)::value;
   uint2 darh[2][4], darl[2][4], dach[2][4], dacl[2][4];
+  uint4 hraw[VC][2];
     // B: the P phase's global operands (dv_new^T and T^T fragments, v rows), requested first
     uint4 pdraw[NVW][2][2], ptraw[4][2][2];
     Wd::W4 pvraw[NVW][4];
@@ -520,6 +527,7 @@ __global__ __launch_bounds__(512, 1) void kda_bwd_fused_kernel(KdaBwdParams p) {
       }
     }
     if (tq < C) sBeta[tq] = __uint_as_float(braw);
+    if constexpr (AHEAD) load_state(Rh, hraw, 0);
     __syncthreads();  // P1: v_new / dO planes and beta visible
     {
     // B: P = T^T dv_new, tiles (vb, I) computed transposed: lane holds P[16I + l16][16vb + 4lg + r]
@@ -603,12 +611,11 @@ __global__ __launch_bounds__(512, 1) void kda_bwd_fused_kernel(KdaBwdParams p) {
       }
     }
 
-  uint4 hraw[VC][2];
   float dbk_acc[2] = {0.f, 0.f};  // per token: sum over channels of 2^G k dbk + k Y1
 #pragma unroll 1
   for (int ps = 0; ps < NPS; ++ps) {
     const int cb = ps * KH;
-    load_state(Rh, hraw, ps);              // S rows of dbk
+    if constexpr (!AHEAD) load_state(Rh, hraw, ps);   // S rows of dbk
     // k of the epilogue's (token, 4 channels), requested with the state rows
     Wd::W4 kvraw[2];
 #pragma unroll
@@ -636,6 +643,7 @@ __global__ __launch_bounds__(512, 1) void kda_bwd_fused_kernel(KdaBwdParams p) {
         sh[vc] = __builtin_bit_cast(bf16x8, make_uint4(h4[0], h4[1], h4[2], h4[3]));
         sl[vc] = __builtin_bit_cast(bf16x8, make_uint4(l4[0], l4[1], l4[2], l4[3]));
       }
+      if constexpr (AHEAD) load_state(Rh, hraw, ps + 1);
       const float4 gm4 = *(const float4*)(sGm + cl);
       const float gmr[4] = {gm4.x, gm4.y, gm4.z, gm4.w};
 #pragma unroll
