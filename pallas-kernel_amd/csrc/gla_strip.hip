@@ -37,6 +37,8 @@
 // stored from the accumulators it was 64 four-byte-per-lane stores per chunk that held the
 // consumers up (interval A 4,600 -> 2,700 cycles).  Producers run at raised wave priority
 // where they are the longer side (interval A; in training B as well: 8,900 -> 8,100 cycles).
+// fp32 checkpoints (more than 128 value columns) take the same route, 16-byte stores of 256-byte
+// rows: chunk_gla forward and backward, B8 T1000 H8 K=128 V=256 bf16, 352 -> 340 us.
 // Bounds: a chunk moves 64 KB per workgroup in training and 48 KB in inference, 3.4 / 2.5 us
 // at the rate a large copy reaches (4.8 TB/s); measured 4.0 / 3.5 us, VALU issue (~500 per
 // producer wave, ~400 per consumer wave and chunk) and LDS reads (~450 KB) next.  B8 T4096 H16
@@ -122,6 +124,8 @@ __global__ __launch_bounds__(64 * (BV / 16 + 4)) void gla_strip_kernel(SweepPara
   constexpr int PL = C * KP;                 // elements of one plane
   constexpr int LY = BV + 8;
   constexpr bool CK16 = VAR == 1;
+  constexpr bool CK32 = VAR == 0 && !SIN && !DELTA;    // fp32 checkpoints by the producers
+  constexpr bool CKP = CK16 || CK32;
   constexpr bool ST = VAR == 3;
   // producer mapping: a wave covers QW column quads x SW row segments
   constexpr int NQ = KP / 4;
@@ -138,10 +142,12 @@ __global__ __launch_bounds__(64 * (BV / 16 + 4)) void gla_strip_kernel(SweepPara
   __shared__ __attribute__((aligned(16))) uint4 sDt[ST ? 1 : 10 * 64];
   __shared__ __attribute__((aligned(16))) float sE[2 * KP];      // e of this and the next chunk
   __shared__ __attribute__((aligned(16))) float sTot[NRW * KP];  // gate totals per row wave
-  // fp16 checkpoints: the state entering the chunk for the producers to store, fp32 [K][BV];
-  // the delta rule, short of LDS by its w planes, hands it over packed, fp16 [BV][K]
+  // checkpoints: the state entering the chunk for the producers to store, fp32 [K][BV]; the
+  // delta rule, short of LDS by its w planes, hands it over packed, fp16 [BV][K].  (fp32
+  // checkpoints of the delta rule and of fp32 / fp16 inputs, whose planes leave no room, are
+  // stored by the consumers, 4 bytes per lane.)
   constexpr int LS = BV + 4, LC = KP + 8;
-  __shared__ __attribute__((aligned(16))) float sS[CK16 && !DELTA ? KP * LS : 4];
+  __shared__ __attribute__((aligned(16))) float sS[CKP && !DELTA ? KP * LS : 4];
   __shared__ __attribute__((aligned(16))) uint16_t sC[CK16 && DELTA ? BV * LC : 8];
   __shared__ uint32_t sMx[4];                // largest |S| of each wave that takes the maxima
 
@@ -187,6 +193,10 @@ __global__ __launch_bounds__(64 * (BV / 16 + 4)) void gla_strip_kernel(SweepPara
   const int NTs = cdiv(L, C);
   const uint32_t rowK = (uint32_t)(H * LDK), rowV = (uint32_t)(H * V);
   auto cidx = [&](int it) { return REV ? NTs - 1 - it : it; };
+  // fp32 checkpoints: of every chunk or of one parity of the chunk index
+  auto keeps_ckpt = [&](int c) {
+    return VAR == 0 && p.ckpt && (p.ckpt_par == 0 || ((cbase + c) & 1) == p.ckpt_par - 1);
+  };
   auto zbuf = [&](int it) { return sZ + (ZB ? 0 : (it & 1) * (2 * PL)); };   // Z~ of a chunk
 
   // row reads of a swizzled plane: piece 4 kc + lg of row l16 (+ 16 rows per block)
@@ -414,7 +424,7 @@ __global__ __launch_bounds__(64 * (BV / 16 + 4)) void gla_strip_kernel(SweepPara
     // checkpoint of the state entering the chunk: read in interval A (the wave maxima to sMx),
     // stored in B, 8 columns of a row per lane
     constexpr int CU = KP / 32;
-    f32x4 cs[CK16 && !DELTA ? 2 * CU : 1];
+    f32x4 cs[CKP && !DELTA ? 2 * CU : 1];
     auto ckpt_read = [&]() {
       if constexpr (DELTA) return;
 #pragma unroll
@@ -423,7 +433,7 @@ __global__ __launch_bounds__(64 * (BV / 16 + 4)) void gla_strip_kernel(SweepPara
         cs[2 * u] = *(const f32x4*)q;
         cs[2 * u + 1] = *(const f32x4*)(q + 4);
       }
-      state_absmax(cs, sMx, pw, lane);
+      if constexpr (CK16) state_absmax(cs, sMx, pw, lane);
     };
     auto ckpt_store = [&](int c) {
       if constexpr (DELTA) {
@@ -440,8 +450,22 @@ __global__ __launch_bounds__(64 * (BV / 16 + 4)) void gla_strip_kernel(SweepPara
         }
         return;
       }
-      const float sinv = ckpt_tile_scale(sMx);
       const size_t slot = (size_t)(cbase + c) * H + hh;
+      if constexpr (CK32) {
+        const rsrc_t R = make_rsrc(p.ckpt + slot * LDK * V, (long long)K * V * 4);
+#pragma unroll
+        for (int u = 0; u < CU; ++u) {
+          const int row = (ptid >> 3) + 32 * u;
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            const int v = vt * BV + 8 * (ptid & 7) + 4 * e;
+            bst128(R, __builtin_bit_cast(uint4, cs[2 * u + e]),
+                   (row < K && v < V) ? ((uint32_t)row * V + v) * 4u : kOOB, 0);
+          }
+        }
+        return;
+      }
+      const float sinv = ckpt_tile_scale(sMx);
       if (ptid == 0) p.ckpt_scale[slot * p.NV + vt] = 1.f / sinv;   // powers of two
       const rsrc_t R = make_rsrc((uint16_t*)p.ckpt + slot * LDK * V, (long long)K * V * 2);
       const int v = vt * BV + 8 * (ptid & 7);
@@ -496,7 +520,8 @@ __global__ __launch_bounds__(64 * (BV / 16 + 4)) void gla_strip_kernel(SweepPara
         dtiles(std::integral_constant<int, 1>{}, 0, 0, z);
       }
       clk.tick(4);
-      if constexpr (CK16) ckpt_read();
+      const bool ck = CK16 || (CK32 && keeps_ckpt(cidx(it)));
+      if (ck) ckpt_read();
       if constexpr (!FWD_DELTA && !ZB) {
         write_y();
         load_y(it + 1);
@@ -514,8 +539,8 @@ __global__ __launch_bounds__(64 * (BV / 16 + 4)) void gla_strip_kernel(SweepPara
       __syncthreads();
       clk.tick(1);
       // B: X~ (and w) of the next chunk, the cumsum of the one after
-      __builtin_amdgcn_s_setprio(CK16 ? 2 : 0);
-      if constexpr (CK16) ckpt_store(cidx(it));
+      __builtin_amdgcn_s_setprio(CKP ? 2 : 0);
+      if (ck) ckpt_store(cidx(it));
       if constexpr (ZB) {
         stage(rk, REV, true, sZ);
         load_rows(pZ, it + 2, rk);
@@ -604,8 +629,8 @@ __global__ __launch_bounds__(64 * (BV / 16 + 4)) void gla_strip_kernel(SweepPara
             make_uint4(pack_f16x2(a[0] * sinv, a[1] * sinv), pack_f16x2(a[2] * sinv, a[3] * sinv),
                        pack_f16x2(b[0] * sinv, b[1] * sinv), pack_f16x2(b[2] * sinv, b[3] * sinv));
       }
-    } else if constexpr (VAR == 0) {
-      if (!(p.ckpt && (p.ckpt_par == 0 || ((cbase + c) & 1) == p.ckpt_par - 1))) return;
+    } else if constexpr (VAR == 0 && !CK32) {
+      if (!keeps_ckpt(c)) return;
       const rsrc_t R = make_rsrc(p.ckpt + ((size_t)(cbase + c) * H + hh) * LDK * V, (long long)K * V * 4);
 #pragma unroll
       for (int t = 0; t < NT; ++t)
@@ -631,7 +656,8 @@ __global__ __launch_bounds__(64 * (BV / 16 + 4)) void gla_strip_kernel(SweepPara
   auto publish_S = [&]() {                     // for the producers' checkpoint
     if constexpr (CK16 && DELTA) {
       state_absmax(S, sMx, wave, lane);
-    } else if constexpr (CK16) {
+    } else if constexpr (CKP) {
+      if (CK32 && !p.ckpt) return;
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll

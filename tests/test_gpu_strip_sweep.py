@@ -17,6 +17,9 @@ pytestmark = pytest.mark.gpu
 CASES = [(T, K, V, dt) for dt in ("bf16", "f32")
          for T, K, V in ((1, 8, 8), (63, 40, 56), (64, 32, 64), (65, 64, 72), (127, 72, 128),
                          (128, 128, 120), (129, 104, 8), (200, 128, 128))]
+# more than 128 value columns: fp32 checkpoints, of every chunk
+CASES += [(T, K, V, dt) for dt in ("bf16", "f32")
+          for T, K, V in ((65, 40, 144), (129, 128, 208), (200, 72, 256))]
 
 
 @pytest.mark.parametrize("T,K,V,dt", CASES, ids=lambda x: str(x))
