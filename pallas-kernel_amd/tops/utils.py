@@ -1,6 +1,7 @@
 """Host-side helpers mirroring tops/utils.py (varlen chunk maps, ceil-div)."""
 from __future__ import annotations
 
+import heapq
 from collections import OrderedDict
 
 import numpy as np
@@ -231,6 +232,75 @@ class SegPlan:
         `cus` CUs (one state-pass workgroup per CU), at least MIN_PIECE_CHUNKS."""
         return max(-(-state_chunks * wgs_per_piece // max(cus, 1)), MIN_PIECE_CHUNKS)
 
+    @staticmethod
+    def rounds(sizes, slots: int) -> int:
+        """Chunks until the last of ``slots`` workers is done, the longest item first (the order
+        in which the sweeps' workgroups take segments and pieces)."""
+        if len(sizes) <= slots:
+            return max(sizes)
+        sizes = sorted(sizes, reverse=True)
+        load = sizes[slots - 1::-1]
+        for x in sizes[slots:]:
+            heapq.heapreplace(load, load[0] + x)
+        return max(load)
+
+    @staticmethod
+    def _parts(n: int, k: int):
+        """Sizes of n chunks in k near-equal parts."""
+        base, rem = divmod(n, k)
+        return [base + 1] * rem + [base] * (k - rem)
+
+    @classmethod
+    def balance_pieces(cls, handing, sub: int, slots: int) -> int:
+        """Piece length from ``sub`` up that ends the state pass of these segments soonest: at
+        ``sub`` itself the remainders of the cuts can be a second, nearly empty round of
+        workgroups (five packed sequences, T8191 H16: 320 on 256 CUs)."""
+        best = None
+        for x in range(sub, 2 * sub + 1, max(sub // 4, 1)):
+            parts = [y for n in handing for y in cls._parts(n, -(-n // x))]
+            span = cls.rounds(parts, slots)
+            if best is None or span < best[0]:
+                best = span, x
+            if len(parts) <= slots:            # one round: longer pieces only take longer
+                break
+        return best[1]
+
+    @classmethod
+    def balance(cls, chunks, m, slots: int):
+        """Segment counts for the target lengths from that of ``m`` up to twice it, by an
+        estimate of state pass + scan + sweep in units of a sweep's chunk: the rounds of the
+        sweep, 2/3 of those of the state pass (bytes: k, v, g against q, k, v, g, out), and
+        the states written and read again, 32 KB per tile, twice, against 48 KB per chunk.
+        Longer segments often win, since the counts of several sequences round up to more
+        segments than workers and the rest are a second, nearly empty round: five packed
+        sequences, T8191 H16 K=V=128 bf16, forward 122 -> 102 us."""
+        ch, c0 = chunks.tolist(), m.tolist()
+        if len(ch) > 256:                      # (the sweeps order up to 256 sequences)
+            return m
+
+        def cost(c):
+            seg = [cls._parts(n, k) for n, k in zip(ch, c)]
+            flat = [x for s in seg for x in s]
+            hand = sum(sum(s[:-1]) for s in seg)
+            sub = max(-(-hand // slots), MIN_PIECE_CHUNKS) if hand else 0
+            states = len(flat) + (-(-hand // sub) if hand else 0)
+            span = cls.rounds(flat, slots)
+            return span + 2 / 3 * sub + 4 / 3 * states / slots, span
+
+        t0 = max(-(-sum(ch) // slots), MIN_SEG_CHUNKS)
+        best, (low, span) = c0, cost(c0)
+        if span > 1.1 * t0:
+            seen = [c0]
+            for t in range(t0, 2 * t0 + 1, max(t0 // 8, 1)):
+                c = [max(-(-n // t), 1) for n in ch]
+                if c in seen or max(c) <= 1:
+                    continue
+                seen.append(c)
+                e = cost(c)[0]
+                if e < low:
+                    best, low = c, e
+        return np.array(best)
+
     @classmethod
     def build(cls, plan: "ChunkPlan", H: int, V: int):
         cu = plan.cu_host.astype(np.int64)
@@ -246,6 +316,8 @@ class SegPlan:
         m = cls.split_counts(chunks, slots, mode)
         if int(m.max()) <= 1:
             return None
+        if mode is None and slots > 0:
+            m = cls.balance(chunks, m, slots)
         return cls(cu, chunks, m, C, plan.device, per=per, cus=cus)
 
     @staticmethod
@@ -278,6 +350,9 @@ class SegPlan:
         # piece length: one round of state-pass workgroups (pieces = segments when unknown)
         state_chunks = sum(cb[-1] - (cb[-1] - cb[-2]) for cb in seq_bounds if len(cb) > 2)
         sub = self.piece_chunks(state_chunks, per, cus) if per and cus else None
+        if sub and cus >= per:
+            handing = [b - a for cb in seq_bounds for a, b in zip(cb[:-2], cb[1:-1])]
+            sub = self.balance_pieces(handing, sub, cus // per)
 
         def row(n, c):                        # token row of chunk boundary c of sequence n
             return min(int(cu[n]) + C * c, int(cu[n + 1]))
