@@ -1,5 +1,5 @@
 // Internal interfaces of the KDA chunk kernels (kda_prep.hip, kda_wy.hip; the state sweeps
-// are the DELTA instances of gla_sweep.hip).
+// are the DELTA instances of gla_strip.hip).
 #pragma once
 #include <hip/hip_runtime.h>
 

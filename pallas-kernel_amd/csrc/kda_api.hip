@@ -2,7 +2,7 @@
 //
 // Forward (tops_kda_chunk_fwd): the chunk-parallel WY preparation (kda_prep.hip: gate
 // cumsum, Akk, T = (I + Akk)^-1, u, w) and the delta-rule state sweep (the DELTA instance of
-// gla_sweep.hip: v_new = u - w S, o, S per chunk), replacing chunk_kda_fwd's four stages
+// gla_strip.hip: v_new = u - w S, o, S per chunk), replacing chunk_kda_fwd's four stages
 // (tops/ops/kda/chunk.py:25-190).
 //
 // Backward (tops_kda_chunk_bwd): the reverse delta-rule sweep (dv_new, dS per chunk,

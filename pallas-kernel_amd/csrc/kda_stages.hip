@@ -2,7 +2,7 @@
 // (tops/ops/kda/chunk_intra.py:91-281, kda_intra_chunk_fwd) and the delta-rule state pass
 // (tops/ops/common/chunk_delta_h.py:44-166, 898-993, chunk_gated_delta_rule_fwd_h; the
 // oracle tops/cpu/ops/common/chunk_delta_h.py:22-118).  The fused KDA path (kda_prep.hip,
-// the DELTA sweeps of gla_sweep.hip) computes the same quantities without writing them in
+// the DELTA sweeps of gla_strip.hip) computes the same quantities without writing them in
 // these layouts; these kernels serve callers that drive the stages themselves.
 //
 // Arithmetic is fp32 FMA throughout (the reference's fp32 accumulation), one workgroup of

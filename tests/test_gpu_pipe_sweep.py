@@ -1,7 +1,7 @@
-"""The software-pipelined chunk sweep (gla_sweep_pipe.hip) against the serial sweep
+"""The strip-specialised chunk sweep (gla_strip.hip) against the serial sweep
 (gla_sweep.hip) and the float64 oracle.
 
-bf16 chunk_gla calls with per-channel gates run on the pipelined kernel;
+bf16 chunk_gla calls with per-channel gates run on the strip kernel;
 TOPS_SWEEP_SERIAL=1 routes the same calls to the serial kernel.  Both perform the same
 products in the same order, so they may differ only by fp32 contraction (the last bit of an
 fp32 value, one bf16 ulp of a rounded output).  Each case runs forward + backward
@@ -13,7 +13,7 @@ fp32 value, one bf16 ulp of a rounded output).  Each case runs forward + backwar
 Cases cover K of 32 / 64 / 128 (the kernel's three row splits), ragged T, varlen with
 one-token sequences, h0 / dht, and the fp32 and paired checkpoint layouts (empty sequences:
 the oracle rejects them, as tops/cpu does; other modules run them).  The default layout keeps
-fp16 checkpoints, which only the pipelined kernel writes: test_gpu_ckpt16.py covers it.
+fp16 checkpoints, which only the strip kernel writes: test_gpu_ckpt16.py covers it.
 """
 import os
 
