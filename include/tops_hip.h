@@ -63,6 +63,23 @@ int64_t tops_gla_state_bytes(int total_chunks, int H, int K, int V);
 int tops_prepare_chunk_indices(const int32_t* cu_seqlens, int N, int C, int32_t* chunk_offsets,
                                int32_t* chunk_indices, int capacity);
 
+/* Host side of the sequence-parallel split (tops.utils.SegPlan; no counterpart in the
+ * reference, whose sweeps run one program per sequence).  Host pointers, lengths in chunks;
+ * `slots` is the number of sequences, segments or pieces that run at once.
+ *   tops_balance_rounds: chunks until the last of `slots` workers is done with `sizes` [n], the
+ *     longest item first (the order in which the sweeps' workgroups take segments).
+ *   tops_segment_balance: counts [N] (in: a first choice, out: the choice) of segments per
+ *     sequence: the candidate with the lowest estimate of state pass + scan + sweep among the
+ *     first choice and targets from max(ceil(sum / slots), min_seg) up to twice that, tried
+ *     only when the first choice's sweep takes over 1.1 times that target.
+ *   tops_piece_balance: the piece length from `sub` up to twice it that ends the state pass of
+ *     the segments `handing` [n] soonest.
+ * The rounds and the length are returned; a negative TOPS_ERR_* code on bad arguments. */
+int tops_balance_rounds(const int32_t* sizes, int n, int slots);
+int tops_segment_balance(const int32_t* chunks, int32_t* counts, int N, int slots, int min_seg,
+                         int min_piece);
+int tops_piece_balance(const int32_t* handing, int n, int sub, int slots);
+
 /* Chunked GLA forward (C = 64 tiles).
  * Replaces tops.ops.gla.chunk_gla_fwd (tops/ops/gla/chunk.py:1103-1199), i.e. the
  * pallas_calls K1 chunk_cumsum (chunk.py:176), K7 chunk_fwd_h (ops/common/chunk_h.py:243),

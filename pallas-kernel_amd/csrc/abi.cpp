@@ -2,6 +2,10 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
+#include <functional>
+#include <vector>
+
 #include "tops_hip.h"
 
 static thread_local char g_err[512] = "";
@@ -49,4 +53,121 @@ extern "C" int tops_prepare_chunk_indices(const int32_t* cu_seqlens, int N, int 
     chunk_offsets[n + 1] = total;
   }
   return total;
+}
+
+// ---- sequence-parallel split: the search of SegPlan (tops/utils.py) over segment counts and
+// piece lengths.  A call with boundaries not seen before runs it between its arguments and its
+// first launch, up to nine candidates with a sort each: in Python it took 32 us for five
+// sequences on 8 slots and 2.2 ms for 200 on 128, more than the sweep time it saves (20 us at
+// five packed sequences, T8191 H16); here 6.5 and 76 us, of a plan of 0.25 and 1.6 ms.
+namespace {
+
+// Chunks until the last of `slots` workers is done, the longest item first.  Sorts `sizes`.
+int64_t lpt_span(std::vector<int32_t>& sizes, int slots, std::vector<int64_t>& load) {
+  if (sizes.empty()) return 0;
+  if (sizes.size() <= (size_t)slots) return *std::max_element(sizes.begin(), sizes.end());
+  std::sort(sizes.begin(), sizes.end(), std::greater<int32_t>());
+  load.assign(sizes.rend() - slots, sizes.rend());      // ascending: a min-heap as it stands
+  for (size_t i = slots; i < sizes.size(); ++i) {
+    std::pop_heap(load.begin(), load.end(), std::greater<int64_t>());
+    load.back() += sizes[i];
+    std::push_heap(load.begin(), load.end(), std::greater<int64_t>());
+  }
+  return *std::max_element(load.begin(), load.end());
+}
+
+// n chunks in k near-equal parts
+void add_parts(std::vector<int32_t>& out, int n, int k) {
+  const int base = n / k, rem = n % k;
+  for (int i = 0; i < k; ++i) out.push_back(base + (i < rem));
+}
+
+// Chunks of parts of at most about x of every segment, and their number.
+int64_t pieces_span(const int32_t* handing, int n, int x, int slots, std::vector<int32_t>& parts,
+                    std::vector<int64_t>& load) {
+  parts.clear();
+  for (int i = 0; i < n; ++i) add_parts(parts, handing[i], (handing[i] + x - 1) / x);
+  return lpt_span(parts, slots, load);
+}
+
+}  // namespace
+
+extern "C" int tops_balance_rounds(const int32_t* sizes, int n, int slots) {
+  if (!sizes || n <= 0 || slots <= 0)
+    return tops_set_error(TOPS_ERR_NULL, "balance_rounds: bad arguments");
+  try {
+    std::vector<int32_t> s(sizes, sizes + n);
+    std::vector<int64_t> load;
+    return (int)lpt_span(s, slots, load);
+  } catch (...) {
+    return tops_set_error(TOPS_ERR_SHAPE, "balance_rounds: out of memory");
+  }
+}
+
+extern "C" int tops_piece_balance(const int32_t* handing, int n, int sub, int slots) {
+  if (!handing || n <= 0 || sub <= 0 || slots <= 0)
+    return tops_set_error(TOPS_ERR_NULL, "piece_balance: bad arguments");
+  for (int i = 0; i < n; ++i)
+    if (handing[i] <= 0) return tops_set_error(TOPS_ERR_SHAPE, "piece_balance: empty segment");
+  try {
+    std::vector<int32_t> parts;
+    std::vector<int64_t> load;
+    int best = sub;
+    int64_t low = -1;
+    for (int x = sub; x <= 2 * sub; x += std::max(sub / 4, 1)) {
+      const int64_t span = pieces_span(handing, n, x, slots, parts, load);
+      if (low < 0 || span < low) { low = span; best = x; }
+      if (parts.size() <= (size_t)slots) break;   // one round: longer pieces only take longer
+    }
+    return best;
+  } catch (...) {
+    return tops_set_error(TOPS_ERR_SHAPE, "piece_balance: out of memory");
+  }
+}
+
+extern "C" int tops_segment_balance(const int32_t* chunks, int32_t* counts, int N, int slots,
+                                    int min_seg, int min_piece) {
+  if (!chunks || !counts || N <= 0 || slots <= 0 || min_seg <= 0 || min_piece <= 0)
+    return tops_set_error(TOPS_ERR_NULL, "segment_balance: bad arguments");
+  int64_t total = 0;
+  for (int i = 0; i < N; ++i) {
+    if (chunks[i] < 0 || counts[i] <= 0)
+      return tops_set_error(TOPS_ERR_SHAPE, "segment_balance: negative length or no segment");
+    total += chunks[i];
+  }
+  try {
+    std::vector<int32_t> flat, best(counts, counts + N), c(N);
+    std::vector<int64_t> load;
+    std::vector<std::vector<int32_t>> seen{best};
+    int64_t span = 0;
+    auto cost = [&](const std::vector<int32_t>& m) {
+      flat.clear();
+      int64_t hand = 0;
+      for (int i = 0; i < N; ++i) {
+        add_parts(flat, chunks[i], m[i]);
+        hand += chunks[i] - chunks[i] / m[i];     // all parts but the last, a shortest one
+      }
+      const int64_t sub = hand ? std::max<int64_t>((hand + slots - 1) / slots, min_piece) : 0;
+      const int64_t states = (int64_t)flat.size() + (hand ? (hand + sub - 1) / sub : 0);
+      span = lpt_span(flat, slots, load);
+      return (double)span + 2.0 / 3.0 * (double)sub + 4.0 / 3.0 * (double)states / slots;
+    };
+    double low = cost(best);
+    const int64_t t0 = std::max<int64_t>((total + slots - 1) / slots, min_seg);
+    if ((double)span > 1.1 * (double)t0) {
+      for (int64_t t = t0; t <= 2 * t0; t += std::max<int64_t>(t0 / 8, 1)) {
+        for (int i = 0; i < N; ++i) c[i] = (int32_t)std::max<int64_t>((chunks[i] + t - 1) / t, 1);
+        if (*std::max_element(c.begin(), c.end()) <= 1 ||
+            std::find(seen.begin(), seen.end(), c) != seen.end())
+          continue;
+        seen.push_back(c);
+        const double e = cost(c);
+        if (e < low) { low = e; best = c; }
+      }
+    }
+    std::copy(best.begin(), best.end(), counts);
+    return TOPS_OK;
+  } catch (...) {
+    return tops_set_error(TOPS_ERR_SHAPE, "segment_balance: out of memory");
+  }
 }

@@ -48,6 +48,9 @@ SIGNATURES = {
     "tops_kda_fused_recurrent_fwd_decode": [_vp] * 9 + [_i32] * 7 + [_f32, _vp],
     "tops_gla_fused_recurrent_bwd": [_vp] * 17 + [_i32] * 7 + [_f32, _i32, _vp],
     "tops_prepare_chunk_indices": [_vp, _i32, _i32, _vp, _vp, _i32],
+    "tops_balance_rounds": [_vp, _i32, _i32],
+    "tops_segment_balance": [_vp, _vp] + [_i32] * 4,
+    "tops_piece_balance": [_vp, _i32, _i32, _i32],
     "tops_kda_chunk_fwd": [_vp] * 16 + [_i32] * 8 + [_f32, _vp],
     "tops_kda_chunk_bwd": [_vp] * 24 + [_i32] * 8 + [_f32, _vp],
     "tops_kda_chunk_fwd_c16": [_vp] * 17 + [_i32] * 8 + [_f32, _vp],

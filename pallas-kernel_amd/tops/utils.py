@@ -1,7 +1,6 @@
 """Host-side helpers mirroring tops/utils.py (varlen chunk maps, ceil-div)."""
 from __future__ import annotations
 
-import heapq
 from collections import OrderedDict
 
 import numpy as np
@@ -54,11 +53,17 @@ def prepare_chunk_indices(cu_seqlens, chunk_size: int) -> np.ndarray:
     cap = int(cu[-1]) // chunk_size + n
     offs = np.empty(n + 1, np.int32)
     idx = np.empty((max(cap, 1), 2), np.int32)
-    total = N._fn("tops_prepare_chunk_indices")(cu.ctypes.data, n, chunk_size, offs.ctypes.data,
-                                               idx.ctypes.data, cap)
-    if total < 0:
-        raise ValueError(N.lib().tops_last_error().decode())
+    total = _host_call("tops_prepare_chunk_indices", cu.ctypes.data, n, chunk_size,
+                       offs.ctypes.data, idx.ctypes.data, cap)
     return idx[:total].copy()
+
+
+def _host_call(name: str, *args) -> int:
+    """A host routine of the library: its result, an error code raised."""
+    r = N._fn(name)(*args)
+    if r < 0:
+        raise ValueError(N.lib().tops_last_error().decode())
+    return r
 
 
 def _upload(a: np.ndarray, device) -> torch.Tensor:
@@ -236,70 +241,34 @@ class SegPlan:
     def rounds(sizes, slots: int) -> int:
         """Chunks until the last of ``slots`` workers is done, the longest item first (the order
         in which the sweeps' workgroups take segments and pieces)."""
-        if len(sizes) <= slots:
-            return max(sizes)
-        sizes = sorted(sizes, reverse=True)
-        load = sizes[slots - 1::-1]
-        for x in sizes[slots:]:
-            heapq.heapreplace(load, load[0] + x)
-        return max(load)
+        s = np.ascontiguousarray(sizes, np.int32)
+        return _host_call("tops_balance_rounds", s.ctypes.data, len(s), slots)
 
     @staticmethod
-    def _parts(n: int, k: int):
-        """Sizes of n chunks in k near-equal parts."""
-        base, rem = divmod(n, k)
-        return [base + 1] * rem + [base] * (k - rem)
-
-    @classmethod
-    def balance_pieces(cls, handing, sub: int, slots: int) -> int:
+    def balance_pieces(handing, sub: int, slots: int) -> int:
         """Piece length from ``sub`` up that ends the state pass of these segments soonest: at
         ``sub`` itself the remainders of the cuts can be a second, nearly empty round of
         workgroups (five packed sequences, T8191 H16: 320 on 256 CUs)."""
-        best = None
-        for x in range(sub, 2 * sub + 1, max(sub // 4, 1)):
-            parts = [y for n in handing for y in cls._parts(n, -(-n // x))]
-            span = cls.rounds(parts, slots)
-            if best is None or span < best[0]:
-                best = span, x
-            if len(parts) <= slots:            # one round: longer pieces only take longer
-                break
-        return best[1]
+        s = np.ascontiguousarray(handing, np.int32)
+        return _host_call("tops_piece_balance", s.ctypes.data, len(s), sub, slots)
 
-    @classmethod
-    def balance(cls, chunks, m, slots: int):
+    @staticmethod
+    def balance(chunks, m, slots: int):
         """Segment counts for the target lengths from that of ``m`` up to twice it, by an
         estimate of state pass + scan + sweep in units of a sweep's chunk: the rounds of the
         sweep, 2/3 of those of the state pass (bytes: k, v, g against q, k, v, g, out), and
         the states written and read again, 32 KB per tile, twice, against 48 KB per chunk.
         Longer segments often win, since the counts of several sequences round up to more
         segments than workers and the rest are a second, nearly empty round: five packed
-        sequences, T8191 H16 K=V=128 bf16, forward 122 -> 102 us."""
-        ch, c0 = chunks.tolist(), m.tolist()
-        if len(ch) > 256:                      # (the sweeps order up to 256 sequences)
-            return m
-
-        def cost(c):
-            seg = [cls._parts(n, k) for n, k in zip(ch, c)]
-            flat = [x for s in seg for x in s]
-            hand = sum(sum(s[:-1]) for s in seg)
-            sub = max(-(-hand // slots), MIN_PIECE_CHUNKS) if hand else 0
-            states = len(flat) + (-(-hand // sub) if hand else 0)
-            span = cls.rounds(flat, slots)
-            return span + 2 / 3 * sub + 4 / 3 * states / slots, span
-
-        t0 = max(-(-sum(ch) // slots), MIN_SEG_CHUNKS)
-        best, (low, span) = c0, cost(c0)
-        if span > 1.1 * t0:
-            seen = [c0]
-            for t in range(t0, 2 * t0 + 1, max(t0 // 8, 1)):
-                c = [max(-(-n // t), 1) for n in ch]
-                if c in seen or max(c) <= 1:
-                    continue
-                seen.append(c)
-                e = cost(c)[0]
-                if e < low:
-                    best, low = c, e
-        return np.array(best)
+        sequences, T8191 H16 K=V=128 bf16, forward 122 -> 102 us.  The search is native
+        (tops_segment_balance): boundaries are new on most calls of a server or a loader, and
+        it stands before their first launch."""
+        ch = np.ascontiguousarray(chunks, np.int32)
+        c = np.array(m, np.int32)
+        if len(ch) <= 256:                     # (the sweeps order up to 256 sequences)
+            _host_call("tops_segment_balance", ch.ctypes.data, c.ctypes.data, len(ch), slots,
+                       MIN_SEG_CHUNKS, MIN_PIECE_CHUNKS)
+        return c
 
     @classmethod
     def build(cls, plan: "ChunkPlan", H: int, V: int):
