@@ -1,12 +1,17 @@
 """CPU replay of the address arithmetic of the buffer-resource kernels (test infrastructure).
 
-Every global access of gla_sweep_kernel (all instances: GLA / simple-GLA gate modes, the KDA
-delta rule, the state-only pass), gla_dqkg_kernel (bf16 / fp32, fp32 v), kda_prep_kernel,
-kda_wy_kernel / kda_bwd_fused_kernel and fr_decode_kernel is re-evaluated here per workgroup, chunk and thread, with the kernels' own
-thread mappings, masks and (voffset, soffset, width) decomposition.  An access whose voffset
-is kOOB is dropped by the hardware and skipped; every other access must lie entirely inside
-its tensor.  The launches are derived from the host code's own plans (ChunkPlan / SegPlan of
-tops.utils), so the segment path and varlen packing are covered as the ops run them.
+Every global access of gla_strip_kernel (per-channel gates and the KDA delta rule: forward,
+reverse, the state-only pass, 16- to 64-column value tiles), gla_strip_s_kernel (bf16, one gate
+per token), gla_sweep_kernel (the other gate forms, the reverse-time recurrence, value-side
+gates), gla_dqkg_kernel (bf16 / fp32, fp32 v), kda_prep_kernel, kda_wy_kernel /
+kda_bwd_fused_kernel and fr_decode_kernel is re-evaluated here per workgroup, chunk and thread,
+with the kernels' own thread mappings, masks and (voffset, soffset, width) decomposition.  An
+access whose voffset is kOOB is dropped by the hardware and skipped; every other access must lie
+entirely inside its tensor.  The launches are derived from the host code's own plans (ChunkPlan /
+SegPlan of tops.utils), so the segment path and varlen packing are covered as the ops run them.
+The strip kernels leave rows past a chunk's last token, and chunks past the sequence's end, to
+the range of the resource: their model drops what the range drops, rejects an access that
+straddles it, and can count how often each word is read and written.
 
 The model restates the offset expressions of the .hip sources line by line; it cannot prove
 that the kernels compute the same numbers, but it catches a wrong mask, a load wider than its
@@ -28,9 +33,11 @@ class OOBError(AssertionError):
 class Checker:
     """Collects accesses; raises on the first one outside its tensor."""
 
-    def __init__(self, sizes: dict):
+    def __init__(self, sizes: dict, track: bool = False):
         self.sizes = sizes          # tensor name -> bytes
         self.count = 0
+        self.track = track          # keep the accesses for cover()
+        self.log = {}               # (tensor name, "r" / "w") -> [(start words, words)]
 
     def acc(self, name, base, voff, soff, width, what):
         base, voff, soff = (np.asarray(x, np.int64) for x in (base, voff, soff))
@@ -46,6 +53,47 @@ class Checker:
         if bad.any():
             i = int(np.argmax(bad))
             raise OOBError(f"{what}: {name} bytes [{start[i]}, {end[i]}) outside [0, {nb})")
+
+    def racc(self, res, voff, soff, width, what, kind="r"):
+        """An access through a resource (name, base, range): dropped where it starts at or past
+        the range's end, kept otherwise (kind "r" or "w")."""
+        name, base, n = res
+        if n <= 0:
+            return
+        at = np.asarray(voff, np.int64) + soff       # (kOOB plus any soff is past every range)
+        live = at < n
+        if (live & (at + width > n)).any():
+            raise OOBError(f"{what}: an access to {name} straddles the end of its range")
+        self.plain(name, (base + at)[live], width, what, kind)
+
+    def plain(self, name, start, width, what, kind="r"):
+        """Accesses at byte offsets `start` of a tensor."""
+        if start.size == 0:
+            return
+        if start.min() < 0 or start.max() + width > self.sizes[name]:
+            raise OOBError(f"{what}: {name} bytes [{start.min()}, {start.max() + width}) outside "
+                           f"[0, {self.sizes[name]})")
+        self.count += start.size
+        if self.track:
+            assert width % 4 == 0 and not (start % 4).any()
+            self.log.setdefault((name, kind), []).append((start // 4, width // 4))
+
+    def cover(self, name, kind):
+        """How often each 4-byte word of the tensor is read ("r") or written ("w")."""
+        n = -(-self.sizes[name] // 4)
+        d = np.zeros(n + 1, np.int64)
+        for w in (1, 2, 4):
+            at = [s for s, ws in self.log.get((name, kind), ()) if ws == w]
+            if at:
+                at = np.concatenate(at)
+                d += np.bincount(at, minlength=n + 1) - np.bincount(at + w, minlength=n + 1)
+        return np.cumsum(d)[:n]
+
+    def times(self, name, kind, n):
+        """Every word of the tensor read ("r") or written ("w") n times."""
+        cov = self.cover(name, kind)
+        if (cov.min(), cov.max()) != (n, n):
+            raise OOBError(f"{name}: {kind} {cov.min()} to {cov.max()} times, expected {n}")
 
     def rows_rsrc(self, name, e0, nrows, width, es):
         """make_rsrc_rows(t, e0, nrows, width): the range must end inside the tensor."""
@@ -66,13 +114,337 @@ def _kp(K):
     return 32 if K <= 32 else (64 if K <= 64 else 128)
 
 
+# ----------------------------------------------------------- gla_strip_kernel, gla_strip_s_kernel
+def strip_route(gm: int, bf16: bool, gshift: bool = False):
+    """The kernel launch_gla_sweep / launch_gla_state_pass take (csrc/gla_sweep.hip)."""
+    if gm == 0 and not gshift:
+        return "strip"
+    if gm in (1, 2) and bf16 and not gshift:
+        return "strip_s"
+    return "sweep"
+
+
+def delta_tile(H: int, N: int, V: int, ckpt: bool, cus: int = 256) -> int:
+    """Value columns per workgroup of the forward delta rule (launch_gla_strip)."""
+    if ckpt or H * N * (-(-V // 64)) > cus // 2:
+        return 64
+    bv = 16 if H * N * (-(-V // 16)) <= cus else 32
+    return bv if H * N * (-(-V // bv)) <= cus else 64
+
+
+def _walk(p, rev, planted):
+    """(n, NTs, at, cbase) per sequence: at(it) = (c, first row, valid tokens) of step `it`, an
+    empty chunk past the end (planted "lookahead": the walk's index taken as it is)."""
+    cu, seg_end, offs = p.get("cu"), p.get("seg_end"), p.get("offsets")
+    for n in range(p["N"]):
+        if cu is not None:
+            row0 = int(cu[n])
+            L = (int(seg_end[n]) if seg_end is not None else int(cu[n + 1])) - row0
+            cbase = int(offs[n]) if offs is not None else 0
+        else:
+            row0, L, cbase = n * p["T"], p["T"], n * (-(-p["T"] // C))
+        NTs = -(-L // C)
+
+        def at(it, row0=row0, L=L, NTs=NTs):
+            inside = it < NTs
+            c = NTs - 1 - it if rev else it
+            if not inside and planted != "lookahead":
+                return 0, row0, 0
+            return c, row0 + c * C, min(C, L - c * C)
+        yield n, NTs, at, cbase
+
+
+def _chunk_res(name, off, e0, nval, tstride, width, es):
+    """chunk_rsrc(t + off, e0, nval, tstride, width)."""
+    return name, off + e0 * width * es, ((nval - 1) * tstride + width) * es if nval > 0 else 0
+
+
+def _state_io(ck, p, n, hh, s_off, ldk, NT, what):
+    """s0 / s_fin of one sequence, one word per row and lane."""
+    V, so = p["V"], p.get("k0", 0) * p["V"] * 4
+    for nm, kind in (("s0", "r"), ("s_fin", "w")):
+        if p.get(nm):
+            res = (p[nm], so + (n * p["H"] + hh) * ldk * V * 4, ldk * V * 4)
+            for t in range(NT):
+                for r in range(4):
+                    ck.racc(res, s_off(t), r * V * 4, 4, f"{what} {nm}", kind)
+
+
+def strip(ck: Checker, p: dict, es: int, rev: bool, var: int, delta: bool = False, bv: int = 64,
+          bf16: bool | None = None, planted=None):
+    """gla_strip_kernel<TIn, KP, REV, DELTA, VAR, BV> (csrc/gla_strip.hip).  p: B, T, H, K, V, N,
+    cu, seg_end, offsets, tensor names of q, k, g, y, out, s0, s_fin, ckpt, ckpt_scale, dec_fin,
+    u, w, y32, ldk / k0 (a channel slice of rows of ldk channels from channel k0), acc32 and
+    acc_mode, ckpt_par.  planted: "lookahead" (no empty range past the end), "tiles" (a narrow
+    tile launched with the value tiles of 64 columns)."""
+    bf16 = es == 2 if bf16 is None else bf16
+    H, K, V = p["H"], p["K"], p["V"]
+    KP, NC = _kp(K), bv // 16
+    KC, NT = KP // 32, KP // 16
+    NV = -(-V // (64 if planted == "tiles" else bv))
+    ldk, koff = p.get("ldk") or K, p.get("k0", 0)
+    fwd_delta, rev_delta = delta and not rev, delta and rev
+    st, ck32 = var == 3, var == 0 and bf16 and not delta
+    assert bv == 64 or var == 2
+    # producers: column quads x row segments
+    NQ = KP // 4
+    QW = min(NQ, 16)
+    SW = 64 // QW
+    NCW = NQ // QW
+    NRW = 4 // NCW
+    RPT = C // (NRW * SW)
+    ptid, lane, pw = _tid(256)
+    l16, lg = lane & 15, lane >> 4
+    cq = lane % QW + QW * (pw % NCW)
+    rw, sl = pw // NCW, lane // QW
+    r0, c0 = (rw * SW + sl) * RPT, 4 * cq
+    rowK, rowV = H * ldk, H * V
+    offQ = np.where(c0 < K, (r0 * rowK + c0) * es, KOOB)
+    offG = np.where(c0 < K, (r0 * rowK + c0) * 4, KOOB)
+    hh = np.arange(H, dtype=np.int64)[:, None, None]
+    vt = np.arange(NV, dtype=np.int64)[None, :, None]
+    each = 0 * (hh + vt)                        # an access of every (head, value tile)
+    yr, yv = ptid // NC, vt * bv + 16 * (ptid % NC)
+    # consumers
+    ctid, cl, cw = _tid(64 * NC)
+    c16, cg = cl & 15, cl >> 4
+    vcol = vt * bv + 16 * cw + c16
+
+    def s_off(t):
+        ch = 32 * (t >> 1) + 8 * cg + 4 * (t & 1)
+        return np.where((ch < K) & (vcol < V), (ch * V + vcol) * 4, KOOB) + each
+
+    for n, NTs, at, cbase in _walk(p, rev, planted):
+        def chunk(it):
+            c, row, nval = at(it)
+            return c, row * H + hh, nval
+
+        def rows(nm, it, off, width, el):       # load_g, load_rows, load_w
+            _, e0, nval = chunk(it)
+            res = _chunk_res(p[nm], koff * el, e0, nval, rowK, ldk, el)
+            for i in range(RPT):
+                ck.racc(res, off + each, i * rowK * el, width, f"strip load {nm}")
+
+        def load_y(it):
+            _, e0, nval = chunk(it)
+            res = _chunk_res(p["y"], 0, e0, nval, rowV, V, es)
+            for i in range(es):                 # 16 columns in 16-byte pieces
+                v = yv + i * (16 // es)
+                ck.racc(res, np.where((yr < C) & (v < V), (yr * rowV + v) * es, KOOB) + each, 0, 16,
+                        "strip load y")
+
+        def load_u(it):
+            _, e0, nval = chunk(it)
+            res = _chunk_res(p["u"], 0, e0, nval, rowV, V, 4)
+            for R in range(4):
+                for r in range(4):
+                    o = np.where(vcol < V, ((16 * R + 4 * cg + r) * rowV + vcol) * 4, KOOB)
+                    ck.racc(res, o + each, 0, 4, "strip load u")
+
+        def load_g(it):
+            rows("g", it, offG, 16, 4)
+
+        def load_z(it):
+            rows("q" if rev else "k", it, offQ, 4 * es, es)
+
+        def load_x(it):
+            rows("k" if rev else "q", it, offQ, 4 * es, es)
+
+        def load_w(it):
+            rows("w", it, offG, 16, 4)
+
+        _state_io(ck, p, n, hh, s_off, ldk, NT, "strip")
+        for f in (load_g, load_z):
+            f(0)
+            f(1)
+        load_g(2)
+        if not st:
+            load_x(0)
+            load_x(1)
+        if delta:
+            load_w(0)
+        if fwd_delta:
+            load_w(1)
+            load_u(0)
+        else:
+            load_y(0)
+        if rev_delta:
+            load_y(1)
+        for it in range(NTs):
+            if fwd_delta:
+                load_u(it + 1)
+            elif not rev_delta:
+                load_y(it + 1)
+            else:
+                load_w(it + 1)
+                load_y(it + 2)
+            load_z(it + 2)
+            if not st:
+                load_x(it + 2)
+            if fwd_delta:
+                load_w(it + 2)
+            load_g(it + 3)
+            c, e0, nval = chunk(it)
+            if st:
+                continue
+            slot = (cbase + c) * H + hh
+            par = p.get("ckpt_par", 0)
+            if var == 1:
+                res = (p["ckpt"], slot * ldk * V * 2, K * V * 2)
+                ck.plain(p["ckpt_scale"], ((slot * NV + vt) * 4).ravel(), 4, "strip ckpt factor", "w")
+                for u in range(KP // 32):
+                    if delta:
+                        cb, h = (pw * (KP // 32) + u) >> 1, (pw * (KP // 32) + u) & 1
+                        row, v = 16 * cb + l16, vt * bv + 32 * h + 8 * lg
+                    else:
+                        row, v = (ptid >> 3) + 32 * u, vt * bv + 8 * (ptid & 7)
+                    o = np.where((row < K) & (v < V), (row * V + v) * 2, KOOB)
+                    ck.racc(res, o + each, 0, 16, "strip ckpt16", "w")
+            elif var == 0 and p.get("ckpt") and (par == 0 or (cbase + c) % 2 == par - 1):
+                res = (p["ckpt"], koff * V * 4 + slot * ldk * V * 4, K * V * 4)
+                for u in range(KP // 32 if ck32 else 0):
+                    for e in range(2):
+                        row, v = (ptid >> 3) + 32 * u, vt * bv + 8 * (ptid & 7) + 4 * e
+                        o = np.where((row < K) & (v < V), (row * V + v) * 4, KOOB)
+                        ck.racc(res, o + each, 0, 16, "strip ckpt32", "w")
+                for t in range(0 if ck32 else NT):
+                    for r in range(4):
+                        ck.racc(res, s_off(t), r * V * 4, 4, "strip ckpt (consumers)", "w")
+            for R in range(4):
+                if fwd_delta and p.get("y32"):
+                    res = _chunk_res(p["y32"], 0, e0, nval, rowV, V, 4)
+                    for r in range(4):
+                        o = np.where(vcol < V, ((16 * R + 4 * cg + r) * rowV + vcol) * 4, KOOB)
+                        ck.racc(res, o + each, 0, 4, "strip store v_new", "w")
+                if rev_delta:
+                    o = np.where(vcol < V, (vcol * C + 16 * R + 4 * cg) * 4, KOOB)
+                    ck.racc((p["y32"], slot * V * C * 4, V * C * 4), o + each, 0, 16,
+                            "strip store dv_new^T", "w")
+                    continue
+                _store_out(ck, p, e0, nval, vt * bv + 16 * cw + 4 * cg, 16 * R + c16, each, es)
+        if st and p.get("dec_fin"):
+            o = ((n * H + hh) * ldk + c0) * 4 + each
+            sel = (vt == 0) & (rw == 0) & (sl == 0) & (c0 < K) & (each == 0)
+            ck.plain(p["dec_fin"], o[sel], 16, "strip dec_fin", "w")
+
+
+def _store_out(ck, p, e0, nval, v0, tok, each, es):
+    """Four adjacent output columns of one token (and the slices' fp32 sum)."""
+    V = p["V"]
+    el = tok * (p["H"] * V) + v0
+    mode = p.get("acc_mode", 0)
+    if mode:
+        res = _chunk_res(p["acc32"], 0, e0, nval, p["H"] * V, V, 4)
+        o = np.where(v0 < V, el * 4, KOOB) + each
+        if mode in (2, 3):
+            ck.racc(res, o, 0, 16, "strip load acc32")
+        if mode in (1, 2):
+            ck.racc(res, o, 0, 16, "strip store acc32", "w")
+    if mode in (0, 3):
+        res = _chunk_res(p["out"], 0, e0, nval, p["H"] * V, V, es)
+        ck.racc(res, np.where(v0 < V, el * es, KOOB) + each, 0, 4 * es, "strip store out", "w")
+
+
+def strip_s(ck: Checker, p: dict, rev: bool, var: int, planted=None):
+    """gla_strip_s_kernel<KP, REV, VAR> (csrc/gla_strip_s.hip; bf16).  p as strip()'s, gate_mode 1
+    (g [B,T,H]) or 2 (g_gamma [H])."""
+    es, bv = 2, 64
+    H, K, V = p["H"], p["K"], p["V"]
+    KP = _kp(K)
+    NT, NP, PR = KP // 16, KP // 32, KP // 8
+    NV = -(-V // bv)
+    ldk, koff = p.get("ldk") or K, p.get("k0", 0)
+    st = var == 3
+    ptid, lane, pw = _tid(256)
+    l16, lg = lane & 15, lane >> 4
+    rowK, rowV = H * ldk, H * V
+    hh = np.arange(H, dtype=np.int64)[:, None, None]
+    vt = np.arange(NV, dtype=np.int64)[None, :, None]
+    each = 0 * (hh + vt)
+    piece = [ptid + 256 * u for u in range(NP)]
+    go = [np.where(8 * (x % PR) < K, ((x // PR) * rowK + 8 * (x % PR)) * 2, KOOB) for x in piece]
+    yr, yv = ptid >> 2, vt * bv + 16 * (ptid & 3)
+    vcol = vt * bv + 16 * pw + l16              # consumer waves map like the producers' ids
+
+    def s_off(t):
+        ch = 32 * (t >> 1) + 8 * lg + 4 * (t & 1)
+        return np.where((ch < K) & (vcol < V), (ch * V + vcol) * 4, KOOB) + each
+
+    for n, NTs, at, cbase in _walk(p, rev, planted):
+        def chunk(it):
+            c, row, nval = at(it)
+            return c, row * H + hh, nval
+
+        def rows(nm, it):
+            _, e0, nval = chunk(it)
+            res = _chunk_res(p[nm], koff * 2, e0, nval, rowK, ldk, 2)
+            for u in range(NP):
+                ck.racc(res, go[u] + each, 0, 16, f"strip_s load {nm}")
+
+        def load_y(it):
+            _, e0, nval = chunk(it)
+            res = _chunk_res(p["y"], 0, e0, nval, rowV, V, 2)
+            for i in range(2):
+                o = np.where(yv + 8 * i < V, (yr * rowV + yv + 8 * i) * 2, KOOB)
+                ck.racc(res, o + each, 0, 16, "strip_s load y")
+
+        def load_g(it):
+            _, e0, nval = chunk(it)
+            if p["gate_mode"] == 1:
+                res = _chunk_res(p["g"], 0, e0, nval, H, 1, 4)
+                ck.racc(res, np.where(pw == 0, lane * H * 4, KOOB) + each, 0, 4, "strip_s load g")
+
+        def load_z(it):
+            rows("q" if rev else "k", it)
+
+        def load_x(it):
+            rows("k" if rev else "q", it)
+
+        if p["gate_mode"] == 2:
+            ck.plain(p["g"], (hh * 4 + each).ravel(), 4, "strip_s g_gamma")
+        _state_io(ck, p, n, hh, s_off, ldk, NT, "strip_s")
+        for f in (load_g, load_z) + (() if st else (load_x,)):
+            f(0)
+            f(1)
+        load_y(0)
+        for it in range(NTs):
+            load_y(it + 1)
+            load_z(it + 2)
+            load_g(it + 2)
+            if st:
+                continue
+            load_x(it + 2)
+            c, e0, nval = chunk(it)
+            slot = (cbase + c) * H + hh
+            par = p.get("ckpt_par", 0)
+            if var == 1:
+                ck.plain(p["ckpt_scale"], ((slot * NV + vt) * 4).ravel(), 4, "strip_s factor", "w")
+                for u in range(NP):
+                    row, v = (ptid >> 3) + 32 * u, vt * bv + 8 * (ptid & 7)
+                    o = np.where((row < K) & (v < V), (row * V + v) * 2, KOOB)
+                    ck.racc((p["ckpt"], slot * ldk * V * 2, K * V * 2), o + each, 0, 16,
+                            "strip_s ckpt16", "w")
+            elif var == 0 and p.get("ckpt") and (par == 0 or (cbase + c) % 2 == par - 1):
+                for t in range(NT):
+                    for r in range(4):
+                        ck.racc((p["ckpt"], koff * V * 4 + slot * ldk * V * 4, K * V * 4), s_off(t),
+                                r * V * 4, 4, "strip_s ckpt", "w")
+            for R in range(4):
+                _store_out(ck, p, e0, nval, vt * bv + 16 * pw + 4 * lg, 16 * R + l16, each, 2)
+        if st and p.get("dec_fin"):
+            for kr in range(0, K, 64):
+                sel = (vt == 0) & (pw == 0) & (kr + lane < K) & (each == 0)
+                ck.plain(p["dec_fin"], (((n * H + hh) * ldk + kr + lane) * 4 + each)[sel], 4,
+                         "strip_s dec_fin", "w")
+
+
 # --------------------------------------------------------------------------- gla_sweep_kernel
-def sweep(ck: Checker, p: dict, es: int, rev: bool, delta: bool = False, st: bool = False,
-          gate_width_bytes: int = 4, unguarded_prefetch: bool = False, gshift: bool = False,
-          planted_shift: bool = False, gv: bool = False):
-    """gla_sweep_kernel<TIn, KP, REV, DELTA, ST> (csrc/gla_sweep.hip).  p holds the SweepParams
+def sweep(ck: Checker, p: dict, es: int, rev: bool, st: bool = False, gate_width_bytes: int = 4,
+          unguarded_prefetch: bool = False, gshift: bool = False, planted_shift: bool = False,
+          gv: bool = False):
+    """gla_sweep_kernel<TIn, KP, REV, ST> (csrc/gla_sweep.hip).  p holds the SweepParams
     fields: B, T, H, K, V, N, cu (host array or None), seg_end, offsets, gate_mode and which of
-    s0 / s_fin / ckpt / y32 / dec_fin / u / w are bound (tensor names in ck.sizes).  gshift:
+    s0 / s_fin / ckpt / dec_fin are bound (tensor names in ck.sizes).  gshift:
     the reverse sweep reads the gate one token later (tops_chunk_reverse_fwd); planted_shift
     moves the gate rows one token earlier in the sequence's first chunk too (the mistake the
     first-chunk case exists for).  gv: the value-gate forward (tops_gla_chunk_fwd_gv): g is
@@ -88,7 +460,6 @@ def sweep(ck: Checker, p: dict, es: int, rev: bool, delta: bool = False, st: boo
     NCQH = NQ // CQL
     NHT = (KP // 16) * (BV // 16) // 8
     YR = 4
-    fwd_delta, rev_delta = delta and not rev, delta and rev
     gm = p.get("gate_mode", 0)
     rowK, rowV = H * K, H * V
     nrows = B * T * H
@@ -132,7 +503,7 @@ def sweep(ck: Checker, p: dict, es: int, rev: bool, delta: bool = False, st: boo
         else:
             row0, L, cbase = n * T, T, n * (-(-T // C))
         NTs = -(-L // C)
-        gsh = gshift and rev and not delta and not st
+        gsh = gshift and rev and not st
         if gsh and L > 0:
             # the decay of h0 by the last token's gate (plain loads, kr < K checked)
             el = (row0 + L - 1) * H + hh
@@ -192,35 +563,16 @@ def sweep(ck: Checker, p: dict, es: int, rev: bool, delta: bool = False, st: boo
                 elif gw and not gv:
                     ck.acc(p["g"], e0 * gname_w * 4, np.where(ok, offGm, KOOB), i * gstride, gw,
                            f"sweep load g (mode {gm}) chunk {c}")
-            if not fwd_delta:
-                for i in range(YR):
-                    ok = yseg * YR + i < nval
-                    ck.acc(p["y"], e0 * V * es, np.where(ok, offY, KOOB), i * rowV * es, 2 * es,
-                           f"sweep load y chunk {c}")
+            for i in range(YR):
+                ok = yseg * YR + i < nval
+                ck.acc(p["y"], e0 * V * es, np.where(ok, offY, KOOB), i * rowV * es, 2 * es,
+                       f"sweep load y chunk {c}")
             if gv:
                 ck.rows_rsrc(p["g"], e0, nrows, V, 4)
                 for i in range(YR):
                     ok = yseg * YR + i < nval
                     ck.acc(p["g"], e0 * V * 4, np.where(ok, offYg, KOOB), i * rowV * 4, 8,
                            f"sweep load gv chunk {c}")
-            if fwd_delta:
-                trow = 16 * R + l16
-                for kc in range(KP // 32):
-                    k0 = 32 * kc + 8 * lg
-                    o = np.where((trow < nval) & (k0 < K), (trow * rowK + k0) * 4, KOOB)
-                    ck.acc(p["w"], e0 * K * 4, o, 0, 32, "sweep load w (delta fwd)")
-                for j in range(2):
-                    vv = vt * BV + 16 * (2 * nh + j) + l16
-                    for r in range(4):
-                        tok = 16 * R + 4 * lg + r
-                        o = np.where((tok < nval) & (vv < V), (tok * rowV + vv) * 4, KOOB)
-                        ck.acc(p["u"], e0 * V * 4, o, 0, 4, "sweep load u")
-                        if p.get("y32"):
-                            ck.acc(p["y32"], e0 * V * 4, o, 0, 4, "sweep store v_new")
-            if rev_delta:
-                for i in range(RPT):
-                    ck.acc(p["w"], e0 * K * 4, np.where(r0 + i < nval, offG, KOOB), i * rowK * 4,
-                           16, "sweep load w (delta rev)")
             if st:
                 continue
             if p.get("ckpt"):
@@ -233,20 +585,13 @@ def sweep(ck: Checker, p: dict, es: int, rev: bool, delta: bool = False, st: boo
                     for r in range(4):
                         ck.acc(p["ckpt"], cbase_b, np.where(kr + r < K, vo, KOOB), r * V * 4, 4,
                                "sweep store checkpoint")
-            if rev_delta:
-                base = ((cbase + c) * H + hh) * V * C * 4
-                for j in range(2):
-                    vv = vt * BV + 16 * (2 * nh + j) + l16
-                    ck.acc(p["y32"], base, np.where(vv < V, (vv * C + 16 * R + 4 * lg) * 4, KOOB),
-                           0, 16, "sweep store dv_new^T")
-            else:
-                tok = 16 * R + l16
-                oo = np.where(tok < nval, (tok * rowV + vt * BV + 4 * lg) * es, KOOB)
-                for j in range(2):
-                    nn = 2 * nh + j
-                    v0 = vt * BV + 16 * nn + 4 * lg
-                    ck.acc(p["out"], e0 * V * es, np.where(v0 < V, oo, KOOB), 16 * nn * es, 4 * es,
-                           "sweep store out")
+            tok = 16 * R + l16
+            oo = np.where(tok < nval, (tok * rowV + vt * BV + 4 * lg) * es, KOOB)
+            for j in range(2):
+                nn = 2 * nh + j
+                v0 = vt * BV + 16 * nn + 4 * lg
+                ck.acc(p["out"], e0 * V * es, np.where(v0 < V, oo, KOOB), 16 * nn * es, 4 * es,
+                       "sweep store out")
 
 
 # --------------------------------------------------------------------------- gla_dqkg_kernel

@@ -1,8 +1,9 @@
 """CPU check that every buffer access of the chunk kernels stays inside its tensor.
 
 The launches are the ones the ops make (ChunkPlan / SegPlan of tops.utils decide the
-sequence-parallel segments, the state passes and the varlen maps); tests/addr_model.py
-replays each kernel's per-lane offset arithmetic over every workgroup and chunk.  Cases:
+sequence-parallel segments, the state passes and the varlen maps; the sweep kernel follows the
+launchers' rules); tests/addr_model.py replays each kernel's per-lane offset arithmetic over every
+workgroup and chunk.  Cases:
 the shapes of test_gpu_reference_shapes.py, test_gpu_simple_gla.py and test_gpu_kda.py, plus
 empty sequences.  A planted mistake (the 16-byte read of the per-token scalar gate, the read
 that ran 12 bytes past a [B,T,H] gate) must be caught.
@@ -27,6 +28,24 @@ def _np(t):
     return None if t is None else (t.numpy() if isinstance(t, torch.Tensor) else np.asarray(t))
 
 
+def _sweep(ck, p, es, rev, st=False, gate_width_bytes=4):
+    """One sweep launch of the chunk ops: with fp32 checkpoints (p as it is) and, on the strip
+    kernels, with fp16 checkpoints (bf16) and with none."""
+    route = M.strip_route(p["gate_mode"], es == 2)
+    if route == "sweep":
+        M.sweep(ck, p, es, rev, st=st, gate_width_bytes=gate_width_bytes)
+        return
+    run = (lambda q, var: M.strip(ck, q, es, rev, var)) if route == "strip" else \
+        (lambda q, var: M.strip_s(ck, q, rev, var))
+    if st:
+        run(p, 3)
+        return
+    run(p, 0)
+    run(dict(p, ckpt=None), 2)
+    if es == 2:
+        run(dict(p, ckpt=p["ckpt"] + "16", ckpt_scale=p["ckpt"] + "_scale"), 1)
+
+
 def chunk_op(B, T, H, K, V, es, cu=None, gate_mode=0, h0=True, dht=True, gate_width_bytes=4,
              paired=None):
     """Forward + backward launches of chunk_gla (gate_mode 0) / chunk_simple_gla (1: g [B,T,H],
@@ -42,6 +61,8 @@ def chunk_op(B, T, H, K, V, es, cu=None, gate_mode=0, h0=True, dht=True, gate_wi
                  g={0: B * T * H * K * 4, 1: B * T * H * 4, 2: H * 4, 3: H * K * 4}[gate_mode],
                  dg={0: B * T * H * K * 4, 1: B * T * H * 4, 2: 0, 3: B * T * H * K * 4}[gate_mode],
                  hs=plan.total * H * K * V * 4, dhs=plan.total * H * K * V * 4,
+                 hs16=plan.total * H * K * V * 2, dhs16=plan.total * H * K * V * 2,
+                 hs_scale=plan.total * H * -(-V // 64) * 4, dhs_scale=plan.total * H * -(-V // 64) * 4,
                  h0=N * H * K * V * 4, ht=N * H * K * V * 4, dht=N * H * K * V * 4, dh0=N * H * K * V * 4)
     ck = M.Checker(sizes)
     base = dict(H=H, K=K, V=V, gate_mode=gate_mode, g="g")
@@ -54,19 +75,19 @@ def chunk_op(B, T, H, K, V, es, cu=None, gate_mode=0, h0=True, dht=True, gate_wi
                      offsets=_np(plan.offsets_dev), q="q", k="k", y=y,
                      out="dv" if rev else "o", ckpt="dhs" if rev else "hs",
                      s0=s_in if (dht if rev else h0) else None, s_fin=s_out)
-            M.sweep(ck, p, es, rev, gate_width_bytes=gate_width_bytes)
+            _sweep(ck, p, es, rev, gate_width_bytes=gate_width_bytes)
             continue
         pc = sp.rev if rev else sp.fwd
         if pc.n:
             ck.sizes.update(s_loc=pc.n * H * K * V * 4, dec=pc.n * H * K * 4)
             p = dict(base, B=1, T=B * T, N=pc.n, cu=pc.start, seg_end=pc.end, q=z, k=z, y=y,
                      s_fin="s_loc", dec_fin="dec")
-            M.sweep(ck, p, es, rev, st=True, gate_width_bytes=gate_width_bytes)
+            _sweep(ck, p, es, rev, st=True, gate_width_bytes=gate_width_bytes)
         ck.sizes.update(init=sp.Nv * H * K * V * 4, fin=sp.Nv * H * K * V * 4)
         p = dict(base, B=1, T=B * T, N=sp.Nv, cu=sp.cu_host, offsets=_np(sp.offsets_dev),
                  q="q", k="k", y=y, out="dv" if rev else "o", ckpt="dhs" if rev else "hs",
                  s0="init", s_fin="fin")
-        M.sweep(ck, p, es, rev, gate_width_bytes=gate_width_bytes)
+        _sweep(ck, p, es, rev, gate_width_bytes=gate_width_bytes)
     p = dict(base, B=B, T=T, total=plan.total, cu=plan.cu_host if plan.varlen else None,
              offsets=_np(plan.offsets_dev), chunk_map=_np(plan.chunk_map_dev),
              q="q", k="k", v="v", do="do", hs="hs", dhs="dhs", dq="dq", dk="dk",
@@ -94,9 +115,17 @@ def kda_op(B, T, H, K, V, es, cu=None, h0=True):
     M.kda_prep(ck, dict(vl, H=H, K=K, V=V, B=B, T=T, total=tot, k="k", g="g", v="v", beta="beta",
                         u="u", w="w", tt="tt"), es)
     sw = dict(vl, B=B, T=T, H=H, K=K, V=V, N=N, gate_mode=0, q="q", k="k", g="g", w="w")
-    M.sweep(ck, dict(sw, u="u", y32="vnew", out="o", ckpt="hs", s0="h0" if h0 else None, s_fin="ht"),
-            es, rev=False, delta=True)
-    M.sweep(ck, dict(sw, y="do", y32="dvnt", ckpt="dhs", s0="dht", s_fin="dh0"), es, rev=True, delta=True)
+    # fp32 checkpoints and (bf16) fp16 ones; without checkpoints the forward's value tile narrows
+    ck.sizes.update(hs16=tot * H * K * V * 2, dhs16=tot * H * K * V * 2,
+                    hs_scale=tot * H * -(-V // 64) * 4, dhs_scale=tot * H * -(-V // 64) * 4)
+    fw = dict(sw, u="u", out="o", s0="h0" if h0 else None, s_fin="ht")
+    bw = dict(sw, y="do", y32="dvnt", s0="dht", s_fin="dh0")
+    M.strip(ck, fw, es, False, 2, delta=True, bv=M.delta_tile(H, N, V, False))
+    for rev, q in ((False, dict(fw, y32="vnew")), (True, bw)):
+        nm = "dhs" if rev else "hs"
+        M.strip(ck, dict(q, ckpt=nm), es, rev, 0, delta=True)
+        if es == 2:
+            M.strip(ck, dict(q, ckpt=nm + "16", ckpt_scale=nm + "_scale"), es, rev, 1, delta=True)
     # bf16: the WY backward and dq / dk / dg run as one kernel (kda_bwd_fused.hip)
     fused = es == 2
     M.kda_wy(ck, dict(vl, H=H, K=K, V=V, B=B, T=T, total=tot, k="k", g="g", v="v", beta="beta",
@@ -196,12 +225,129 @@ def test_empty_sequences_in_bounds(cu):
 def test_planted_unguarded_empty_prefetch_is_caught():
     """Prefetching chunk cidx(0) = -1 of an empty first sequence reads before the tensor."""
     plan = U.ChunkPlan(1, 64, [0, 0, 64], "cpu")
-    ck = M.Checker(dict(q=64 * 2 * 32 * 2, k=64 * 2 * 32 * 2, g=64 * 2 * 32 * 4, do=64 * 2 * 32 * 2))
+    ck = M.Checker(dict(q=64 * 2 * 32 * 4, k=64 * 2 * 32 * 4, g=64 * 2 * 4, do=64 * 2 * 32 * 4))
     p = dict(B=1, T=64, H=2, K=32, V=32, N=2, cu=plan.cu_host, offsets=_np(plan.offsets_dev),
-             gate_mode=0, g="g", q="q", k="k", y="do")
-    M.sweep(ck, p, 2, rev=True, st=True)
+             gate_mode=1, g="g", q="q", k="k", y="do")
+    assert M.strip_route(1, bf16=False) == "sweep"
+    M.sweep(ck, p, 4, rev=True, st=True)
     with pytest.raises(M.OOBError):
-        M.sweep(ck, p, 2, rev=True, st=True, unguarded_prefetch=True)
+        M.sweep(ck, p, 4, rev=True, st=True, unguarded_prefetch=True)
+
+
+# The strip kernels: every element of every tensor read and written as often as the launch means
+# it to be.  Channel remainders of the 32 / 64 / 128 instances, value remainders of every tile
+# width, lengths around one and two chunks, packed sequences with empty ones.
+STRIP = [dict(B=2, T=1, H=1, K=8, V=8), dict(B=2, T=63, H=2, K=40, V=56),
+         dict(B=1, T=64, H=2, K=32, V=64), dict(B=2, T=65, H=2, K=64, V=72),
+         dict(B=1, T=129, H=3, K=104, V=8), dict(B=1, T=200, H=2, K=128, V=128),
+         dict(B=1, T=150, H=2, K=72, V=120, cu=[0, 0, 13, 13, 64, 65, 150, 150])]
+# (variant, element bytes, bf16): fp32 and paired checkpoints in all three types, fp16
+# checkpoints, none, the state pass
+FORMS = [(0, 2, True), (0, 4, False), (0, 2, False), ("paired", 2, True), (1, 2, True),
+         (2, 2, True), (2, 4, False), (3, 2, True), (3, 4, False)]
+
+
+def strip_launch(c, form, rev, gate="k", delta=False, bv=64, slices=1, planted=None):
+    """One strip launch (per slice of the channels) over fresh tensors, and what it has to touch."""
+    var, es, bf16 = form
+    B, T, H, K, V = (c[x] for x in "BTHKV")
+    plan = U.ChunkPlan(B, T, c.get("cu"), "cpu")
+    N, tot, rows, NV = plan.N, plan.total, B * T * H, -(-V // bv)
+    paired, var = var == "paired", 0 if var == "paired" else var
+    KS = K * slices                              # the tensors' channels
+    sizes = dict(q=rows * KS * es, k=rows * KS * es, y=rows * V * es, out=rows * V * es,
+                 acc32=rows * V * 4, s0=N * H * KS * V * 4, s_fin=N * H * KS * V * 4,
+                 u=rows * V * 4, w=rows * K * 4, dec_fin=N * H * KS * 4,
+                 g={"k": rows * KS * 4, "s": rows * 4, "gamma": H * 4}[gate],
+                 y32=tot * H * V * C * 4 if rev else rows * V * 4,
+                 ckpt=tot * H * KS * V * (2 if var == 1 else 4), ckpt_scale=tot * H * NV * 4)
+    ck = M.Checker(sizes, track=True)
+    p = dict(B=B, T=T, H=H, K=K, V=V, N=N, cu=plan.cu_host if plan.varlen else None,
+             offsets=_np(plan.offsets_dev), gate_mode={"k": 0, "s": 1, "gamma": 2}[gate], q="q",
+             k="k", g="g", y="y", out="out", s0="s0", s_fin="s_fin", dec_fin="dec_fin", u="u", w="w",
+             y32="y32" if delta else None, ckpt="ckpt" if var in (0, 1) else None,
+             ckpt_scale="ckpt_scale", ckpt_par=(2 if rev else 1) if paired else 0)
+    for a in range(slices):
+        if slices > 1:
+            p.update(ldk=KS, k0=a * K, acc32="acc32", acc_mode=1 if a == 0 else 3 if a == slices - 1 else 2)
+        if gate == "k":
+            M.strip(ck, p, es, rev, var, delta=delta, bv=bv, bf16=bf16, planted=planted)
+        else:
+            M.strip_s(ck, p, rev, var, planted=planted)
+    ck.times("k" if rev and var == 3 else "q", "r", 0 if var == 3 else NV)   # X~
+    ck.times("q" if rev and var == 3 else "k", "r", NV)                      # Z~
+    if gate == "k" or slices == 1 and gate == "s":
+        ck.times("g", "r", NV)
+    if delta and not rev:
+        ck.times("u", "r", 1)
+    else:
+        ck.times("y", "r", slices)
+    if delta:
+        ck.times("w", "r", NV)
+        ck.times("y32", "w", 1)
+    ck.times("s0", "r", 1)
+    ck.times("s_fin", "w", 1)
+    if var == 3:
+        ck.times("dec_fin", "w", 1)
+    elif not (delta and rev):
+        ck.times("out", "w", 1)
+        if slices > 1:
+            ck.times("acc32", "w", slices - 1)
+            ck.times("acc32", "r", slices - 1)
+    if paired:
+        got = ck.cover("ckpt", "w").reshape(tot, -1)
+        assert all((row == (i % 2 == (1 if rev else 0))).all() for i, row in enumerate(got))
+    elif var in (0, 1):
+        ck.times("ckpt", "w", 1)
+        if var == 1:
+            ck.times("ckpt_scale", "w", 1)
+    return ck
+
+
+_cid = lambda c: "B{B}-T{T}-H{H}-K{K}-V{V}".format(**c)    # noqa: E731
+
+
+@pytest.mark.parametrize("rev", [False, True], ids=["fwd", "rev"])
+@pytest.mark.parametrize("c", STRIP, ids=_cid)
+def test_strip_accesses(c, rev):
+    for form in FORMS:
+        strip_launch(c, form, rev)
+    for form in ((0, 2, True), (0, 4, False), (0, 2, False)):
+        strip_launch(c, form, rev, slices=2)
+        strip_launch(c, form, rev, slices=3)
+
+
+@pytest.mark.parametrize("rev", [False, True], ids=["fwd", "rev"])
+@pytest.mark.parametrize("c", STRIP, ids=_cid)
+def test_strip_token_gate_accesses(c, rev):
+    for gate in ("s", "gamma"):
+        for form in ((0, 2, True), ("paired", 2, True), (1, 2, True), (2, 2, True), (3, 2, True)):
+            strip_launch(c, form, rev, gate=gate)
+        strip_launch(c, (0, 2, True), rev, gate=gate, slices=2)
+
+
+@pytest.mark.parametrize("rev", [False, True], ids=["fwd", "rev"])
+@pytest.mark.parametrize("c", STRIP, ids=_cid)
+def test_strip_delta_rule_accesses(c, rev):
+    for form in ((0, 2, True), (0, 4, False), (1, 2, True)):
+        strip_launch(c, form, rev, delta=True)
+    if not rev:
+        for es in (2, 4):
+            for bv in (16, 32, 64):
+                strip_launch(c, (2, es, es == 2), False, delta=True, bv=bv)
+
+
+def test_planted_strip_mistakes_are_caught():
+    """Loads a chunk past the end of a reverse walk run before the tensor; a narrow tile launched
+    with the 64-column tile count leaves columns out."""
+    c = dict(B=1, T=100, H=2, K=32, V=72)
+    for gate in ("k", "s"):
+        with pytest.raises(M.OOBError, match="outside"):
+            strip_launch(c, (2, 2, True), True, gate=gate, planted="lookahead")
+    with pytest.raises(M.OOBError, match="times, expected"):
+        strip_launch(c, (2, 2, True), False, delta=True, bv=16, planted="tiles")
+    with pytest.raises(M.OOBError, match="straddles"):
+        strip_launch(dict(c, V=76), (2, 2, True), False)     # V % 8: refused by the entry points
 
 
 def test_planted_paired_partner_past_end_is_caught():
