@@ -302,29 +302,31 @@ class SegPlan:
         return out
 
     def __init__(self, cu, chunks, m, C, device, per=None, cus=None):
-        coff = np.concatenate([[0], np.cumsum(chunks)])
+        # (plain ints: a NumPy scalar per element made this loop a third of the plan)
+        coff = np.concatenate([[0], np.cumsum(chunks)]).tolist()
+        cu = cu.tolist()
         starts, offs, seg_first = [], [], [0]
         seq_bounds = []                       # per sequence: segment boundaries in chunks
-        for n in range(len(chunks)):
-            base, rem = divmod(int(chunks[n]), int(m[n]))
-            sizes = [base + (1 if j < rem else 0) for j in range(int(m[n]))]
+        for n, (size, k) in enumerate(zip(chunks.tolist(), m.tolist())):
+            base, rem = divmod(size, k)
+            sizes = [base + (1 if j < rem else 0) for j in range(k)]
             cb = [0]
             for sz in sizes:
                 cb.append(cb[-1] + sz)
             seq_bounds.append(cb)
             for j in range(len(sizes)):
-                starts.append(int(cu[n]) + C * cb[j])
-                offs.append(int(coff[n]) + cb[j])
+                starts.append(cu[n] + C * cb[j])
+                offs.append(coff[n] + cb[j])
             seg_first.append(seg_first[-1] + len(sizes))
         # piece length: one round of state-pass workgroups (pieces = segments when unknown)
         state_chunks = sum(cb[-1] - (cb[-1] - cb[-2]) for cb in seq_bounds if len(cb) > 2)
         sub = self.piece_chunks(state_chunks, per, cus) if per and cus else None
         if sub and cus >= per:
-            handing = [b - a for cb in seq_bounds for a, b in zip(cb[:-2], cb[1:-1])]
+            handing = [b - a for cb in seq_bounds if len(cb) > 2 for a, b in zip(cb[:-2], cb[1:-1])]
             sub = self.balance_pieces(handing, sub, cus // per)
 
         def row(n, c):                        # token row of chunk boundary c of sequence n
-            return min(int(cu[n]) + C * c, int(cu[n + 1]))
+            return min(cu[n] + C * c, cu[n + 1])
 
         fwd = ([], [], [0], [])
         rev = ([], [], [0], [])
@@ -352,8 +354,8 @@ class SegPlan:
         self.fwd = self.Pieces(*fwd)
         self.rev = self.Pieces(*rev)
         self.Nv = len(starts)
-        cu_v = np.array(starts + [int(cu[-1])], np.int32)
-        offs_v = np.array(offs + [int(coff[-1])], np.int32)
+        cu_v = np.array(starts + [cu[-1]], np.int32)
+        offs_v = np.array(offs + [coff[-1]], np.int32)
         sf = np.array(seg_first, np.int32)
         self.seg_first = sf
         self.cu_host = cu_v

@@ -95,7 +95,7 @@ def test_native_search_rejects_bad_arguments():
 @pytest.mark.parametrize("n,T,H,V", [(16, 16384, 4, 128), (200, 65536, 2, 64), (100, 131072, 2, 128)])
 def test_search_is_a_small_share_of_the_plan(n, T, H, V, monkeypatch):
     """Boundaries are new on most calls of a loader or a server: the search may take a fifth of
-    the plan's time (measured 2 to 5 %; 14 to 42 % when it ran in Python)."""
+    the plan's time (measured 1 to 5 %; 14 to 42 % when it ran in Python)."""
     monkeypatch.setattr(U, "_device_cus", lambda device: 256)
     rng = np.random.default_rng(n)
     cu = np.array([0] + sorted(rng.choice(np.arange(1, T), n - 1, replace=False).tolist()) + [T])
