@@ -51,6 +51,7 @@
 // the default priority in interval A.
 #include <stdlib.h>
 
+#include <atomic>
 #include <type_traits>
 
 #include "gla_sweep.h"
@@ -921,6 +922,21 @@ bool gla_strip_eligible(const SweepParams& p) {
   return !(e && e[0] == '1');
 }
 
+// Compute units of the current device (kept per device; 256 where it cannot be asked).
+static int device_cus() {
+  static std::atomic<int> known[64];
+  int dev = 0, n = 0;
+  if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64 &&
+      (n = known[dev].load(std::memory_order_relaxed)) > 0)
+    return n;
+  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) {
+    (void)hipGetLastError();
+    return 256;
+  }
+  if (dev >= 0 && dev < 64) known[dev].store(n, std::memory_order_relaxed);
+  return n;
+}
+
 template <typename TIn, bool REV, bool DELTA>
 hipError_t launch_gla_strip(const SweepParams& p, hipStream_t s) {
   const int kp = p.K <= 32 ? 32 : (p.K <= 64 ? 64 : 128);
@@ -930,14 +946,17 @@ hipError_t launch_gla_strip(const SweepParams& p, hipStream_t s) {
   dim3 grid(p.NV * p.H * p.N);
   if constexpr (DELTA && !REV) {
     // Few heads and sequences leave CUs idle and the sweep is one long chain: the narrowest
-    // value tile whose workgroups are still one round on the chip's 256 CUs (B1 T5000 H32
-    // K=V=128 fp32: 64 columns 367 us, 32 columns 302, 16 columns 289, the staging repeated
-    // but each consumer alone with its LDS reads; the per-channel-gate sweeps, whose
-    // consumers share the D tiles, gain nothing: 27 us at B1 T512 H4 against 30)
-    constexpr long long kCus = 256;
+    // value tile whose workgroups are still one round on the device's CUs, the staging repeated
+    // but each consumer alone with its LDS reads.  chunk_kda forward without checkpoints, B1
+    // T2048 K=V=128 bf16 by heads, tiles of 16 / 32 / 64 columns: H4 137 / 142 / 161 us, H32
+    // (256 workgroups of 16) 165 / 170 / 187, H33 294 / 180 / 200, H64 (256 of 32) 324 / 213 /
+    // 231, H65 463 / 347 / 245; fp32 and K, V of 64 order the same way on the same lines.  (The
+    // per-channel-gate sweeps, whose consumers share the D tiles, gain nothing: 27 us at B1 T512
+    // H4 against 30.)
+    const long long cus = device_cus();
     const long long wgs = (long long)p.H * p.N;
-    const int bv = (var != 2 || wgs * p.NV > kCus / 2) ? 64 : (wgs * ((p.V + 15) / 16) <= kCus ? 16 : 32);
-    if (bv < 64 && wgs * ((p.V + bv - 1) / bv) <= kCus) {
+    const int bv = (var != 2 || wgs * p.NV > cus / 2) ? 64 : (wgs * ((p.V + 15) / 16) <= cus ? 16 : 32);
+    if (bv < 64 && wgs * ((p.V + bv - 1) / bv) <= cus) {
       SweepParams q = p;
       q.NV = (p.V + bv - 1) / bv;
       const dim3 gn((unsigned)(q.NV * wgs)), bn(64 * (bv / 16 + 4));

@@ -143,32 +143,59 @@ def test_strip_sweep_token_gate_tile_edges(T, K, V, gate, cuda_device):
         assert err <= 1e-3 * scale, f"dg: {err / scale:.3e} of its terms"
 
 
-@pytest.mark.parametrize("B,H,V,dt", [(1, 2, 128, "bf16"), (1, 2, 8, "f32"), (1, 20, 128, "bf16"),
-                                      (1, 40, 72, "f32"), (2, 33, 128, "bf16")],
-                         ids=lambda x: str(x))
-def test_strip_sweep_delta_rule_narrow_tiles(B, H, V, dt, cuda_device):
+# (B, H, K, V, dtype, packed boundaries), the tile the call takes, the factor of the heads whose
+# call takes the tile after it (on 256 CUs)
+NARROW = [((1, 2, 64, 128, "bf16", None), 16, (20, 32)), ((1, 2, 64, 8, "f32", None), 16, (65, 64)),
+          ((1, 20, 64, 128, "bf16", None), 16, (2, 32)), ((1, 40, 64, 72, "f32", None), 16, (2, 64)),
+          ((2, 33, 64, 128, "bf16", None), 64, None),
+          ((2, 17, 128, 128, "bf16", None), 32, (2, 64)), ((2, 32, 32, 128, "f32", None), 32, (2, 64)),
+          ((1, 65, 64, 64, "bf16", None), 32, (2, 64)), ((1, 40, 128, 120, "f32", None), 32, (2, 64)),
+          ((1, 40, 32, 104, "bf16", None), 32, (2, 64)),
+          ((1, 12, 64, 128, "bf16", [0, 1, 65, 130]), 32, (2, 64)),
+          ((1, 12, 128, 72, "f32", [0, 64, 127, 130]), 16, (2, 64))]
+
+
+@pytest.mark.parametrize("shape,bv,wider", NARROW, ids=lambda x: str(x))
+def test_strip_sweep_delta_rule_narrow_tiles(shape, bv, wider, cuda_device):
     """The forward delta rule without checkpoints takes 16- or 32-column tiles while their
-    workgroups are one round on the chip.  Both sides of the rule's lines (20 heads of 128
-    columns: 160 workgroups of 16 columns; 40 of 72: 200; 66 heads: 64-column tiles) within
-    the bounds of the oracle, and the same up to fp32 rounding as those heads in a call of four
-    times as many, which takes wider tiles."""
+    workgroups are one round on the chip.  Every width, at the edges of the rule and with channel
+    and value remainders, within the bounds of the oracle, and the same up to fp32 rounding as
+    those heads in a call of more, which takes the next tile.  The widths are those of the
+    launcher's rule, restated in addr_model.delta_tile."""
     import numpy as np
+    from addr_model import delta_tile
     from oracle import kda as OK
     from _inputs import kda_inputs
     from tops.ops.kda import chunk_kda
+    B, H, K, V, dt, cu = shape
+    N = len(cu) - 1 if cu else B
+    cus = torch.cuda.get_device_properties(cuda_device).multi_processor_count
+    if cus == 256:
+        assert delta_tile(H, N, V, False) == bv
+        assert wider is None or delta_tile(H * wider[0], N, V, False) == wider[1]
     dtype = {"bf16": torch.bfloat16, "f32": torch.float32}[dt]
-    T, K = 130, 64
-    d = kda_inputs(B, T, H, K, V, 40 + H, gate_div=4.0, h0=True)
+    T = 130
+    d = kda_inputs(B, T, H, K, V, 40 + H, gate_div=4.0, h0=True, N=N)
     x = [to_dev(d[n], dtype, cuda_device) for n in "qkv"] + \
         [to_dev(d[n], torch.float32, cuda_device) for n in ("g", "beta")]
     h0 = to_dev(d["h0"], torch.float32, cuda_device)
-    print(f"narrow tiles B={B} H={H} V={V} {dt}", flush=True)
-    o, ht = chunk_kda(*x, initial_state=h0, output_final_state=True)
-    ro, rht = OK.chunk_kda(*(seen(d[n], dtype) for n in "qkv"), np.float64(d["g"]),
-                           np.float64(d["beta"]), K ** -0.5, np.float64(d["h0"]), True)
+    print(f"narrow tiles {shape} bv={bv}", flush=True)
+    o, ht = chunk_kda(*x, initial_state=h0, output_final_state=True, cu_seqlens=cu)
+    ins = [seen(d[n], dtype) for n in "qkv"] + [np.float64(d[n]) for n in ("g", "beta")]
+    h64 = np.float64(d["h0"])
+    if cu is None:
+        ro, rht = OK.chunk_kda(*ins, K ** -0.5, h64, True)
+    else:                                      # the oracle takes one sequence length
+        parts = [OK.chunk_kda(*(t[:, lo:hi] for t in ins), K ** -0.5, h64[n:n + 1], True)
+                 for n, (lo, hi) in enumerate(zip(cu, cu[1:]))]
+        ro, rht = (np.concatenate(t, axis) for t, axis in zip(zip(*parts), (1, 0)))
     for n, got, ref in (("o", o, ro), ("ht", ht, rht)):
         e, lim = rel(host(got), ref), out_bound(ref, dtype, got.dtype)
         assert e < lim, f"{n}: rel-err {e:.3e} vs oracle (bound {lim:.2e})"
-    rep = [torch.cat([t] * 4, 2).contiguous() for t in x]      # four times the heads: wider tiles
-    o4, ht4 = chunk_kda(*rep, initial_state=torch.cat([h0] * 4, 1), output_final_state=True)
-    assert rel(host(o4[:, :, :H]), host(o)) <= 1e-3 and rel(host(ht4[:, :H]), host(ht)) <= 1e-5
+    if wider is None:
+        return
+    rep = [torch.cat([t] * wider[0], 2).contiguous() for t in x]
+    ow, htw = chunk_kda(*rep, initial_state=torch.cat([h0] * wider[0], 1), output_final_state=True,
+                        cu_seqlens=cu)
+    # fp32 sums in the same order: the last bit of a state, one ulp of a rounded output
+    assert rel(host(ow[:, :, :H]), host(o)) <= 1e-3 and rel(host(htw[:, :H]), host(ht)) <= 1e-5
