@@ -284,8 +284,11 @@ __global__ __launch_bounds__(64 * (BV / 16 + 4)) void gla_strip_kernel(SweepPara
       }
     };
 
-    // gate cumsum of the raw chunk (natural-log units): thread rows, the wave's row segments
-    // on the VALU, the wave totals to sTot
+    // gate cumsum of the raw chunk: thread rows, the wave's row segments on the VALU, the wave
+    // totals to sTot.  In log2 units, as the kernels before and after the sweep sum it: in
+    // natural units, scaled where the exponents are formed, the final state of chunk_gla was
+    // 4.79e-6 off instead of 4.06e-6 and KDA's dbeta 7.5e-6 instead of 6.7e-6 at gates of -1.6 a
+    // token (times unchanged; one long KDA chain, B1 T5000 H32, 536.0 -> 537.5 us)
     float G[RPT][4], pre[4];
     auto cumsum = [&]() {
       float tot[4];
@@ -294,7 +297,7 @@ __global__ __launch_bounds__(64 * (BV / 16 + 4)) void gla_strip_kernel(SweepPara
         float x[4];
         unpack4(rg[i], x);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) G[i][j] = x[j] + (i > 0 ? G[i - 1][j] : 0.f);
+        for (int j = 0; j < 4; ++j) G[i][j] = x[j] * kLog2e + (i > 0 ? G[i - 1][j] : 0.f);
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -315,7 +318,7 @@ __global__ __launch_bounds__(64 * (BV / 16 + 4)) void gla_strip_kernel(SweepPara
       }
       if (sl == 0) *(float4*)(sTot + rw * KP + c0) = make_float4(tot[0], tot[1], tot[2], tot[3]);
     };
-    // pm: x = G log2 e + pm is the exponent G - Gm of a row; gm2 = Gm (log2 units)
+    // pm: x = G + pm is the exponent G - Gm of a row; gm2 = Gm
     float pm[4], gm2[4], dsum[4] = {0.f, 0.f, 0.f, 0.f};
     auto sums = [&](int buf) {
       float gam[4] = {0.f, 0.f, 0.f, 0.f};
@@ -327,9 +330,9 @@ __global__ __launch_bounds__(64 * (BV / 16 + 4)) void gla_strip_kernel(SweepPara
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        gm2[j] = 0.5f * kLog2e * gam[j];
+        gm2[j] = 0.5f * gam[j];
         if constexpr (ST) dsum[j] += 2.f * gm2[j];   // (a chunk past the sequence adds zero)
-        pm[j] = pre[j] * kLog2e - gm2[j];
+        pm[j] = pre[j] - gm2[j];
       }
       if (rw == 0 && sl == 0)
         *(float4*)(sE + buf * KP + c0) =
@@ -351,7 +354,7 @@ __global__ __launch_bounds__(64 * (BV / 16 + 4)) void gla_strip_kernel(SweepPara
         unpack4(raw[i], v);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          if (first) G[i][j] = __builtin_fmaf(G[i][j], kLog2e, pm[j]);
+          if (first) G[i][j] += pm[j];
           x[j] = v[j] * fast_exp2(up ? G[i][j] : -G[i][j]);
         }
         put(hi, i, x);

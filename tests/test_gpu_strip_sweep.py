@@ -199,3 +199,24 @@ def test_strip_sweep_delta_rule_narrow_tiles(shape, bv, wider, cuda_device):
                         cu_seqlens=cu)
     # fp32 sums in the same order: the last bit of a state, one ulp of a rounded output
     assert rel(host(ow[:, :, :H]), host(o)) <= 1e-3 and rel(host(htw[:, :H]), host(ht)) <= 1e-5
+
+
+def test_strip_sweep_gate_sum_precision(cuda_device):
+    """Strong gates: the in-chunk gate sums reach 150 (log2 units), and the rounding of the sums
+    shows in the final state beside the 2.4e-6 of the bf16 hi + lo operands.  Summed in log2
+    units, as kda_prep and dq/dk/dg sum them, the state is 4.06e-6 off float64; summed in
+    natural units and scaled afterwards (a rounding more per row and per total) 4.79e-6."""
+    from tops.ops.gla import chunk_gla
+    B, T, H, K = 4, 300, 32, 64
+    gen = torch.Generator().manual_seed(77)
+    q, k, v = (torch.randn(B, T, H, K, generator=gen).to(cuda_device, torch.bfloat16) for _ in range(3))
+    g = -2 * torch.nn.functional.softplus(torch.randn(B, T, H, K, generator=gen)).to(cuda_device)
+    h0 = torch.randn(B, H, K, K, generator=gen).to(cuda_device)
+    print("gate sum precision", flush=True)
+    _, ht = chunk_gla(q, k, v, g, initial_state=h0, output_final_state=True)
+    S = h0.double()
+    for t in range(T):
+        S = S * g[:, t].double().exp()[..., None] + k[:, t].double()[..., None] * v[:, t].double()[..., None, :]
+    err = float((ht.double() - S).norm() / S.norm())
+    print(f"ht error {err:.3e}", flush=True)
+    assert err < 4.35e-6, f"ht: {err:.3e} of float64"
