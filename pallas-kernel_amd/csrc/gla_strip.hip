@@ -916,11 +916,12 @@ __global__ __launch_bounds__(64 * (BV / 16 + 4)) void gla_strip_kernel(SweepPara
 
 // Whether launch_gla_sweep routes a call to this kernel: per-channel gates without the gate
 // shift of the reverse-time recurrence, any input type.  TOPS_SWEEP_SERIAL=1 in the
-// environment keeps such calls on gla_sweep_kernel (comparisons), except those that write fp16
-// checkpoints, which only this kernel does for per-channel gates.
-bool gla_strip_eligible(const SweepParams& p) {
+// environment keeps bf16 calls on gla_sweep_kernel (comparisons), except those that write fp16
+// checkpoints, which only this kernel does for per-channel gates; gla_sweep_kernel has no such
+// instances of the other types.
+bool gla_strip_eligible(const SweepParams& p, bool bf16) {
   if (p.gate_mode != kGateK || p.gshift) return false;
-  if (p.ckpt16) return true;
+  if (p.ckpt16 || !bf16) return true;
   const char* e = getenv("TOPS_SWEEP_SERIAL");
   return !(e && e[0] == '1');
 }
@@ -979,7 +980,11 @@ hipError_t launch_gla_strip(const SweepParams& p, hipStream_t s) {
   if (var == 1) { \
     if constexpr (std::is_same<TIn, uint16_t>::value) TOPS_STRIP(KPV, 1); \
     else return hipErrorInvalidValue; \
-  } else if (var == 2) TOPS_STRIP(KPV, 2); else TOPS_STRIP(KPV, 0)
+  } else if (var == 2) { \
+    /* (the KDA backward always keeps dS) */ \
+    if constexpr (!(DELTA && REV)) TOPS_STRIP(KPV, 2); \
+    else return hipErrorInvalidValue; \
+  } else TOPS_STRIP(KPV, 0)
   if (kp == 32) { TOPS_STRIP_K(32); }
   else if (kp == 64) { TOPS_STRIP_K(64); }
   else { TOPS_STRIP_K(128); }

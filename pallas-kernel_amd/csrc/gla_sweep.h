@@ -71,7 +71,7 @@ hipError_t launch_gla_sweep(const SweepParams& p, hipStream_t s);
 
 // The strip-specialised sweep (gla_strip.hip) for per-channel gates: launch_gla_sweep routes
 // eligible calls to it.  DELTA = the KDA delta-rule sweep (forward, v_new = u - w S replaces v).
-bool gla_strip_eligible(const SweepParams& p);
+bool gla_strip_eligible(const SweepParams& p, bool bf16);
 template <typename TIn, bool REV, bool DELTA>
 hipError_t launch_gla_strip(const SweepParams& p, hipStream_t s);
 // Its state-only pass: the end state s_fin and the decay sums dec_fin of every sequence.

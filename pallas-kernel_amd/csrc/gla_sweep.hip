@@ -57,9 +57,9 @@
 
 namespace tops {
 
-// GK: the per-channel gate mode only (kGateK, the GLA and KDA path), compiled on its own so
-// that the hot path carries no gate-mode branches; !GK serves the per-token and constant
-// gates (kGateS, kGateGamma, kGateGammaK) chosen at run time.
+// GK: the per-channel gate mode only (kGateK: the reverse-time recurrence, and bf16 calls kept
+// here for comparison), compiled on its own so that it carries no gate-mode branches; !GK serves
+// the per-token and constant gates (kGateS, kGateGamma, kGateGammaK) chosen at run time.
 template <typename TIn, int KP, bool REV, bool ST, bool GK, bool GV = false>
 __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
   constexpr int NW = 8;                  // wave64s per workgroup
@@ -749,8 +749,9 @@ __global__ __launch_bounds__(512) void gla_sweep_kernel(SweepParams p) {
 
 template <typename TIn, bool REV>
 hipError_t launch_gla_sweep(const SweepParams& p, hipStream_t s) {
-  if (gla_strip_eligible(p)) return launch_gla_strip<TIn, REV, false>(p, s);
-  if constexpr (std::is_same<TIn, uint16_t>::value) {
+  constexpr bool BF = std::is_same<TIn, uint16_t>::value;
+  if (gla_strip_eligible(p, BF)) return launch_gla_strip<TIn, REV, false>(p, s);
+  if constexpr (BF) {
     if (gla_strip_s_eligible(p)) return launch_gla_strip_s<REV>(p, false, s);
   }
   if (p.ckpt16) return hipErrorInvalidValue;   // the strip kernels write fp16 checkpoints
@@ -759,9 +760,14 @@ hipError_t launch_gla_sweep(const SweepParams& p, hipStream_t s) {
 #define TOPS_SWEEP(KPV, GKV) \
   hipLaunchKernelGGL((gla_sweep_kernel<TIn, KPV, REV, false, GKV>), grid, dim3(512), 0, s, p)
   if (p.gate_mode == kGateK) {
-    if (kp == 32) TOPS_SWEEP(32, true);
-    else if (kp == 64) TOPS_SWEEP(64, true);
-    else TOPS_SWEEP(128, true);
+    // the reverse-time recurrence (any type), or a bf16 call under TOPS_SWEEP_SERIAL
+    if constexpr (REV || BF) {
+      if (kp == 32) TOPS_SWEEP(32, true);
+      else if (kp == 64) TOPS_SWEEP(64, true);
+      else TOPS_SWEEP(128, true);
+    } else {
+      return hipErrorInvalidValue;
+    }
   } else {
     if (kp == 32) TOPS_SWEEP(32, false);
     else if (kp == 64) TOPS_SWEEP(64, false);

@@ -104,3 +104,23 @@ def test_pipe_vs_serial_and_oracle(cfg, layout, cuda_device):
         lim = 1e-3 if stored == bf else 1e-5
         ab = rel(x, y)
         assert ab <= lim, f"{name}: pipelined vs serial rel {ab:.3e} > {lim}"
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.float16], ids=["f32", "f16"])
+def test_other_types_have_one_sweep(dt, cuda_device, monkeypatch):
+    """fp32 and fp16 calls run on the strip kernel whatever TOPS_SWEEP_SERIAL says (the serial
+    kernel has no per-channel-gate forward for them): the same bits either way."""
+    from tops.ops.gla import chunk_gla
+    d = gla_inputs(2, 200, 2, 64, 72, 5, gate_div=16.0, h0=True, grads=True)
+    res = []
+    for serial in ("0", "1"):
+        monkeypatch.setenv("TOPS_SWEEP_SERIAL", serial)
+        x = [to_dev(d[n], dt, cuda_device).requires_grad_() for n in "qkv"]
+        x += [to_dev(d[n], torch.float32, cuda_device).requires_grad_() for n in ("g", "h0")]
+        print(f"one sweep {dt} serial={serial}", flush=True)
+        o, ht = chunk_gla(*x[:4], initial_state=x[4], output_final_state=True)
+        gr = torch.autograd.grad((o, ht), x, (to_dev(d["do"], dt, cuda_device),
+                                              to_dev(d["dht"], torch.float32, cuda_device)))
+        res.append([o, ht, *gr])
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
