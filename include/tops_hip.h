@@ -58,8 +58,8 @@ int64_t tops_gla_state_bytes(int total_chunks, int H, int K, int V);
  * tops/cpu/ops/gla/chunk.py:206-212.  Host pointers.
  *   cu_seqlens [N+1]; chunk_offsets [N+1] (out; chunk_offsets[N] = total);
  *   chunk_indices [capacity][2] (out, may be NULL): (sequence id, chunk id).
- * Returns the total number of chunks, or a negative TOPS_ERR_* code
- * (empty segments are rejected, as tops/cpu/ops/gla/chunk.py:686 does). */
+ * Returns the total number of chunks (an empty sequence has none), or a negative TOPS_ERR_*
+ * code. */
 int tops_prepare_chunk_indices(const int32_t* cu_seqlens, int N, int C, int32_t* chunk_offsets,
                                int32_t* chunk_indices, int capacity);
 

@@ -7,7 +7,8 @@
 // SIMD) are consumers: wave j holds the fp32 state of 16 V columns, all K rows, in MFMA
 // accumulators for the whole walk, and runs every product that touches it.  Waves 4-7 are
 // producers: they load the raw q / k / g / Y rows, do the gate cumsum, the exponentials and
-// the bf16 hi / lo splits, and the causal D tiles.  With G the in-chunk inclusive gate cumsum
+// the bf16 hi / lo splits.  The causal D tiles are the consumers' work, except in the forward
+// delta rule, where the producers compute them.  With G the in-chunk inclusive gate cumsum
 // (log2 units), Gm half its last row, e = 2^Gm, X~ = q 2^(G-Gm), Z~ = k 2^(Gm-G) (reverse: X~
 // and Z~ exchanged), D[p][r] = Z~_p . X~_r on the causal side:
 //   T = e S,   out^T = T^T X~^T + Y^T D,   S' = e (T + Z~^T Y)
@@ -20,19 +21,20 @@
 // consecutive channels (A of out^T, B of w S).  The row order is free, as Z~^T is read
 // transposed (ds_read_b64_tr_b16) from addresses of the lane's choosing.
 // Each chunk is two intervals between barriers:
-//   A: consumers T^T X~^T (delta: w S, v_new)   | producers D(c), Y(c), Z~(c + 1)
+//   A: consumers T^T X~^T, D(c)                 | producers Y(c), Z~(c + 1)
+//      (forward delta: w S, v_new, T^T X~^T     |            D(c), Z~(c + 1))
 //   B: consumers Y^T D, state update, next T    | producers X~(c + 1), cumsum of c + 2
 // so the VALU staging of one chunk runs beside the matrix products of another on every SIMD.
 // X~, Y and D are single planes (written in the interval that does not read them), Z~ two.
-// Planes are row-major without padding, 16-byte pieces XOR-swizzled by row so that the row
-// reads, the transposed reads and the staging writes are free of bank conflicts.
+// Planes are row-major without padding, their 16-byte pieces swizzled by row (swz in strip.h).
 // Delta rule (KDA): forward, Y = v_new = u - w S comes from the state operand and the staged
 // planes of w 2^-Gm (against T = 2^Gm S), token-major, which is the operand layout of the
 // products that follow; reverse, the state update gains - w^T dv_new, and dv_new is stored
 // transposed per chunk for the WY backward.
-// The D tiles sit with the consumers, which have the X~ fragments in registers already: with
-// the producers they cost 80 KB more of LDS reads per chunk and made interval A
-// producer-bound (9,200 -> 8,900 cycles per training chunk, 8,000 -> 6,700 inference).  The
+// Why the D tiles sit with the consumers: those have the X~ fragments in registers already, and
+// with the producers they cost 80 KB more of LDS reads per chunk and made interval A
+// producer-bound (9,200 -> 8,900 cycles per training chunk, 8,000 -> 6,700 inference); in the
+// forward delta rule the consumers carry w S instead.  The
 // fp16 checkpoint goes through LDS to the producers, which store whole 128-byte rows:
 // stored from the accumulators it was 64 four-byte-per-lane stores per chunk that held the
 // consumers up (interval A 4,600 -> 2,700 cycles).  Producers run at raised wave priority
@@ -47,8 +49,8 @@
 // multiplied and passed the state through LDS.  Delta rule, B4 T8192 H32 K=V=128 bf16:
 // forward with checkpoints 1187 -> 800 us, without 1047 -> 680, reverse 970 -> 710 (2.7 to
 // 3.5 GB per launch, 500-720 us at the copy rate); fp32, B1 T5000 H32 (64 workgroups, so
-// latency alone): 756 -> 370, 289 on 16-column tiles.  There producers keep the D tiles (the consumers carry w S) and
-// the default priority in interval A.
+// latency alone): 756 -> 370, 289 on 16-column tiles.  There the producers keep the default
+// priority in interval A.
 #include <stdlib.h>
 
 #include <atomic>

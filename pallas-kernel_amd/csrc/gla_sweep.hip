@@ -9,8 +9,9 @@
 // following the oracle tops/cpu/ops/gla/chunk.py:310-354, 387-427.
 //
 // Calls with per-channel gates, and KDA's delta rule, run on the strip-specialised sweep of
-// gla_strip.hip; this kernel keeps the other gate forms, the reverse-time recurrence and the
-// value-side gates.
+// gla_strip.hip, bf16 calls with one gate per token or a constant per head on that of
+// gla_strip_s.hip.  This kernel keeps those gates of fp32 and fp16 calls, the constant
+// per-channel gates (any type), the reverse-time recurrence and the value-side gates.
 //
 // One workgroup (8 wave64, two per SIMD) owns one (sequence, head, 64-wide V tile) and
 // walks the sequence chunk by chunk (C = 64), forwards or backwards.  A K x 64 fp32 state S

@@ -4,7 +4,11 @@
 
 namespace tops {
 
-// piece swizzle of plane row r (see above); KP channels per row, 16-byte pieces
+// The LDS planes are row-major, KP channels per row, without padding.  The 16-byte piece c of
+// row r lies at piece c ^ swz(r) of that row, so that the three ways a plane is used spread over
+// the banks: staging writes (8 or 16 bytes of adjacent pieces of a few rows), row reads
+// (ds_read_b128, one piece of 16 rows) and transposed reads (ds_read_b64_tr_b16, four rows at
+// four adjacent pieces).
 template <int KP>
 __device__ __forceinline__ constexpr int swz(int r) {
   const int b0 = r & 1, b1 = (r >> 1) & 1, b2 = (r >> 2) & 1, b3 = (r >> 3) & 1;

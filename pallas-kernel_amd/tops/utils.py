@@ -176,12 +176,13 @@ def set_sequence_split(mode=None) -> None:
 
 # Residual states of the GLA / simple-GLA training path.  "full": the forward keeps the
 # state before every chunk and the backward's reverse sweep writes dh for every chunk
-# (2 x chunks x H x K x V).  For bf16 inputs with per-channel gates (chunk_gla, K, V <= 128)
-# these are fp16 times a power-of-two factor per (chunk, head, 64 columns of V); other
-# calls keep fp32.  "full32": fp32 everywhere.  "paired" (bf16 inputs): one fp32 buffer of
-# chunks x H x K x V holding h before the even chunks and dh after the odd ones; the dq / dk
-# / dg kernel rebuilds the rest from each chunk's pair partner.  Half the memory and
-# checkpoint bytes of "full32", but the rebuild needs both chunks of a pair on one CU.
+# (2 x chunks x H x K x V).  For bf16 inputs with K, V <= 128 and per-channel or per-token
+# gates (chunk_gla, chunk_simple_gla, chunk_kda) these are fp16 times a power-of-two factor per
+# (chunk, head, 64 columns of V); other calls keep fp32.  "full32": fp32 everywhere.  "paired"
+# (bf16 inputs): one fp32 buffer of chunks x H x K x V holding h before the even chunks and dh
+# after the odd ones; the dq / dk / dg kernel rebuilds the rest from each chunk's pair partner.
+# Half the memory and checkpoint bytes of "full32", but the rebuild needs both chunks of a pair
+# on one CU.
 _CKPT = {"layout": "full"}
 
 
